@@ -21,24 +21,83 @@ namespace lm {
 constexpr int kHistTile = 256;
 constexpr int kHistMaxBins = 256;
 
+// Bytes of one row per workgroup: 8 vectors of 16 bytes per lane, all in
+// flight.  Reading a byte per lane and load moved 326 GB/s (1082 us for 720
+// rows of 490,000); 16 bytes per load move 5.6 TB/s (63 us), HBM's rate.
+constexpr int kCountVecs = 8;
+constexpr int64_t kCountBytes = 16ll * kCountVecs * kBlock;
+
+// Adds the bytes equal to 1, 2, 3 of a word to c[0..2].  Codes 0..3 take two
+// bits: popcounts of their combinations; a word with any other code is
+// counted byte by byte.
+__device__ __forceinline__ void count_word(uint32_t w, uint32_t (&c)[3]) {
+    if ((w & 0xfcfcfcfcu) == 0u) {
+        const uint32_t lo = w & 0x01010101u, hi = (w >> 1) & 0x01010101u;
+        c[0] += __popc(lo & ~hi);
+        c[1] += __popc(hi & ~lo);
+        c[2] += __popc(lo & hi);
+    } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t v = (w >> (8 * q)) & 0xffu;
+            c[0] += v == 1u;
+            c[1] += v == 2u;
+            c[2] += v == 3u;
+        }
+    }
+}
+
+// Rows may start at any byte: the aligned 16-byte vectors in between are
+// shared out over blockIdx.x, and the row's first block takes the bytes
+// before and after them.
 __global__ void __launch_bounds__(kBlock)
 species_count_kernel(const int8_t* __restrict__ rec, int64_t n, int64_t stride,
                      unsigned long long* __restrict__ counts) {
     __shared__ uint32_t part[kBlock / 64][4];
     const int64_t s = blockIdx.y;
-    uint32_t c0 = 0, c1 = 0, c2 = 0, c3 = 0;
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
-        const int v = rec[s * stride + i];
-        c1 += v == 1;
-        c2 += v == 2;
-        c3 += v == 3;
-        c0 += v < 1 || v > 3;
+    const int8_t* row = rec + s * stride;
+    const int64_t head0 = (int64_t)((16u - (unsigned)((uintptr_t)row & 15u)) & 15u);
+    const int64_t head = head0 < n ? head0 : n;
+    const int64_t nv = (n - head) / 16;
+    const uint4* vec = reinterpret_cast<const uint4*>(row + head);
+    uint32_t c[3] = {0, 0, 0}, seen = 0;
+    for (int64_t v0 = (int64_t)blockIdx.x * kCountVecs * kBlock; v0 < nv; v0 += (int64_t)gridDim.x * kCountVecs * kBlock) {
+        uint4 q[kCountVecs];
+#pragma unroll
+        for (int k = 0; k < kCountVecs; ++k) {
+            const int64_t v = v0 + k * kBlock + threadIdx.x;
+            q[k] = make_uint4(0u, 0u, 0u, 0u);
+            if (v < nv) {
+                q[k] = vec[v];
+                seen += 16;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < kCountVecs; ++k) {
+            count_word(q[k].x, c);
+            count_word(q[k].y, c);
+            count_word(q[k].z, c);
+            count_word(q[k].w, c);
+        }
     }
-    uint32_t c[4] = {c0, c1, c2, c3};
+    if (blockIdx.x == 0) {
+        const int64_t t = threadIdx.x, tail = n - head - 16 * nv;  // head, tail < 16
+        int64_t at = -1;
+        if (t < head) at = t;
+        else if (t >= 16 && t - 16 < tail) at = head + 16 * nv + (t - 16);
+        if (at >= 0) {
+            const int v = row[at];
+            c[0] += v == 1;
+            c[1] += v == 2;
+            c[2] += v == 3;
+            seen += 1;
+        }
+    }
+    uint32_t all[4] = {seen - c[0] - c[1] - c[2], c[0], c[1], c[2]};
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        uint32_t x = c[k];
+        uint32_t x = all[k];
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
         if (lane == 0) part[wave][k] = x;
@@ -110,8 +169,7 @@ int lm_species_counts(const int8_t* species, int64_t n, int32_t nsteps, int64_t 
     LM_REQUIRE(nsteps <= 1 || stride >= n, LM_ERR_ARG, "stride < n");
     if (n == 0 || nsteps == 0) return LM_OK;
     LM_REQUIRE(species && counts, LM_ERR_ARG, "NULL pointer");
-    unsigned gx = lm::grid_for(n);
-    gx = gx > 1024u ? 1024u : gx;
+    unsigned gx = (unsigned)((n + lm::kCountBytes - 1) / lm::kCountBytes < 1024 ? (n + lm::kCountBytes - 1) / lm::kCountBytes : 1024);
     LM_LAUNCH(lm::K_SPECIES_COUNT, lm::species_count_kernel, dim3(gx, (unsigned)nsteps), dim3(lm::kBlock), 0,
               (hipStream_t)stream, species, n, nsteps <= 1 ? n : stride,
               reinterpret_cast<unsigned long long*>(counts));
