@@ -11,10 +11,16 @@
 // oracle reproduces a bit for bit) is binned against increasing thresholds:
 // bin = number of thresholds <= a.  The caller derives the thresholds from
 // distance edges (d = 2 R asin(sqrt(a))), so the bins are distance bins and
-// the counts are exact integers.  Work: a triangular grid of 256 x 256 pair
-// tiles, the j tile's positions and cosines staged in LDS, one LDS histogram
-// per wavefront, one global atomic per non-empty bin per block.
+// the counts are exact integers.
+//
+// A float32 value of a decides nearly every pair: its error is bounded (see
+// kHistTol), so a pair farther than that from every threshold lands in the
+// bin the float64 value lands in, and only the others (about 2 in 100,000 at
+// ten bins per decade) evaluate the float64 term.
 #include "lm_common.h"
+
+#include <cfloat>
+#include <cmath>
 
 namespace lm {
 
@@ -110,51 +116,236 @@ species_count_kernel(const int8_t* __restrict__ rec, int64_t n, int64_t stride,
     }
 }
 
+// ---------------------------------------------------------------------------
+// distance histogram
+// ---------------------------------------------------------------------------
+// The float32 term, for |dlon|, |dlat| <= 30 (WIDE: 180) degrees and
+// latitudes in [-90, 90]: sin^2(d / 2) = z (1 - z / 3 + 2 z^2 / 45 - ...) in
+// z = (d / 2)^2 rad^2, so both summands are products without cancellation.
+// With u = 2^-24: the difference of two float32 positions is within u
+// (relative), z within 3 u, the narrow polynomial within 2.2 u (its later
+// terms are below 0.023 of the first; truncation 3e-9), cos cos within 3 u,
+// the sum within 11 u.  The wide polynomial's terms cancel to 0.4 of 2.1 at 90
+// degrees: within 30 u in all.  kHistTol (67 u) covers both.
+constexpr float kHistTol = 4e-6f;
+constexpr float kHistNarrow = 30.0f, kHistWide = 180.0f;
+
+constexpr double half_deg_rad2() { return 0.25 * LM_DEG2RAD * LM_DEG2RAD; }
+
+// Coefficient m (from 1) of sin^2 x = sum_m c_m x^(2m): (-1)^(m+1) 2^(2m-1) / (2m)!.
+constexpr double sin2_coef(int m) {
+    double c = 1.0;  // m = 1: 2 / 2!
+    for (int k = 2; k <= m; ++k) c *= -4.0 / ((2.0 * k) * (2.0 * k - 1.0));
+    return c;
+}
+
+template <bool WIDE>
+__device__ __forceinline__ float sin2_half(float d) {
+    if constexpr (WIDE) {
+        const float t = d * (float)(0.5 * LM_DEG2RAD);
+        const float z = t * t;
+        float p = (float)sin2_coef(12);
+#pragma unroll
+        for (int m = 11; m >= 1; --m) p = fmaf(p, z, (float)sin2_coef(m));
+        return z * p;
+    } else {
+        // in degrees: the scale is in the coefficients
+        constexpr double r = half_deg_rad2();
+        const float z = d * d;
+        float p = (float)(sin2_coef(4) * r * r * r * r);
+        p = fmaf(p, z, (float)(sin2_coef(3) * r * r * r));
+        p = fmaf(p, z, (float)(sin2_coef(2) * r * r));
+        p = fmaf(p, z, (float)(sin2_coef(1) * r));
+        return z * p;
+    }
+}
+
+// Table over the float32 values of a in [2^-60, 2): cells of 1/16 octave,
+// found from the value's top bits.  A cell holds the number of thresholds
+// below it (less the tolerance) and the one threshold that may lie in it
+// (FLT_MAX: none); more than one, and values outside the table, have a NaN
+// threshold, on which no comparison decides.
+constexpr int kLutShift = 19;
+constexpr uint32_t kLutBase = (127u - 60u) << (23 - kLutShift);
+constexpr uint32_t kLutCells = 61u << (23 - kLutShift);
+
+// Number of increasing edges e[0 .. m) with e * scale <= v (or < v).
+template <bool STRICT>
+__device__ __forceinline__ int edges_below(const double* e, int m, double scale, double v) {
+    int lo = 0, hi = m;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        const double x = e[mid] * scale;
+        if (STRICT ? x < v : x <= v) lo = mid + 1;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// A pair's bin from its float64 term.
+__device__ __forceinline__ int exact_bin(const double* e, int m, float xi, float yi, float xj, float yj) {
+    const double s1 = sin_deg(0.5 * ((double)yj - (double)yi));
+    const double s2 = sin_deg(0.5 * ((double)xj - (double)xi));
+    const double a = s1 * s1 + (cos_deg((double)yi) * cos_deg((double)yj)) * (s2 * s2);
+    return edges_below<false>(e, m, 1.0, a);
+}
+
+// A workgroup takes a tile of 512 points i (two per lane) against `per`
+// tiles of 256 points j (staged in LDS, read by all lanes at once), from the
+// diagonal on.  Counters: a column per lane, [bin][lane], shared by the
+// wavefronts: neighbouring lanes' pairs mostly share a bin, and adds to one
+// counter would go one after the other (the first version, one counter per
+// wavefront and bin, and FP64 sines and a binary search for every pair, took
+// 16.2 ms for 98,587 points; this one takes 3.2 ms, bound by VALU issue, ~30
+// instructions per pair).
+constexpr int kHistI = 2;
+
+struct HistShared {
+    float4 pj[kHistTile];             // x, y, cos(lat)
+    float2 lut[kLutCells + 1];        // threshold, bin below it
+    double edges[kHistMaxBins];
+    float box[4][kHistTile / 64];
+    uint32_t turn;                    // (float bits) below every threshold that is less than the one before it
+};
+
+template <bool WIDE>
+__device__ __forceinline__ void hist_tile(const HistShared& S, uint32_t* __restrict__ h, int jend, const float (&xi)[kHistI],
+                                          const float (&yi)[kHistI], const float (&ci)[kHistI],
+                                          const int (&after)[kHistI], int nedges, uint32_t cols, uint32_t col) {
+    for (int k0 = 0; k0 < jend; k0 += 32) {
+        const int m = min(32, jend - k0);
+        uint32_t amb[kHistI] = {};  // pairs the float32 term does not decide
+#pragma unroll 4
+        for (int kk = 0; kk < m; ++kk) {
+            const float4 p = S.pj[k0 + kk];
+#pragma unroll
+            for (int u = 0; u < kHistI; ++u) {
+                const float a = fmaf(ci[u] * p.z, sin2_half<WIDE>(p.x - xi[u]), sin2_half<WIDE>(p.y - yi[u]));
+                // out of the table (0, tiny, above 2, negative, NaN): the last entry
+                const uint32_t cell = min((__float_as_uint(a) >> kLutShift) - kLutBase, kLutCells);
+                const float2 e = S.lut[cell];
+                const bool above = a > e.x * (1.0f + kHistTol), below = a < e.x * (1.0f - kHistTol);
+                const bool ok = k0 + kk > after[u], clear = above | below;
+                const uint32_t bin = __float_as_uint(e.y) + (above ? 1u : 0u);
+                atomicAdd(&h[bin * cols + col], (ok & clear) ? 1u : 0u);
+                amb[u] |= ((ok & !clear) ? 1u : 0u) << kk;
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kHistI; ++u)
+            while (amb[u]) {
+                const float4 p = S.pj[k0 + __ffs(amb[u]) - 1];
+                amb[u] &= amb[u] - 1u;
+                atomicAdd(&h[(uint32_t)exact_bin(S.edges, nedges, xi[u], yi[u], p.x, p.y) * cols + col], 1u);
+            }
+    }
+}
+
 __global__ void __launch_bounds__(kHistTile)
 dist_hist_kernel(int64_t n, const float* __restrict__ lon, const float* __restrict__ lat, int nbins,
-                 const double* __restrict__ edges, unsigned long long* __restrict__ hist) {
-    const int64_t ti = blockIdx.x, tj = blockIdx.y;
-    if (tj < ti) return;  // the lower triangle of the tile grid has no pairs i < j
-    __shared__ double sx[kHistTile], sy[kHistTile], sc[kHistTile];
-    __shared__ double se[kHistMaxBins];
-    __shared__ uint32_t h[kHistTile / 64][kHistMaxBins];
-    const int t = threadIdx.x, wave = t >> 6;
-    const int64_t j0 = tj * kHistTile, i = ti * kHistTile + t;
-    {
-        const int64_t j = j0 + t;
-        const double x = j < n ? (double)lon[j] : 0.0, y = j < n ? (double)lat[j] : 0.0;
-        sx[t] = x;
-        sy[t] = y;
-        sc[t] = cos_deg(y);
+                 const double* __restrict__ edges, unsigned long long* __restrict__ hist, int per, uint32_t cols) {
+    extern __shared__ uint32_t h[];  // [nbins][cols]
+    __shared__ HistShared S;
+    const int64_t i0 = (int64_t)blockIdx.x * (kHistTile * kHistI);
+    const int64_t jt0 = (int64_t)blockIdx.x * kHistI + (int64_t)blockIdx.y * per;  // first j tile
+    if (jt0 * kHistTile >= n) return;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const uint32_t col = (uint32_t)lane & (cols - 1u);
+    const int nedges = nbins - 1;
+    for (uint32_t b = t; b < (uint32_t)nbins * cols; b += kHistTile) h[b] = 0u;
+    for (int b = t; b < nedges; b += kHistTile) S.edges[b] = edges[b];
+    float xi[kHistI], yi[kHistI], ci[kHistI];
+    // extents of the i tile; a position that is not finite, or a latitude
+    // past the poles, leaves it unbounded and so every pair to the float64 term
+    float lo_x = INFINITY, hi_x = -INFINITY, lo_y = INFINITY, hi_y = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < kHistI; ++u) {
+        const int64_t i = i0 + u * kHistTile + t;
+        const bool in = i < n;
+        xi[u] = in ? lon[i] : 0.0f;
+        yi[u] = in ? lat[i] : 0.0f;
+        ci[u] = (float)cos_deg((double)yi[u]);
+        if (in) {
+            const bool fine = fabsf(xi[u]) < 1e6f && fabsf(yi[u]) <= 90.0f;
+            lo_x = fine ? fminf(lo_x, xi[u]) : -INFINITY;
+            hi_x = fine ? fmaxf(hi_x, xi[u]) : INFINITY;
+            lo_y = fine ? fminf(lo_y, yi[u]) : -INFINITY;
+            hi_y = fine ? fmaxf(hi_y, yi[u]) : INFINITY;
+        }
     }
-    for (int b = t; b < nbins - 1; b += kHistTile) se[b] = edges[b];
-    for (int b = t; b < (kHistTile / 64) * kHistMaxBins; b += kHistTile) (&h[0][0])[b] = 0u;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+        lo_x = fminf(lo_x, __shfl_xor(lo_x, d, 64));
+        hi_x = fmaxf(hi_x, __shfl_xor(hi_x, d, 64));
+        lo_y = fminf(lo_y, __shfl_xor(lo_y, d, 64));
+        hi_y = fmaxf(hi_y, __shfl_xor(hi_y, d, 64));
+    }
+    if (t == 0) S.turn = __float_as_uint(FLT_MAX);
+    if (lane == 0) {
+        S.box[0][wave] = lo_x;
+        S.box[1][wave] = hi_x;
+        S.box[2][wave] = lo_y;
+        S.box[3][wave] = hi_y;
+    }
     __syncthreads();
-    if (i < n) {
-        const double xi = (double)lon[i], yi = (double)lat[i], ci = cos_deg(yi);
-        const int64_t jend = n - j0 < kHistTile ? n - j0 : kHistTile;
-        // pairs (i, j) with j > i: the whole tile when tj > ti, past the diagonal when tj == ti
-        const int k0 = tj == ti ? t + 1 : 0;
-        for (int k = k0; k < (int)jend; ++k) {
-            const double s1 = sin_deg(0.5 * (sy[k] - yi));
-            const double s2 = sin_deg(0.5 * (sx[k] - xi));
-            const double a = s1 * s1 + (ci * sc[k]) * (s2 * s2);
-            // bin = number of thresholds <= a (the thresholds increase)
-            int lo = 0, hi = nbins - 1;
-            while (lo < hi) {
-                const int mid = (lo + hi) >> 1;
-                if (se[mid] <= a) lo = mid + 1;
-                else hi = mid;
-            }
-            atomicAdd(&h[wave][lo], 1u);
+#pragma unroll
+    for (int w = 0; w < kHistTile / 64; ++w) {
+        lo_x = fminf(lo_x, S.box[0][w]);
+        hi_x = fmaxf(hi_x, S.box[1][w]);
+        lo_y = fminf(lo_y, S.box[2][w]);
+        hi_y = fmaxf(hi_y, S.box[3][w]);
+    }
+    // thresholds past the antipodes turn back (a = sin^2): cells from the
+    // lowest such one on are left to the binary search, as for every pair before
+    for (int b = t + 1; b < nedges; b += kHistTile)
+        if (!(S.edges[b] >= S.edges[b - 1]))
+            atomicMin(&S.turn, __float_as_uint(fmaxf((float)S.edges[b] * (1.0f - kHistTol), 0.0f)));
+    __syncthreads();
+    const float turn = __uint_as_float(S.turn);
+    for (uint32_t c = t; c <= kLutCells; c += kHistTile) {
+        const float from = __uint_as_float((c + kLutBase) << kLutShift);
+        const float to = __uint_as_float((c + 1u + kLutBase) << kLutShift);
+        const int b0 = edges_below<false>(S.edges, nedges, 1.0 + (double)kHistTol, (double)from);
+        const int b1 = edges_below<true>(S.edges, nedges, 1.0 - (double)kHistTol, (double)to);
+        float e = b1 == b0 ? FLT_MAX : b1 == b0 + 1 ? (float)S.edges[b0] : NAN;
+        if (c == kLutCells || to >= turn) e = NAN;
+        S.lut[c] = make_float2(e, __uint_as_float((uint32_t)b0));
+    }
+    for (int q = 0; q < per; ++q) {
+        const int64_t j0 = (jt0 + q) * kHistTile;
+        if (j0 >= n) break;  // uniform over the block
+        const bool in = j0 + t < n;
+        const float x = in ? lon[j0 + t] : 0.0f, y = in ? lat[j0 + t] : 0.0f;
+        const float far = fmaxf(fmaxf(x - lo_x, hi_x - x), fmaxf(y - lo_y, hi_y - y));
+        const bool fine = fabsf(x) < 1e6f && fabsf(y) <= 90.0f;
+        __syncthreads();  // the tile before has been read
+        S.pj[t] = make_float4(x, y, (float)cos_deg((double)y), 0.0f);
+        const bool narrow = __syncthreads_and(!in || (fine && far <= kHistNarrow));
+        const bool wide = __syncthreads_and(!in || (fine && far <= kHistWide));
+        const int jend = (int)(n - j0 < kHistTile ? n - j0 : kHistTile);
+        int after[kHistI];  // pairs (i, j0 + k) with k > after
+#pragma unroll
+        for (int u = 0; u < kHistI; ++u) {
+            const int64_t i = i0 + u * kHistTile + t;
+            after[u] = i >= n ? jend : i < j0 ? -1 : (int)(i - j0);
+        }
+        if (narrow) {
+            hist_tile<false>(S, h, jend, xi, yi, ci, after, nedges, cols, col);
+        } else if (wide) {
+            hist_tile<true>(S, h, jend, xi, yi, ci, after, nedges, cols, col);
+        } else {
+            for (int k = 0; k < jend; ++k)
+                for (int u = 0; u < kHistI; ++u)
+                    if (k > after[u])
+                        atomicAdd(&h[(uint32_t)exact_bin(S.edges, nedges, xi[u], yi[u], S.pj[k].x, S.pj[k].y) * cols + col], 1u);
         }
     }
     __syncthreads();
-    for (int b = t; b < nbins; b += kHistTile) {
-        uint32_t v = 0;
+    for (int b = wave; b < nbins; b += kHistTile / 64) {
+        uint32_t v = lane < (int)cols ? h[(uint32_t)b * cols + lane] : 0u;
 #pragma unroll
-        for (int w = 0; w < kHistTile / 64; ++w) v += h[w][b];
-        if (v) atomicAdd(hist + b, (unsigned long long)v);
+        for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
+        if (lane == 0 && v) atomicAdd(hist + b, (unsigned long long)v);
     }
 }
 
@@ -185,8 +376,16 @@ int lm_distance_histogram(int64_t n, const float* lon, const float* lat, int32_t
     LM_REQUIRE(ntiles <= 65535, LM_ERR_ARG, "at most %lld points", (long long)65535 * lm::kHistTile);
     if (n < 2) return LM_OK;
     LM_REQUIRE(lon && lat && hist && (nbins == 1 || edges), LM_ERR_ARG, "NULL pointer");
-    LM_LAUNCH(lm::K_DIST_HIST, lm::dist_hist_kernel, dim3((unsigned)ntiles, (unsigned)ntiles), dim3(lm::kHistTile),
-              0, (hipStream_t)stream, n, lon, lat, (int)nbins, edges, reinterpret_cast<unsigned long long*>(hist));
+    const int64_t itiles = (n + lm::kHistTile * lm::kHistI - 1) / (lm::kHistTile * lm::kHistI);
+    // j tiles per workgroup: as many as leave 4096 workgroups (16 per CU), at
+    // most 16, so that the table each one builds is a few percent of its work
+    int64_t per = itiles * ntiles / 2 / 4096;
+    per = per < 1 ? 1 : per > 16 ? 16 : per;
+    // a counter column per lane while the counters take at most 32 KB
+    const uint32_t cols = nbins <= 128 ? 64u : 32u;
+    LM_LAUNCH(lm::K_DIST_HIST, lm::dist_hist_kernel, dim3((unsigned)itiles, (unsigned)((ntiles + per - 1) / per)),
+              dim3(lm::kHistTile), (unsigned)(sizeof(uint32_t) * nbins * cols), (hipStream_t)stream, n, lon, lat,
+              (int)nbins, edges, reinterpret_cast<unsigned long long*>(hist), (int)per, cols);
     LM_LAUNCH_CHECK();
     return LM_OK;
 }

@@ -19,3 +19,25 @@ def test_counts_at_every_alignment(gpu, n, skip):
     rows = sp[skip:].reshape(5, n)
     got = analysis.species_counts(torch.from_numpy(sp).cuda()[skip:].view(5, n)).cpu().numpy()
     assert np.array_equal(got, np.stack([[np.sum(r == c) for c in (1, 2, 3)] for r in rows]))
+
+
+def spread(kind, n, rng):
+    if kind == "lattice":  # equal distances again and again, duplicates
+        k = np.arange(n)
+        return 205.0 + 0.0143 * (k // 40), 25.0 + 0.0143 * (k % 40) * (k % 7 > 0)
+    if kind == "ocean":  # up to 150 degrees apart
+        return rng.uniform(100.0, 250.0, n), rng.uniform(-70.0, 70.0, n)
+    if kind == "globe":  # more than 180 degrees apart, the poles among them
+        return rng.uniform(0.0, 360.0, n), np.where(rng.random(n) < 0.05, 90.0, rng.uniform(-90.0, 90.0, n))
+    lon, lat = rng.uniform(200.0, 201.0, n), rng.uniform(-0.5, 0.5, n)  # a position that is not a number
+    lon[n // 3] = np.nan
+    return lon, lat
+
+
+@pytest.mark.parametrize("kind", ["lattice", "ocean", "globe", "nan"])
+@pytest.mark.parametrize("n,bins", [(2, 70), (511, 70), (513, 1), (1281, 72), (1300, 128), (769, 129)])
+def test_histogram_at_the_edges(gpu, kind, n, bins):
+    lon, lat = (a.astype(np.float32) for a in spread(kind, n, np.random.default_rng(n)))
+    radius = analysis.EARTH_RADIUS_M if bins < 100 else 10.0 ** (0.1 * bins)  # thresholds that increase
+    got = analysis.distance_histogram(torch.from_numpy(lon).cuda(), torch.from_numpy(lat).cuda(), bins, radius)
+    assert np.array_equal(got, oracle.distance_histogram(lon, lat, analysis.haversine_thresholds(bins, radius)))
