@@ -86,6 +86,8 @@ enum KernelId {
     K_SPECIES_COUNT,
     K_DIST_HIST,
     K_RPS_TILE,
+    K_PAIR_SMALL,
+    K_EMIT_SMALL,
     K_NUM_KERNELS
 };
 bool timing_on();

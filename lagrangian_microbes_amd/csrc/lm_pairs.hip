@@ -26,6 +26,8 @@
 // run, so a stencil visits the cells of its own run and candidates of other
 // runs whose cells alias into the same buckets are dropped: pairs never cross
 // runs.
+// Small populations (kSmallMax particles, no runs) take two launches instead,
+// whose workgroups bin a whole step in LDS (see "small populations" below).
 // Distances use the float32 positions widened to double, with the same
 // operations cKDTree applies: dx*dx + dy*dy <= r*r for p = 2, evaluated as
 // written (the library is built without FMA contraction).  For positions of
@@ -33,9 +35,11 @@
 // its square.
 #include "lm_common.h"
 #include "lm_scan.h"
+#include "lm_small.h"
 #include "lm_sort.h"
 
 #include <cmath>
+#include <type_traits>
 
 namespace lm {
 
@@ -97,6 +101,31 @@ __device__ __forceinline__ bool within(const Metric& m, float xa, float ya, floa
     else if constexpr (KIND == kL1) return fabs(dx) + fabs(dy) <= m.r;
     else if constexpr (KIND == kLinf) return fmax(fabs(dx), fabs(dy)) <= m.r;
     else return pow(fabs(dx), m.p) + pow(fabs(dy), m.p) <= m.r2;
+}
+
+// The same decision, mostly in float32, for a candidate (cand) or false.
+template <int KIND>
+__device__ __forceinline__ bool pair_hit(const Metric& m, bool cand, float xa, float ya, float xb, float yb) {
+    if constexpr (KIND == kL2) {
+        // A float32 difference of two float32 positions is within one
+        // rounding (relative 2^-24) of the exact one, so the float32
+        // dx*dx + dy*dy is within 2.4e-7 (relative) of the exact sum of
+        // squares, and the float64 test within 2^-52: outside r^2 (1 -/+
+        // 1e-6) both decide alike.  Only candidates in that band take
+        // the float64 test (a branch almost never taken).
+        const float dx = xb - xa, dy = yb - ya;
+        const float d2 = fmaf(dx, dx, dy * dy);
+        bool hit = cand & (d2 <= m.sure_in);
+        if (cand & !(d2 <= m.sure_in) & !(d2 > m.sure_out)) hit = within<KIND>(m, xa, ya, xb, yb);
+        return hit;
+    } else {
+        // |dx| <= r and |dy| <= r hold for every p >= 1; a float32
+        // difference is within one rounding (relative 2^-24) of the exact
+        // one and m.box lies above r by more than that, so the prefilter
+        // only drops pairs the exact test drops.
+        const float ax = fabsf(xb - xa), ay = fabsf(yb - ya);
+        return cand & (ax <= m.box) & (ay <= m.box) & within<KIND>(m, xa, ya, xb, yb);
+    }
 }
 
 // Visit the record slots of the (up to) 3x3 cells around (cx, cy).  Slot
@@ -343,27 +372,7 @@ pair_count_kernel(int64_t n, CellGrid g, Metric m, Strides st, const uint32_t* _
         for (int u = 0; u < kCand; ++u) {
             const uint32_t j = __float_as_uint(o[u].z);
             const bool cand = (t0 + u < total) & (j > i) & (__float_as_uint(o[u].w) == my_run);
-            bool hit;
-            if constexpr (KIND == kL2) {
-                // A float32 difference of two float32 positions is within one
-                // rounding (relative 2^-24) of the exact one, so the float32
-                // dx*dx + dy*dy is within 2.4e-7 (relative) of the exact sum of
-                // squares, and the float64 test within 2^-52: outside r^2 (1 -/+
-                // 1e-6) both decide alike.  Only candidates in that band take
-                // the float64 test (a branch almost never taken).
-                const float dx = o[u].x - me.x, dy = o[u].y - me.y;
-                const float d2 = fmaf(dx, dx, dy * dy);
-                hit = cand & (d2 <= m.sure_in);
-                if (cand & !(d2 <= m.sure_in) & !(d2 > m.sure_out))
-                    hit = within<KIND>(m, me.x, me.y, o[u].x, o[u].y);
-            } else {
-                // |dx| <= r and |dy| <= r hold for every p >= 1; a float32
-                // difference is within one rounding (relative 2^-24) of the exact
-                // one and m.box lies above r by more than that, so the prefilter
-                // only drops pairs the exact test drops.
-                const float ax = fabsf(o[u].x - me.x), ay = fabsf(o[u].y - me.y);
-                hit = cand & (ax <= m.box) & (ay <= m.box) & within<KIND>(m, me.x, me.y, o[u].x, o[u].y);
-            }
+            const bool hit = pair_hit<KIND>(m, cand, me.x, me.y, o[u].x, o[u].y);
             if (hit & (cnt < kNbr)) row[cnt] = j;
             cnt += hit ? 1u : 0u;
         }
@@ -472,6 +481,212 @@ pair_emit_kernel(int64_t n, const float* __restrict__ x_all, const float* __rest
     }
 }
 
+// ---------------------------------------------------------------------------
+// small populations
+// ---------------------------------------------------------------------------
+// Two launches.  Launch latency was the cost of these sizes: the search of
+// 2,500 particles took ten launches of 3 to 9 us each, 42 us in all, and takes
+// 13.4 us with these two (8 and 4.5 us); twelve steps of 10,000 took 107 us
+// and take 28.  The line is where a step's particles still fit one LDS.
+//   count  workgroups of 1024 lanes, each binning the whole step into its LDS
+//          (positions and indices in bucket order, behind one bucket table)
+//          and searching its own 1024 / LPP particles, LPP lanes each (with
+//          4, three lanes take a stencil row each): partners above each
+//          particle, counted, the first kSmallNbr kept
+//   emit   every workgroup sums the counts before its 1024 rows, scans its
+//          own and writes them sorted; a row of more than kSmallNbr partners
+//          is found again by its wavefront, 64 particles at a time in index
+//          order
+// The cells wrap onto a torus of 2^LWX x 2^LWY buckets (a stencil's nine cells
+// always fall into nine buckets: the sides are at least 64; cells further
+// apart may share one, and the distance test drops what the stencil does not
+// reach), so the table fits LDS whatever the box.
+constexpr int kSmallNbr = 16;  // 16-bit partners kept per particle, in the bytes of kNbr 32-bit ones
+
+template <int LWX, int LWY, typename F>
+__device__ __forceinline__ void small_row(const uint32_t* start, const CellGrid& g, int cx, int row, F&& visit) {
+    constexpr uint32_t WX = 1u << LWX, WY = 1u << LWY;
+    if (row < 0 || row >= g.ny) return;
+    const uint32_t a = (uint32_t)(cx > 0 ? cx - 1 : 0) & (WX - 1u);
+    const uint32_t b = (uint32_t)(cx < g.nx - 1 ? cx + 1 : g.nx - 1) & (WX - 1u);
+    const uint32_t base = ((uint32_t)row & (WY - 1u)) << LWX;
+    // one bucket range, or two when the row wraps
+    const uint32_t e0 = start[base + (a <= b ? b + 1u : WX)];
+    for (uint32_t s = start[base + a]; s < e0; ++s) visit(s);
+    if (a > b) {
+        const uint32_t e1 = start[base + b + 1u];
+        for (uint32_t s = start[base]; s < e1; ++s) visit(s);
+    }
+}
+
+template <int KIND, int NMAX, int LWX, int LWY, int LPP>
+__global__ void __launch_bounds__(kSmallBlock)
+pair_small_count_kernel(int n, const float* __restrict__ x_all, const float* __restrict__ y_all, CellGrid g, Metric m,
+                        Strides st, uint32_t* __restrict__ cnt_all, uint16_t* __restrict__ nbr_all) {
+    constexpr int kItems = NMAX / kSmallBlock;
+    constexpr uint32_t T = 1u << (LWX + LWY);
+    static_assert(NMAX % kSmallBlock == 0 && NMAX <= 65536, "16-bit indices, whole items");
+    static_assert(LPP == 1 || LPP == 4, "a lane per particle, or one per stencil row");
+    __shared__ float2 pos[NMAX];  // in bucket order
+    __shared__ uint16_t idx[NMAX];
+    __shared__ uint32_t start[T + 1];
+    __shared__ uint32_t scan_lds[kSmallBlock / 64];
+    const int64_t s = blockIdx.y;
+    const float* x = x_all + s * st.pos;
+    const float* y = y_all + s * st.pos;
+    const int t = threadIdx.x;
+    float px[kItems], py[kItems];
+    uint32_t bucket[kItems], slot[kItems];
+#pragma unroll
+    for (int q = 0; q < kItems; ++q) {
+        const int i = q * kSmallBlock + t;
+        px[q] = i < n ? x[i] : 0.0f;
+        py[q] = i < n ? y[i] : 0.0f;
+    }
+    for (uint32_t b = t; b <= T; b += kSmallBlock) start[b] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kItems; ++q) {
+        bucket[q] = slot[q] = 0u;
+        if (q * kSmallBlock + t < n) {
+            int cx, cy;
+            cell_of(g, px[q], py[q], &cx, &cy);
+            bucket[q] = (((uint32_t)cy & ((1u << LWY) - 1u)) << LWX) | ((uint32_t)cx & ((1u << LWX) - 1u));
+            slot[q] = atomicAdd(&start[bucket[q]], 1u);
+        }
+    }
+    __syncthreads();
+    small_scan_array(start, T, scan_lds);
+    if (t == 0) start[T] = (uint32_t)n;
+#pragma unroll
+    for (int q = 0; q < kItems; ++q) {
+        const int i = q * kSmallBlock + t;
+        if (i < n) {
+            const uint32_t at = start[bucket[q]] + slot[q];
+            pos[at] = make_float2(px[q], py[q]);
+            idx[at] = (uint16_t)i;
+        }
+    }
+    __syncthreads();
+    const int i = (int)blockIdx.x * (kSmallBlock / LPP) + t / LPP, sub = t % LPP;
+    if (i >= n) return;  // all lanes of a particle
+    const float xi = x[i], yi = y[i];
+    int cx, cy;
+    cell_of(g, xi, yi, &cx, &cy);
+    auto search = [&](auto&& visit) {
+        if constexpr (LPP == 4) {
+            if (sub < 3) small_row<LWX, LWY>(start, g, cx, cy + sub - 1, visit);
+        } else {
+            for (int r = -1; r <= 1; ++r) small_row<LWX, LWY>(start, g, cx, cy + r, visit);
+        }
+    };
+    uint32_t c = 0;
+    search([&](uint32_t k) {
+        const float2 o = pos[k];
+        c += pair_hit<KIND>(m, (int)idx[k] > i, xi, yi, o.x, o.y) ? 1u : 0u;
+    });
+    uint32_t at = 0, all = c;
+    if constexpr (LPP == 4) {  // the particle's lanes add up
+        const uint32_t up1 = __shfl_up(c, 1, 4), up2 = __shfl_up(c, 2, 4);
+        at = (sub > 0 ? up1 : 0u) + (sub > 1 ? up2 : 0u);
+        all = __shfl(at + c, 2, 4);
+    }
+    if (sub == 0) cnt_all[s * st.row + i] = all;
+    if (c == 0) return;
+    uint16_t* row = nbr_all + 2 * s * st.nbr + (int64_t)i * kSmallNbr;
+    search([&](uint32_t k) {
+        const float2 o = pos[k];
+        if (pair_hit<KIND>(m, (int)idx[k] > i, xi, yi, o.x, o.y)) {
+            if (at < (uint32_t)kSmallNbr) row[at] = idx[k];
+            ++at;
+        }
+    });
+}
+
+template <int KIND>
+__global__ void __launch_bounds__(kSmallBlock)
+pair_small_emit_kernel(int n, const float* __restrict__ x_all, const float* __restrict__ y_all, Metric m, Strides st,
+                       const uint32_t* __restrict__ cnt_all, const uint16_t* __restrict__ nbr_all,
+                       int32_t* __restrict__ pair_i_all, int32_t* __restrict__ pair_j_all,
+                       int64_t* __restrict__ npairs) {
+    __shared__ uint32_t scan_lds[kSmallBlock / 64];
+    const int64_t s = blockIdx.y;
+    const int t = threadIdx.x, lane = t & 63, i0 = (int)blockIdx.x * kSmallBlock, i = i0 + t;
+    const uint32_t* cnt = cnt_all + s * st.row;
+    const uint16_t* row = nbr_all + 2 * s * st.nbr + (int64_t)(i < n ? i : 0) * kSmallNbr;
+    // this row's count and partners (read whatever the count) and the counts
+    // before and after the workgroup's rows load together
+    uint32_t c = i < n ? cnt[i] : 0u;
+    const uint4 lo = reinterpret_cast<const uint4*>(row)[0], hi = reinterpret_cast<const uint4*>(row)[1];
+    uint32_t before = 0, after = 0;
+#pragma unroll
+    for (int q = 0; q < (int)(kSmallMax / kSmallBlock); ++q) {
+        const int k = q * kSmallBlock + t;
+        const uint32_t v = k < n && (k < i0 || k >= i0 + kSmallBlock) ? cnt[k] : 0u;
+        before += k < i0 ? v : 0u;
+        after += k < i0 ? 0u : v;
+    }
+    uint32_t sum_before, sum_after, sum_own;
+    (void)small_exclusive_scan(before, scan_lds, &sum_before);
+    (void)small_exclusive_scan(after, scan_lds, &sum_after);
+    const uint32_t o = sum_before + small_exclusive_scan(c, scan_lds, &sum_own);
+    const uint32_t total = sum_before + sum_own + sum_after;
+    if (blockIdx.x == 0 && t == 0) npairs[s] = (int64_t)total;
+    if ((int64_t)total > st.pair) return;  // caller enlarges and calls again
+    int32_t* pair_i = pair_i_all + s * st.pair;
+    int32_t* pair_j = pair_j_all + s * st.pair;
+    if (c > 0 && c <= (uint32_t)kSmallNbr) {
+        const uint32_t w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        uint32_t v[kSmallNbr];
+#pragma unroll
+        for (int k = 0; k < kSmallNbr; ++k) v[k] = (uint32_t)k < c ? (w[k >> 1] >> (16 * (k & 1))) & 0xffffu : 0xffffffffu;
+        auto sort = [&](auto K) {
+            constexpr int N = decltype(K)::value;
+#pragma unroll
+            for (int a = 1; a < N; ++a)
+#pragma unroll
+                for (int b = a; b > 0; --b) {
+                    const uint32_t x = min(v[b - 1], v[b]), y = max(v[b - 1], v[b]);
+                    v[b - 1] = x;
+                    v[b] = y;
+                }
+        };
+        if (c <= 4) sort(std::integral_constant<int, 4>{});
+        else sort(std::integral_constant<int, kSmallNbr>{});
+#pragma unroll
+        for (int k = 0; k < kSmallNbr; ++k)
+            if ((uint32_t)k < c) {
+                pair_i[o + k] = i;
+                pair_j[o + k] = (int32_t)v[k];
+            }
+    }
+    // crowded rows, one after another by the whole wavefront
+    const float* x = x_all + s * st.pos;
+    const float* y = y_all + s * st.pos;
+    for (uint64_t left = __ballot(c > (uint32_t)kSmallNbr); left != 0; left &= left - 1) {
+        const int src = __ffsll((unsigned long long)left) - 1;
+        const int r = __shfl(i, src, 64);
+        const uint32_t rc = __shfl(c, src, 64);
+        uint32_t at = __shfl(o, src, 64);
+        const uint32_t end = at + rc;
+        const float xr = x[r], yr = y[r];
+        for (int j0 = r + 1; j0 < n && at < end; j0 += 64) {
+            const int j = j0 + lane;
+            const float xj = j < n ? x[j] : 0.0f, yj = j < n ? y[j] : 0.0f;
+            const bool hit = pair_hit<KIND>(m, j < n, xr, yr, xj, yj);
+            const uint64_t hits = __ballot(hit);
+            if (hit) {
+                const uint32_t k = at + (uint32_t)__popcll(hits & ((1ull << lane) - 1ull));
+                if (k < end) {
+                    pair_i[k] = r;
+                    pair_j[k] = j;
+                }
+            }
+            at += (uint32_t)__popcll(hits);
+        }
+    }
+}
+
 __global__ void zero_i64_kernel(int64_t* p, int64_t count) {
     for (int64_t k = threadIdx.x; k < count; k += blockDim.x) p[k] = 0;
 }
@@ -550,6 +765,39 @@ static int count_and_emit(lm_pairs_ws* ws, int32_t nsteps, int64_t n, const floa
     LM_LAUNCH(K_PAIR_EMIT, pair_emit_kernel<KIND>, grid, dim3(kBlock), 0, s, n, lon, lat, run, g, m, st,
               (const uint32_t*)ws->start, (const float4*)ws->recs, (const uint32_t*)ws->nbr_cnt,
               (const uint32_t*)ws->nbr, (const uint32_t*)ws->row_off, pair_i, pair_j);
+    LM_LAUNCH_CHECK();
+    return LM_OK;
+}
+
+// The search of a small population.  A table of 64 x 64 buckets up to 4,096
+// particles, 128 x 64 above: about one particle in each.  Four lanes per
+// particle while the workgroups they take still run at once (one fills a
+// CU's LDS), else one.
+template <int KIND>
+static int search_small(lm_pairs_ws* ws, int32_t nsteps, int64_t n, const float* lon, const float* lat,
+                        const CellGrid& g, const Metric& m, const Strides& st, int64_t* npairs, int32_t* pair_i,
+                        int32_t* pair_j, hipStream_t s) {
+    uint16_t* nbr = reinterpret_cast<uint16_t*>(ws->nbr);
+    const bool wide = (n + kSmallBlock / 4 - 1) / (kSmallBlock / 4) * nsteps <= 256;
+    const dim3 grid(grid_for(n, wide ? kSmallBlock / 4 : kSmallBlock), (unsigned)nsteps), block(kSmallBlock);
+    if (n <= 4096) {
+        if (wide)
+            LM_LAUNCH(K_PAIR_SMALL, (pair_small_count_kernel<KIND, 4096, 6, 6, 4>), grid, block, 0, s, (int)n, lon, lat,
+                      g, m, st, ws->nbr_cnt, nbr);
+        else
+            LM_LAUNCH(K_PAIR_SMALL, (pair_small_count_kernel<KIND, 4096, 6, 6, 1>), grid, block, 0, s, (int)n, lon, lat,
+                      g, m, st, ws->nbr_cnt, nbr);
+    } else {
+        if (wide)
+            LM_LAUNCH(K_PAIR_SMALL, (pair_small_count_kernel<KIND, (int)kSmallMax, 7, 6, 4>), grid, block, 0, s, (int)n,
+                      lon, lat, g, m, st, ws->nbr_cnt, nbr);
+        else
+            LM_LAUNCH(K_PAIR_SMALL, (pair_small_count_kernel<KIND, (int)kSmallMax, 7, 6, 1>), grid, block, 0, s, (int)n,
+                      lon, lat, g, m, st, ws->nbr_cnt, nbr);
+    }
+    LM_LAUNCH_CHECK();
+    LM_LAUNCH(K_EMIT_SMALL, pair_small_emit_kernel<KIND>, dim3(grid_for(n, kSmallBlock), (unsigned)nsteps), block, 0, s,
+              (int)n, lon, lat, m, st, (const uint32_t*)ws->nbr_cnt, (const uint16_t*)nbr, pair_i, pair_j, npairs);
     LM_LAUNCH_CHECK();
     return LM_OK;
 }
@@ -703,6 +951,14 @@ int lm_query_pairs_runs(lm_pairs_ws* ws, int32_t nsteps, int64_t n, const float*
     st.row = ws->row_stride;
     st.nbr = ws->n_max * lm::kNbr;
     st.pair = pair_stride;
+    if (n <= lm::kSmallMax && run == nullptr) {
+        switch (m.kind) {
+            case lm::kL2: return lm::search_small<lm::kL2>(ws, nsteps, n, lon, lat, g, m, st, npairs, pair_i, pair_j, s);
+            case lm::kL1: return lm::search_small<lm::kL1>(ws, nsteps, n, lon, lat, g, m, st, npairs, pair_i, pair_j, s);
+            case lm::kLinf: return lm::search_small<lm::kLinf>(ws, nsteps, n, lon, lat, g, m, st, npairs, pair_i, pair_j, s);
+            default: return lm::search_small<lm::kLp>(ws, nsteps, n, lon, lat, g, m, st, npairs, pair_i, pair_j, s);
+        }
+    }
     // two-level binning: one radix pass on the high bits of the bucket, then
     // a block per super-bucket sorts its fine buckets in LDS
     // 12 fine bits in LDS (13 above 2^22 buckets), the rest in one radix pass
