@@ -246,6 +246,14 @@ int lm_rps_prepare_runs(lm_rps_ws* ws, int32_t nsteps, int64_t n, const int32_t*
 int lm_rps_play(lm_rps_ws* ws, int32_t step, int64_t n, const int8_t* species_in,
                 int8_t* species_out, void* stream);
 
+/* Steps 0 .. nsteps - 1 of the last prepare in one call: species_out +
+ * s * out_stride (out_stride >= n) = the species after step s, the first from
+ * species_in; the same results as lm_rps_play(s) in turn.  No reference
+ * counterpart (the reference records every step's species in its own loop,
+ * interaction_simulator.py:107-110). */
+int lm_rps_play_steps(lm_rps_ws* ws, int32_t nsteps, int64_t n, const int8_t* species_in, int8_t* species_out,
+                      int64_t out_stride, void* stream);
+
 /* Size statistics of the interaction components of step `step` of the last
  * prepare, written to device int64[8]: components with at least one pair,
  * largest component (pairs), largest component (particles), total pairs,

@@ -88,6 +88,8 @@ enum KernelId {
     K_RPS_TILE,
     K_PAIR_SMALL,
     K_EMIT_SMALL,
+    K_RPS_SMALL,
+    K_PLAY_SMALL,
     K_NUM_KERNELS
 };
 bool timing_on();

@@ -53,8 +53,13 @@
 //            dependency rounds
 //   small    one lane per component of <= 32 pairs, replayed in order
 //   copy     particles without pairs keep their species
+//
+// Small populations (kSmallMax particles, no runs) take two kernels instead,
+// one for the whole prepare and one that replays all steps of a batch (see
+// "small populations" below).
 #include "lm_common.h"
 #include "lm_scan.h"
+#include "lm_small.h"
 #include "lm_sort.h"
 
 namespace lm {
@@ -1236,6 +1241,343 @@ rps_play_kernel(int64_t n, int64_t s, RpsArrays A, RpsStrides st, const int8_t* 
     }
 }
 
+// ---------------------------------------------------------------------------
+// small populations
+// ---------------------------------------------------------------------------
+// Up to kSmallMax particles the whole state of a step fits a workgroup, and
+// launches are what the general path's time goes to (24 steps of 10,000
+// particles: 78 prepare launches and 24 replays of 8 to 28 us).  No
+// components here:
+//   prepare  a workgroup per step: per pair its outcome bits and, for each of
+//            its two particles, the pairs before and after it that touch the
+//            particle
+//   play     one workgroup replays the batch's steps one after another.  A
+//            pair's result is a function of the results of the two pairs
+//            before it; the pairs are acyclic, so the sequential result is the
+//            one fixed point of playing pairs from each other's last results.
+//            From "nobody loses" as the first guess every pair plays once;
+//            then, round by round, only the pairs right after one whose result
+//            changed.  Values only travel where they change: 6,500 pairs whose
+//            longest chain is 126 settle in 10 to 18 rounds of ever fewer
+//            pairs (levels, one after another, would take 126).  A step of
+//            10,000 particles and 6,500 pairs takes about 11 us, where the
+//            general replay's launch takes 8 to 28; a run of 24 such steps
+//            from the lattice went from 1,070 to 635 us in all.
+// Pairs go in windows of kSmallWindow; a pair whose predecessor is in an
+// earlier window starts from the particle's species, which a window's last
+// pair at it updates.  A pair whose j is no other particle changes nothing.
+// rec: x = source at i | source at j << 16, y = next at i | next at j << 14 |
+// outcome bits << 28 | kSmallNoop; source = 2 * (pair in the window) + side,
+// or kSmallSpecies + particle; next = pair in the window or kSmallNone.
+// lend: i | j << 14 | kSmallValid.
+constexpr uint32_t kSmallValid = 0x80000000u, kSmallNoop = 0x80000000u;
+constexpr int kSmallPairs = 8;  // pairs per thread in a window
+constexpr uint32_t kSmallWindow = kSmallBlock * kSmallPairs;
+constexpr uint32_t kSmallSpecies = 2 * kSmallWindow;
+constexpr uint32_t kSmallNone = kSmallWindow;
+static_assert(kSmallMax <= 1 << 14 && kSmallSpecies + kSmallMax <= 1 << 16 && kSmallNone < 1 << 14, "record fields");
+
+__global__ void __launch_bounds__(kSmallBlock)
+rps_small_kernel(uint32_t n, const int32_t* __restrict__ pi_all, const int32_t* __restrict__ pj_all,
+                 const int64_t* __restrict__ npairs, RpsArrays A, RpsStrides st, double pRS, double pPR, double pSP,
+                 uint64_t k0, uint64_t k1, uint64_t step0) {
+    __shared__ uint32_t ends[kSmallMax];                   // counts, then ends of the lists of pairs by j
+    __shared__ uint32_t rbeg[kSmallMax], rend[kSmallMax];  // rows: the pairs by i
+    __shared__ uint32_t scan_lds[kSmallBlock / 64];
+    const int64_t s = blockIdx.x, po = s * st.pair;
+    const uint32_t t = threadIdx.x;
+    const int64_t P64 = step_pairs(npairs, s, st.pair);
+    const uint32_t P = P64 < 0 ? 0u : (uint32_t)P64;
+    if (t == 0) A.plen[s] = P;
+    const int32_t* pi = pi_all + po;
+    const int32_t* pj = pj_all + po;
+    uint32_t* list = reinterpret_cast<uint32_t*>(A.deps + po);  // pairs by j
+    for (uint32_t v = t; v < n; v += kSmallBlock) ends[v] = rbeg[v] = rend[v] = 0u;
+    __syncthreads();
+    for (uint32_t k = t; k < P; k += kSmallBlock) {
+        const uint32_t a = (uint32_t)pi[k], b = (uint32_t)pj[k];
+        const uint32_t before = (uint32_t)pi[k > 0 ? k - 1 : 0], after = (uint32_t)pi[k + 1 < P ? k + 1 : k];
+        if (a >= n) continue;
+        if (k == 0 || before != a) rbeg[a] = k;
+        if (k + 1 == P || after != a) rend[a] = k + 1;
+        if (b < n && b != a) atomicAdd(&ends[b], 1u);
+    }
+    __syncthreads();
+    small_scan_array(ends, n, scan_lds);
+    for (uint32_t k = t; k < P; k += kSmallBlock) {
+        const uint32_t a = (uint32_t)pi[k], b = (uint32_t)pj[k];
+        if (a < n && b < n && b != a) list[atomicAdd(&ends[b], 1u)] = k;  // the cursor ends at the list's end
+    }
+    __threadfence_block();
+    __syncthreads();
+    // the pairs before and after k at particle v, 2 * pair + side (kUnset: none),
+    // of those whose j is v
+    auto around = [&](uint32_t v, uint32_t k, uint32_t* prev, uint32_t* next) {
+        uint32_t lo = kUnset, hi = kUnset;
+        for (uint32_t q = v > 0 ? ends[v - 1] : 0u; q < ends[v]; ++q) {
+            const uint32_t e = list[q];
+            if (e < k) lo = lo == kUnset ? e : max(lo, e);
+            else if (e > k) hi = min(hi, e);
+        }
+        *prev = lo == kUnset ? kUnset : 2u * lo + 1u;
+        *next = hi == kUnset ? kUnset : 2u * hi + 1u;
+    };
+    auto source = [&](uint32_t prev, uint32_t k, uint32_t v) {
+        const bool here = prev != kUnset && (prev >> 1) / kSmallWindow == k / kSmallWindow;
+        return here ? prev % kSmallSpecies : kSmallSpecies + v;
+    };
+    auto after_it = [&](uint32_t next, uint32_t k) {
+        const bool here = next != kUnset && (next >> 1) / kSmallWindow == k / kSmallWindow;
+        return here ? (next >> 1) % kSmallWindow : kSmallNone;
+    };
+    for (uint32_t k = t; k < P; k += kSmallBlock) {
+        const uint32_t a = (uint32_t)pi[k], b = (uint32_t)pj[k];
+        uint2 r = make_uint2(0u, 0u);
+        uint32_t who = 0u;
+        if (a < n) {
+            const double u = u01_from_u64(philox4x64_10(k, step0 + (uint64_t)s, kStreamPairs, 0, k0, k1).v[0]);
+            const uint32_t bits = (u < pRS ? 1u : 0u) | (u < pPR ? 2u : 0u) | (u < pSP ? 4u : 0u);
+            const bool two = b < n && b != a;
+            uint32_t prev, next;
+            around(a, k, &prev, &next);
+            if (k > rbeg[a]) prev = 2u * (k - 1u);  // i's row is one run of pairs
+            if (k + 1u < rend[a]) next = 2u * (k + 1u);
+            r.x = source(prev, k, a);
+            r.y = after_it(next, k) | bits << 28;
+            if (two) {
+                around(b, k, &prev, &next);
+                if (rend[b] > rbeg[b]) {  // j's own row, all of it before or after k
+                    if (rend[b] <= k && (prev == kUnset || 2u * (rend[b] - 1u) > prev)) prev = 2u * (rend[b] - 1u);
+                    if (rbeg[b] > k && (next == kUnset || 2u * rbeg[b] < next)) next = 2u * rbeg[b];
+                }
+                r.x |= source(prev, k, b) << 16;
+                r.y |= after_it(next, k) << 14;
+            } else {
+                r.x |= r.x << 16;
+                r.y |= kSmallNone << 14 | kSmallNoop;
+            }
+            who = a | (two ? b : a) << 14 | kSmallValid;
+        }
+        A.rec[po + k] = r;
+        A.lend[po + k] = who;
+    }
+}
+
+// play_pair for every pair of species indices (species - 1, or 3 for any code
+// that never interacts): two bits per pair at 2 * (4 ui + uj) for i's new
+// index (x) and j's (y).
+__device__ __forceinline__ uint2 small_table(uint32_t bits, bool two) {
+    uint2 t = make_uint2(0u, 0u);
+    for (int ui = 0; ui < 4; ++ui)
+        for (int uj = 0; uj < 4; ++uj) {
+            int si = ui + 1, sj = uj + 1;  // 4 is outside {1, 2, 3}
+            if (two) play_pair(si, sj, bits);
+            t.x |= (uint32_t)(si - 1) << (2 * (4 * ui + uj));
+            t.y |= (uint32_t)(sj - 1) << (2 * (4 * ui + uj));
+        }
+    return t;
+}
+
+// A barrier that waits for this wavefront's LDS operations only: records on
+// their way from memory, and species on their way there, stay in flight.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+__global__ void __launch_bounds__(kSmallBlock)
+rps_play_small_kernel(uint32_t n, int64_t s0, int nsteps, RpsArrays A, RpsStrides st, const int8_t* sp_in,
+                      int8_t* sp_out, int64_t out_stride) {
+    // the window's results, two bytes per pair, then the species indices
+    __shared__ __align__(16) uint8_t val[kSmallSpecies + kSmallMax];
+    __shared__ uint2 recs[kSmallWindow];
+    __shared__ uint16_t queue[2][kSmallWindow];  // pairs to play in this round and the next
+    __shared__ uint32_t queued[3];               // of this round, the next, the one after
+    __shared__ uint2 tables[9];
+    uint8_t* sp = val + kSmallSpecies;
+    uint16_t* res = reinterpret_cast<uint16_t*>(val);
+    const uint32_t t = threadIdx.x;
+    if (t < 9) tables[t] = small_table(t & 7u, t < 8u);
+    if (t < 3) queued[t] = 0u;
+    for (uint32_t v = t; v < n; v += kSmallBlock) {
+        const uint32_t u = (uint32_t)(sp_in[v] - 1);
+        sp[v] = (uint8_t)(u < 3u ? u : 3u);
+    }
+    uint2 next_rec[kSmallPairs];
+    uint32_t next_who[kSmallPairs];
+    auto load = [&](int64_t s, uint32_t w, uint32_t P) {
+        const uint2* rec = A.rec + s * st.pair + w;  // uniform
+        const uint32_t* lend = A.lend + s * st.pair + w;
+        const uint32_t left = P - w;
+#pragma unroll
+        for (int q = 0; q < kSmallPairs; ++q) {
+            const uint32_t k = q * kSmallBlock + t;
+            const uint32_t kc = k < left ? k : 0u;
+            next_rec[q] = rec[kc];
+            next_who[q] = k < left ? lend[kc] : 0u;
+        }
+    };
+    // plays pair p from the results in LDS; true if its result changed
+    auto play = [&](uint32_t p, uint2 r) {
+        const uint32_t a = __hip_atomic_load(val + (r.x & 0xffffu), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        const uint32_t b = __hip_atomic_load(val + (r.x >> 16), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        const uint32_t was = __hip_atomic_load(res + p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        const uint2 tab = tables[(r.y & kSmallNoop) ? 8u : (r.y >> 28) & 7u];
+        const uint32_t at = a << 3 | b << 1;
+        const uint32_t out = ((tab.x >> at) & 3u) | ((tab.y >> at) & 3u) << 8;
+        if (out == was) return false;
+        __hip_atomic_store(res + p, (uint16_t)out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        return true;
+    };
+    // appends the pairs after the flagged ones to a queue, one LDS add per
+    // wavefront and call; pairs past its end only count
+    auto push_after = [&](bool changed, uint32_t y, uint16_t* q, uint32_t* count) {
+        const uint32_t ni = y & 0x3fffu, nj = (y >> 14) & 0x3fffu, lane = t & 63u;
+        const uint64_t mi = __ballot(changed && ni < kSmallNone), mj = __ballot(changed && nj < kSmallNone);
+        if ((mi | mj) == 0) return;
+        const uint32_t ci = (uint32_t)__popcll(mi);
+        uint32_t base = 0;
+        if (lane == 0) base = atomicAdd(count, ci + (uint32_t)__popcll(mj));
+        base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+        const uint64_t below = (1ull << lane) - 1ull;
+        const uint32_t ai = base + (uint32_t)__popcll(mi & below), aj = base + ci + (uint32_t)__popcll(mj & below);
+        if ((mi >> lane & 1ull) && ai < kSmallWindow) q[ai] = (uint16_t)ni;
+        if ((mj >> lane & 1ull) && aj < kSmallWindow) q[aj] = (uint16_t)nj;
+    };
+    uint32_t P = (uint32_t)A.plen[s0];
+    load(s0, 0, P);  // (a step without pairs reads its first record, which counts for nothing)
+    __syncthreads();
+    for (int s = 0; s < nsteps; ++s) {
+        const bool more = s + 1 < nsteps;
+        const uint32_t P_next = more ? (uint32_t)A.plen[s0 + s + 1] : 0u;
+        if (P == 0 && more) load(s0 + s + 1, 0, P_next);
+        for (uint32_t w = 0; w < P; w += kSmallWindow) {
+            const uint32_t most = min(P - w, kSmallWindow);
+            uint32_t who[kSmallPairs], was[kSmallPairs], after[kSmallPairs];
+            // first guess: both keep their species, which are then every
+            // pair's inputs, so it plays at once
+#pragma unroll
+            for (int q = 0; q < kSmallPairs; ++q) {
+                who[q] = next_who[q];
+                was[q] = (uint32_t)sp[who[q] & 0x3fffu] | (uint32_t)sp[(who[q] >> 14) & 0x3fffu] << 8;
+            }
+            uint32_t changed = 0;
+#pragma unroll
+            for (int q = 0; q < kSmallPairs; ++q) {
+                after[q] = next_rec[q].y;
+                const uint2 tab = tables[(after[q] & kSmallNoop) ? 8u : (after[q] >> 28) & 7u];
+                const uint32_t at = (was[q] & 3u) << 3 | (was[q] >> 8) << 1;
+                const uint32_t out = ((tab.x >> at) & 3u) | ((tab.y >> at) & 3u) << 8;
+                if (who[q] & kSmallValid) {
+                    recs[q * kSmallBlock + t] = next_rec[q];
+                    res[q * kSmallBlock + t] = (uint16_t)out;
+                    changed |= out != was[q] ? 1u << q : 0u;
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < kSmallPairs; ++q)
+                if ((uint32_t)q * kSmallBlock < most) push_after(changed >> q & 1u, after[q], queue[1], &queued[1]);
+            // the next window's records, or the next step's first, meanwhile
+            if (w + kSmallWindow < P) load(s0 + s, w + kSmallWindow, P);
+            else if (more) load(s0 + s + 1, 0, P_next);
+            lds_barrier();
+            // a round per link of the longest chain of changes: at most one per
+            // pair (a list not sorted by (i, j), outside the contract, ends there)
+            for (uint32_t round = 1; round <= most; ++round) {
+                const uint32_t now = round % 3, then = (round + 1) % 3;
+                const uint32_t count = queued[now];
+                if (count == 0u) break;  // uniform: the last round's barrier precedes the read
+                if (t == 0) queued[(round + 2) % 3] = 0u;
+                if (count <= kSmallWindow) {
+                    for (uint32_t k0 = 0; k0 < count; k0 += kSmallBlock) {
+                        const bool live = k0 + t < count;
+                        const uint32_t p = live ? queue[round & 1u][k0 + t] : 0u;
+                        const uint2 r = recs[p];
+                        push_after(live && play(p, r), r.y, queue[(round + 1) & 1u], &queued[then]);
+                    }
+                } else {  // more than the queue holds: every pair
+                    for (uint32_t k0 = 0; k0 < most; k0 += kSmallBlock) {
+                        const bool live = k0 + t < most && (A.lend[(s0 + s) * st.pair + w + k0 + t] & kSmallValid) != 0u;
+                        const uint32_t p = live ? k0 + t : 0u;
+                        const uint2 r = recs[p];
+                        push_after(live && play(p, r), r.y, queue[(round + 1) & 1u], &queued[then]);
+                    }
+                }
+                lds_barrier();
+            }
+#pragma unroll
+            for (int q = 0; q < kSmallPairs; ++q) {
+                if ((who[q] & kSmallValid) == 0u) continue;
+                const uint32_t out = res[q * kSmallBlock + t], y = recs[q * kSmallBlock + t].y;
+                if ((y & 0x3fffu) == kSmallNone) sp[who[q] & 0x3fffu] = (uint8_t)out;
+                if ((y >> 14 & 0x3fffu) == kSmallNone && !(y & kSmallNoop)) sp[who[q] >> 14 & 0x3fffu] = (uint8_t)(out >> 8);
+            }
+            if (t < 3) queued[t] = 0u;
+            lds_barrier();
+        }
+        int8_t* out = sp_out + s * out_stride;
+        auto code = [&](uint32_t v) { return sp[v] < 3u ? (int8_t)(sp[v] + 1u) : sp_in[v]; };
+        if ((((uintptr_t)out | n) & 3u) == 0) {
+            for (uint32_t v = t; v < n / 4u; v += kSmallBlock) {
+                const uint32_t w = reinterpret_cast<const uint32_t*>(sp)[v];
+                if ((w & w >> 1 & 0x01010101u) == 0u)
+                    reinterpret_cast<uint32_t*>(out)[v] = w + 0x01010101u;
+                else
+                    for (uint32_t q = 0; q < 4; ++q) out[4u * v + q] = code(4u * v + q);
+            }
+        } else {
+            for (uint32_t v = t; v < n; v += kSmallBlock) out[v] = code(v);
+        }
+        lds_barrier();  // read before the next step's last pairs write
+        P = P_next;
+    }
+}
+
+// Component statistics of a step that rps_small prepared (diagnostic): one
+// workgroup joins its pairs in an LDS forest.
+__global__ void __launch_bounds__(kSmallBlock)
+rps_small_stats_kernel(uint32_t n, int64_t s, RpsArrays A, RpsStrides st, int64_t* __restrict__ stats) {
+    __shared__ uint32_t par[kSmallMax], cp[kSmallMax], cs[kSmallMax];  // parents; pairs and particles by root
+    const uint32_t t = threadIdx.x, P = (uint32_t)A.plen[s];
+    for (uint32_t v = t; v < n; v += kSmallBlock) {
+        par[v] = v;
+        cp[v] = cs[v] = 0u;
+    }
+    __syncthreads();
+    for (uint32_t k = t; k < P; k += kSmallBlock) {
+        const uint32_t r = A.lend[s * st.pair + k];
+        const uint32_t a = r & 0x3fffu, b = (r >> 14) & 0x3fffu;
+        if (!(r & kSmallValid)) continue;
+        cs[a] = cs[b] = 1u;  // has pairs
+        if (a != b) lds_unite(par, a, b);
+    }
+    __syncthreads();
+    for (uint32_t k = t; k < P; k += kSmallBlock) {
+        const uint32_t r = A.lend[s * st.pair + k];
+        if (r & kSmallValid) atomicAdd(&cp[lds_find(par, r & 0x3fffu)], 1u);
+    }
+    __syncthreads();
+    uint32_t has[kSmallMax / kSmallBlock];
+#pragma unroll
+    for (int q = 0; q < (int)(kSmallMax / kSmallBlock); ++q) {
+        const uint32_t v = q * kSmallBlock + t;
+        has[q] = v < n ? cs[v] : 0u;
+    }
+    __syncthreads();
+    for (uint32_t v = t; v < n; v += kSmallBlock) cs[v] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < (int)(kSmallMax / kSmallBlock); ++q)
+        if (has[q]) atomicAdd(&cs[lds_find(par, q * kSmallBlock + t)], 1u);
+    __syncthreads();
+    for (uint32_t v = t; v < n; v += kSmallBlock) {
+        const unsigned long long p = cp[v], c = cs[v], wide = p > kNarrowPairs;
+        if (p == 0) continue;
+        const unsigned long long add[8] = {1, p, c, p, wide, wide * p, wide * c, c};
+        for (int q = 0; q < 8; ++q) {
+            if (q == 1 || q == 2) atomicMax((unsigned long long*)&stats[q], add[q]);
+            else atomicAdd((unsigned long long*)&stats[q], add[q]);
+        }
+    }
+}
+
 // Component size statistics of one prepared step (diagnostic, on request):
 // stats = {components, max pairs in one, max particles in one, total pairs,
 //          wide components, their pairs, their particles, particles with pairs}.
@@ -1296,6 +1638,7 @@ struct lm_rps_ws {
     uint32_t* tile_off = nullptr;  // [steps][tiles1] first pair of each particle tile
     int tiles1 = 0;                // tiles of n_max particles, plus one
     int64_t run_off_cap = 0;
+    bool small = false;            // the last prepare was rps_small's
     unsigned play_wide = lm::kPlayWideBlocks;      // replay workgroups on wide components
     unsigned play_narrow = lm::kPlayNarrowBlocks;  // replay workgroups on small components (64 each)
 };
@@ -1491,6 +1834,18 @@ static int rps_prepare_impl(lm_rps_ws* ws, int32_t nsteps, int64_t n, const int3
     const lm::RpsStrides sp{ws->row, pair_stride};
     lm::RpsArrays& A = ws->A;
     const unsigned S = (unsigned)nsteps;
+    // one workgroup holds a small step; without pairs the general replay's
+    // copy is all there is to do, and an ensemble's runs have keys of their own
+    ws->small = n <= lm::kSmallMax && run == nullptr && pair_stride > 0;
+    if (ws->small) {
+        LM_LAUNCH(lm::K_RPS_SMALL, lm::rps_small_kernel, dim3(S), dim3(lm::kSmallBlock), 0, s, (uint32_t)n, pair_i,
+                  pair_j, npairs, A, sp, pRS, pPR, pSP, key0, key1, step0);
+        LM_LAUNCH_CHECK();
+        ws->pair_stride_used = pair_stride;
+        ws->last_n = n;
+        ws->last_steps = nsteps;
+        return LM_OK;
+    }
     const unsigned nbp = lm::grid_for(n);
     const int ntiles = (int)((n + lm::kTile - 1) / lm::kTile);
     LM_REQUIRE(ntiles + 1 <= ws->tiles1, LM_ERR_ARG, "internal: tile offsets");
@@ -1581,6 +1936,29 @@ static int rps_prepare_impl(lm_rps_ws* ws, int32_t nsteps, int64_t n, const int3
     return LM_OK;
 }
 
+// Steps step .. step + nsteps - 1 of the last prepare, species_out + k * stride
+// after step step + k: one launch for a small population, else one per step.
+static int rps_play_range(lm_rps_ws* ws, int32_t step, int32_t nsteps, int64_t n, const int8_t* species_in,
+                          int8_t* species_out, int64_t stride, hipStream_t s) {
+    const lm::RpsStrides sp{ws->row, ws->pair_stride_used};
+    if (ws->small) {
+        LM_LAUNCH(lm::K_PLAY_SMALL, lm::rps_play_small_kernel, dim3(1), dim3(lm::kSmallBlock), 0, s, (uint32_t)n,
+                  (int64_t)step, (int)nsteps, ws->A, sp, species_in, species_out, stride);
+        LM_LAUNCH_CHECK();
+        return LM_OK;
+    }
+    const unsigned nwide = ws->pair_stride_used > 0 ? ws->play_wide : 0u;
+    const unsigned nnarrow = ws->pair_stride_used > 0 ? ws->play_narrow : 0u;
+    const unsigned ncopy = (unsigned)((n + 64 * lm::kCopyItems - 1) / (64 * lm::kCopyItems));
+    for (int32_t k = 0; k < nsteps; ++k) {
+        const int8_t* in = k == 0 ? species_in : species_out + (k - 1) * stride;
+        LM_LAUNCH(lm::K_RPS_PLAY, lm::rps_play_kernel, dim3(nwide + nnarrow + ncopy), dim3(64), 0, s, n,
+                  (int64_t)(step + k), ws->A, sp, in, species_out + k * stride, nwide, nnarrow);
+        LM_LAUNCH_CHECK();
+    }
+    return LM_OK;
+}
+
 int lm_rps_prepare(lm_rps_ws* ws, int32_t nsteps, int64_t n, const int32_t* pair_i, const int32_t* pair_j,
                    int64_t pair_stride, const int64_t* npairs, double pRS, double pPR, double pSP,
                    uint64_t key0, uint64_t key1, uint64_t step0, void* stream) {
@@ -1605,15 +1983,21 @@ int lm_rps_play(lm_rps_ws* ws, int32_t step, int64_t n, const int8_t* species_in
                ws->last_steps, (long long)ws->last_n);
     if (n == 0) return LM_OK;
     LM_REQUIRE(species_in && species_out, LM_ERR_ARG, "NULL species");
-    hipStream_t s = (hipStream_t)stream;
-    lm::RpsStrides sp{ws->row, ws->pair_stride_used};
-    const unsigned nwide = ws->pair_stride_used > 0 ? ws->play_wide : 0u;
-    const unsigned nnarrow = ws->pair_stride_used > 0 ? ws->play_narrow : 0u;
-    const unsigned ncopy = (unsigned)((n + 64 * lm::kCopyItems - 1) / (64 * lm::kCopyItems));
-    LM_LAUNCH(lm::K_RPS_PLAY, lm::rps_play_kernel, dim3(nwide + nnarrow + ncopy), dim3(64), 0, s, n,
-              (int64_t)step, ws->A, sp, species_in, species_out, nwide, nnarrow);
-    LM_LAUNCH_CHECK();
-    return LM_OK;
+    return rps_play_range(ws, step, 1, n, species_in, species_out, 0, (hipStream_t)stream);
+}
+
+int lm_rps_play_steps(lm_rps_ws* ws, int32_t nsteps, int64_t n, const int8_t* species_in, int8_t* species_out,
+                      int64_t out_stride, void* stream) {
+    LM_REQUIRE(ws != nullptr, LM_ERR_ARG, "workspace is NULL");
+    LM_REQUIRE(nsteps >= 0, LM_ERR_ARG, "negative step count");
+    if (nsteps == 0) return LM_OK;
+    LM_REQUIRE(n == ws->last_n && nsteps <= ws->last_steps, LM_ERR_ARG,
+               "%d steps / n %lld do not match the last prepare (%d steps, n %lld)", nsteps, (long long)n,
+               ws->last_steps, (long long)ws->last_n);
+    if (n == 0) return LM_OK;
+    LM_REQUIRE(species_in && species_out, LM_ERR_ARG, "NULL species");
+    LM_REQUIRE(nsteps == 1 || out_stride >= n, LM_ERR_ARG, "species stride < n");
+    return rps_play_range(ws, 0, nsteps, n, species_in, species_out, out_stride, (hipStream_t)stream);
 }
 
 int lm_rps_ws_reserve(lm_rps_ws* ws, int64_t pairs_per_step, void* stream) {
@@ -1647,7 +2031,11 @@ int lm_rps_component_stats(lm_rps_ws* ws, int32_t step, int64_t* out8, void* str
     LM_LAUNCH_CHECK();
     if (ws->last_n > 0 && ws->last_steps > 0 && ws->pair_stride_used > 0) {
         lm::RpsStrides sp{ws->row, ws->pair_stride_used};
-        hipLaunchKernelGGL(lm::rps_stats_kernel, dim3(256), dim3(lm::kBlock), 0, s, (int64_t)step, ws->A, sp,
+        if (ws->small)
+            hipLaunchKernelGGL(lm::rps_small_stats_kernel, dim3(1), dim3(lm::kSmallBlock), 0, s, (uint32_t)ws->last_n,
+                               (int64_t)step, ws->A, sp, out8);
+        else
+            hipLaunchKernelGGL(lm::rps_stats_kernel, dim3(256), dim3(lm::kBlock), 0, s, (int64_t)step, ws->A, sp,
                            out8);
         LM_LAUNCH_CHECK();
     }

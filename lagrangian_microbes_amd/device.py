@@ -451,6 +451,18 @@ class RPSUpdater:
         require(species_out, torch.int8, numel=n, name="species_out")
         check(lib().lm_rps_play(self._ws, int(step), n, ptr(species_in), ptr(species_out), stream_ptr()))
 
+    def play_steps(self, steps, species_in, rec_species):
+        """Steps 0 .. steps - 1 of the last prepare: rec_species[s] (int8
+        [>= steps, n], each row contiguous) = the species after step s."""
+        n = species_in.numel()
+        require(species_in, torch.int8, name="species_in")
+        if (rec_species.dim() != 2 or rec_species.dtype != torch.int8 or rec_species.device.type != "cuda"
+                or rec_species.shape[0] < steps or rec_species.shape[1] != n
+                or (n > 1 and rec_species.stride(1) != 1)):
+            raise ValueError(f"rec_species must be an int8 GPU tensor [>= {steps}, {n}] with contiguous rows")
+        check(lib().lm_rps_play_steps(self._ws, int(steps), n, ptr(species_in), ptr(rec_species),
+                                      rec_species.stride(0), stream_ptr()))
+
     def component_stats(self, step=0):
         """Component sizes of step ``step`` of the last prepare (a ComponentStats)."""
         check(lib().lm_rps_component_stats(self._ws, int(step), ptr(self._stats), stream_ptr()))

@@ -130,7 +130,13 @@ class InteractionEngine:
         species.copy_(rec_species[S - 1])
 
     def _play_steps(self, b, S, species, rec_species):
-        sp_in = species
+        n = species.numel()
+        if (isinstance(rec_species, torch.Tensor) and rec_species.dim() == 2 and rec_species.dtype == torch.int8
+                and rec_species.is_cuda and rec_species.shape[0] >= S and rec_species.shape[1] == n
+                and rec_species.stride(0) >= n and rec_species.stride(1) == 1):
+            self.rps_sets[b].play_steps(S, species, rec_species)
+            return
+        sp_in = species  # rows of another form: one call per step
         for s in range(S):
             self.rps_sets[b].play(s, sp_in, rec_species[s])
             sp_in = rec_species[s]
@@ -154,11 +160,11 @@ class InteractionEngine:
         while True:
             self.prepare_set(0, rec_x, rec_y, params, key, step0)
             cnt = self.npairs[:S]
-            sp_in = species
-            for s in range(S):
-                out = rec_species[s] if rec_species is not None else species
-                self.rps.play(s, sp_in, out)
-                sp_in = out
+            if rec_species is not None:
+                self._play_steps(0, S, species, rec_species)
+            else:
+                for s in range(S):
+                    self.rps.play(s, species, species)
             if self.fits(self.worst_count(0, S)):
                 if rec_species is not None:
                     species.copy_(rec_species[S - 1])

@@ -37,3 +37,95 @@ def test_pairs_of_a_crowd(gpu, n):
     gi, gj = gpu_pairs(x, y, R)
     bi, bj = oracle.pairs_bruteforce(x, y, R)
     assert np.array_equal(gi, bi) and np.array_equal(gj, bj)
+
+
+def star_and_chain(n):
+    pairs = {(0, k) for k in range(1, n)} | {(k, k + 1) for k in range(n - 1)}
+    return np.array(sorted(pairs), dtype=np.int32)
+
+
+@pytest.mark.parametrize("n", [2, 1025, 12288, 12289])
+def test_rps_star_and_chain(gpu, n):
+    # every pair waits for another: one play after the other, several windows of pairs
+    arr = star_and_chain(n)
+    sp = np.random.default_rng(n).integers(0, 5, n).astype(np.int8)
+    args = (0.5, 0.6, 0.4, (n, 1), 3)
+    g, up = gpu_rps(sp, arr[:, 0], arr[:, 1], *args)
+    assert np.array_equal(g, oracle.rps_sequential(sp, arr[:, 0], arr[:, 1], *args))
+    st = up.component_stats()
+    assert st.components == 1 and st.pairs == st.max_pairs == len(arr) and st.touched == st.max_particles == n
+
+
+@pytest.mark.parametrize("n", [900, 20000])
+def test_rps_pairs_in_any_direction(gpu, n):
+    # sorted by (i, j), with j below i, on itself and out of range as well
+    rng = np.random.default_rng(n)
+    a, b = rng.integers(0, n, (2, 2 * n))
+    b[::50] = n + 3
+    b[25::50] = -1
+    b[10::50] = a[10::50]
+    arr = np.unique(np.stack([a, b], 1), axis=0).astype(np.int32)
+    sp = rng.integers(1, 4, n).astype(np.int8)
+    args = (0.5, 0.6, 0.4, (5, 1), 3)
+    g, _ = gpu_rps(sp, arr[:, 0], arr[:, 1], *args)
+    ref = sp.copy()
+    u = oracle.philox_uniforms(len(arr), 0, 3, 0, 0, 5, 1)
+    p = {(1, 3): 0.5, (2, 1): 0.6, (3, 2): 0.4}  # (winner, loser) of a forward outcome
+    for k, (i, j) in enumerate(arr.tolist()):
+        if 0 <= j < n and ref[i] != ref[j]:
+            si, sj = int(ref[i]), int(ref[j])
+            win, lose = (si, sj) if (si, sj) in p else (sj, si)
+            w = win if u[k] < p[win, lose] else lose
+            ref[i] = ref[j] = w
+    assert np.array_equal(g, ref)
+
+
+@pytest.mark.parametrize("n,out", [(9001, 9001), (9000, 9016), (15000, 15000)])
+def test_play_steps_matches_single_steps(gpu, n, out):
+    rng = np.random.default_rng(n)
+    S, cap = 5, 2 * n
+    pi, pj = np.zeros((S, cap), np.int32), np.zeros((S, cap), np.int32)
+    counts = np.zeros(S, np.int64)
+    for s in range(S):
+        m = [n, 0, 3, 2 * n, n // 2][s]
+        a, b = random_pairs(rng, n, max(m, 1))
+        pi[s, :m], pj[s, :m], counts[s] = a[:m], b[:m], m
+    counts[4] = cap + 1  # too many for the buffers: the step changes nothing
+    sp = rng.integers(1, 4, n).astype(np.int8)
+    up = dev.RPSUpdater(n, steps_max=S)
+    up.prepare(n, T(pi), T(pj), T(counts), 0.55, 0.5, 0.45, (3, 4), 17)
+    rec = torch.zeros((S, out), dtype=torch.int8, device="cuda")[:, :n]
+    up.play_steps(S, T(sp), rec)
+    ref = sp
+    for s in range(S):
+        if s < 4:
+            ref = oracle.rps_sequential(ref, pi[s, :counts[s]], pj[s, :counts[s]], 0.55, 0.5, 0.45, (3, 4), 17 + s)
+        assert np.array_equal(rec[s].cpu().numpy(), ref), s
+    one = rec[2].clone()
+    up.play(3, one, one)  # a step by itself, in place
+    assert torch.equal(one, rec[3])
+
+
+@pytest.mark.parametrize("seed", [0, 1])
+def test_general_replay_of_every_component_size(gpu, seed):
+    # components of 2 to 3,000 particles among as many without pairs, above the small kernels' sizes
+    rng = np.random.default_rng(seed)
+    sizes = [2, 3, 5, 9] * 50 + [12, 40, 100] * 10 + [60] * 3 + [400, 1500] + [3000]
+    n = 20000
+    perm, pairs, at = rng.permutation(n), set(), 0
+    for s in sizes:
+        ids = perm[at:at + s]
+        at += s
+        for a in range(1, s):
+            b = int(rng.integers(0, a))
+            pairs.add((int(min(ids[a], ids[b])), int(max(ids[a], ids[b]))))
+        for _ in range(12 * s if s == 60 else s):
+            a, b = (int(v) for v in rng.choice(ids, 2, replace=False))
+            pairs.add((min(a, b), max(a, b)))
+    arr = np.array(sorted(pairs), dtype=np.int32)
+    sp = rng.integers(1, 4, n).astype(np.int8)
+    args = (0.5, 0.6, 0.4, (seed, 9), 21)
+    g, up = gpu_rps(sp, arr[:, 0], arr[:, 1], *args)
+    assert np.array_equal(g, oracle.rps_sequential(sp, arr[:, 0], arr[:, 1], *args))
+    st = up.component_stats()
+    assert st.components == len(sizes) and st.pairs == len(arr) and st.touched == at
