@@ -31,6 +31,8 @@ logger = logging.getLogger(__name__)
 
 # Smallest chunk the tapered end of a pipelined run uses.
 TAPER_MIN = 8
+# Largest population whose batches take a launch per phase (kSmallMax of liblm).
+SMALL_POPULATION = 12288
 
 
 def chunk_schedule(total, chunk, taper_min=TAPER_MIN):
@@ -147,6 +149,8 @@ class FusedRunner:
         nsets = self.PIPELINE_SETS
         main = torch.cuda.current_stream(self.device)
         side, adv = self._side, self._adv
+        # a small population's replay is one launch: the caller's stream does
+        play = self._play if self.n > SMALL_POPULATION else main
         sizes = chunk_schedule(total, self.chunk)
         if max(sizes) > self.chunk:  # the chunk buffers hold self.chunk steps
             raise RuntimeError(f"chunk schedule exceeds the buffers: {sizes}")
@@ -174,10 +178,10 @@ class FusedRunner:
         # The events are the runner's own, recorded again every chunk: a set's
         # event is re-recorded only after every wait on its previous record
         # has been issued (chunk c + 3 reuses chunk c's set)
-        ev_adv, ev_prep, ev_play, ev_count, ev_join = self._events
+        ev_adv, ev_prep, ev_play, ev_count, ev_replay, ev_join = self._events
         ev_join[0].record(main)          # the state as the caller left it
-        side.wait_event(ev_join[0])
-        adv.wait_event(ev_join[0])
+        for st in {side, adv, play} - {main}:
+            st.wait_event(ev_join[0])
 
         def advect(c):
             b, k = c % nsets, sizes[c]
@@ -203,21 +207,12 @@ class FusedRunner:
                 ev.record(side)
                 prepared[c] = ev
 
-        # chunk 0's preparation goes out before chunk 1's advection: it waits
-        # for nothing else
-        advect(0)
-        group(0)
-        if len(sizes) > 1:
-            advect(1)
-        backup, worst_host = self._backup, self._worst_host
-        for c, k in enumerate(sizes):
-            b = c % nsets
-            if c + 1 < len(sizes):
-                group(c + 1)
-            if c + 2 < len(sizes):
-                advect(c + 2)
-            main.wait_event(prepared[c])
-            rx, ry, rs = recs(c)
+        def replay(c):
+            b, k = c % nsets, sizes[c]
+            play.wait_event(prepared[c])
+            if c > 0 and play is not main:  # the callback may read the species
+                play.wait_event(played[(c - 1) % nsets])
+            rs = recs(c)[2]
             # The replay goes out before the host has seen the chunk's pair
             # counts, so it starts as soon as the preparation ends; the counts
             # come back (a pinned copy) while it runs.  A step that overflowed
@@ -225,12 +220,12 @@ class FusedRunner:
             # again with larger buffers (positions are kept; so is the next
             # prepared chunk, whose buffers are replaced) and replayed from its
             # starting species.
-            backup.copy_(self.species)
-            worst_host.copy_(eng.npairs_sets[b][:k].max(), non_blocking=True)
-            counted = ev_count
-            counted.record(main)
-            eng.play_set(b, k, self.species, rs)
-            counted.synchronize()
+            with torch.cuda.stream(play):
+                backup.copy_(self.species)
+                worst_host.copy_(eng.npairs_sets[b][:k].max(), non_blocking=True)
+                ev_count.record(play)
+                eng.play_set(b, k, self.species, rs)
+            ev_count.synchronize()
             worst = int(worst_host.item())
             while worst > eng.capacity:
                 torch.cuda.synchronize(self.device)
@@ -238,23 +233,47 @@ class FusedRunner:
                 group(c)
                 if c + 1 < len(sizes):
                     group(c + 1)
-                main.wait_event(prepared[c])
-                self.species.copy_(backup)
-                eng.play_set(b, k, self.species, rs)
-                worst = eng.worst_count(b, k)
-            ret = None
-            if on_chunk is not None:
-                ret = on_chunk(k, rx, ry, rs, eng.npairs_sets[b][:k])
-            ev = ev_play[b]  # after the callback's own work on this stream
-            ev.record(main)
-            played[b] = ev
-            released[b] = ret if isinstance(ret, torch.cuda.Event) else None
-            self.step += k
-            self.clock_steps += k
-        ev_join[1].record(side)
-        ev_join[2].record(adv)
-        main.wait_event(ev_join[1])
-        main.wait_event(ev_join[2])
+                play.wait_event(prepared[c])
+                with torch.cuda.stream(play):
+                    self.species.copy_(backup)
+                    eng.play_set(b, k, self.species, rs)
+                    worst = eng.worst_count(b, k)
+            if play is not main:
+                ev_replay.record(play)
+                main.wait_event(ev_replay)
+
+        backup, worst_host = self._backup, self._worst_host
+        try:
+            # chunk 0's preparation goes out before chunk 1's advection: it waits
+            # for nothing else
+            advect(0)
+            group(0)
+            if len(sizes) > 1:
+                advect(1)
+            for c, k in enumerate(sizes):
+                b = c % nsets
+                if c + 1 < len(sizes):
+                    group(c + 1)
+                if c + 2 < len(sizes):
+                    advect(c + 2)
+                replay(c)
+                ret = None
+                if on_chunk is not None:
+                    rx, ry, rs = recs(c)
+                    ret = on_chunk(k, rx, ry, rs, eng.npairs_sets[b][:k])
+                ev = ev_play[b]  # after the callback's own work on this stream
+                ev.record(main)
+                played[b] = ev
+                released[b] = ret if isinstance(ret, torch.cuda.Event) else None
+                self.step += k
+                self.clock_steps += k
+        finally:
+            # also after an error: what the streams still read is freed or
+            # written on the caller's only after them
+            for ev, st in zip(ev_join[1:], (side, adv, play)):
+                if st is not main:
+                    ev.record(st)
+                    main.wait_event(ev)
         return total
 
     def _ensure_pipeline(self):
@@ -262,14 +281,19 @@ class FusedRunner:
             extra = [tuple(torch.empty_like(t) for t in (self.rec_x, self.rec_y, self.rec_s))
                      for _ in range(self.PIPELINE_SETS - 1)]
             self._rec_sets = [(self.rec_x, self.rec_y, self.rec_s)] + extra
-            self._side = torch.cuda.Stream(self.device)
-            self._adv = torch.cuda.Stream(self.device)
+            # Three streams in a row: the runtime shares its (four) hardware
+            # queues out in turn, so consecutive streams are on different ones
+            # and their kernels run side by side.  With two, and the replay on
+            # the caller's stream, the three met on one queue in half of the
+            # runners: up to 127 ms for 720 steps of 490,000 microbes, 61 to 92 now (by the
+            # field, whose eddies set the longest chain of pairs).
+            self._play, self._side, self._adv = (torch.cuda.Stream(self.device) for _ in range(3))
             self._backup = torch.empty_like(self.species)  # a chunk's starting species
             self._worst_host = torch.zeros((), dtype=torch.int64, pin_memory=True)
             sets = range(self.PIPELINE_SETS)
             self._events = ([torch.cuda.Event() for _ in sets], [torch.cuda.Event() for _ in sets],
-                            [torch.cuda.Event() for _ in sets], torch.cuda.Event(),
-                            [torch.cuda.Event() for _ in range(3)])
+                            [torch.cuda.Event() for _ in sets], torch.cuda.Event(), torch.cuda.Event(),
+                            [torch.cuda.Event() for _ in range(4)])
 
     def check_domain(self):
         n_oob = int(self.oob.item())
