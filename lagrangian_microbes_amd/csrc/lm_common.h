@@ -70,8 +70,7 @@ enum KernelId {
     K_RPS_COMPS,
     K_RPS_PLAY,
     K_RPS_FILL,
-    K_RPS_DEPS,
-    K_RPS_LEVELS,
+    K_RPS_LINKS,
     K_PHILOX,
     K_COPY,
     K_SORT_HIST,

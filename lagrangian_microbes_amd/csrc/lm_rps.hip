@@ -39,22 +39,17 @@
 //                        component listed once, as small (<= 32 pairs) or wide
 //           8. fill      pair records (slot_i | bits << 29, slot_j) at their
 //                        run positions
-//           9. deps      for the wide components, per 64-pair window, the
-//                        bitmask of earlier pairs of the window sharing a slot
-//          10. levels    for wide components of up to kLevelPairs pairs: each
-//                        pair's level (longest chain of earlier pairs sharing a
-//                        particle), pairs counting-sorted by level
+//           9. links     for the wide components, per 64-pair window, the pair
+//                        before each one at each of its two particles
 //   No global atomics but the union's CAS and one add per block for the
 //   component lists.
 // Only the replay itself runs per step, in one launch of one-wavefront blocks:
-//   wide     one wavefront per larger component, species in LDS: level by
-//            level (a level's pairs share no particle, so they play at once),
-//            or for components past the level limits window by window in
-//            dependency rounds
+//   wide     one wavefront per larger component, species in LDS, a window of
+//            64 pairs at a time, each solved as a fixed point
 //   small    one lane per component of <= 32 pairs, replayed in order
 //   copy     particles without pairs keep their species
 //
-// Small populations (kSmallMax particles, no runs) take two kernels instead,
+// Small populations (workspaces of kSmallMax particles, no runs) take two kernels instead,
 // one for the whole prepare and one that replays all steps of a batch (see
 // "small populations" below).
 #include "lm_common.h"
@@ -67,8 +62,6 @@ namespace lm {
 constexpr uint32_t kUnset = 0xffffffffu;
 constexpr uint32_t kNarrowPairs = 32;
 constexpr uint32_t kNarrowSlots = kNarrowPairs + 1;  // a component of P pairs has <= P + 1 particles
-constexpr uint32_t kLevelPairs = 4096;               // components of up to this many pairs replay by levels
-constexpr uint32_t kLevelSlots = kLevelPairs + 1;    // ... and so have at most this many particles
 constexpr uint32_t kSlotMask = (1u << 29) - 1u;
 constexpr int kCompItems = 4;                        // sorted positions per thread when listing components
 
@@ -95,11 +88,9 @@ struct RpsArrays {
     int64_t* plen;                        // [step]: pairs taken (0 for an overflowed step)
     uint8_t* bits;                        // per pair (by rank)
     uint2* rec;                           // per pair (run order)
-    unsigned long long* deps;             // per pair (run order, wide components)
-    uint2* lrec;                          // per pair: wide components' records in level order,
-                                          // {slot_i, slot_j | win_table << 16}
-    uint32_t* lend;                       // per pair: end of each level, from a component's first pair
-    uint32_t* depth;                      // per wide component: levels, 0 = windowed replay
+    uint32_t* links;                      // per pair (run order, wide components): its neighbours in its
+                                          // window; small populations: its particles
+    uint32_t* list;                       // small populations, per pair: pairs by j
 };
 
 __device__ __forceinline__ uint32_t find_root(const uint32_t* parent_c, uint32_t v) {
@@ -148,7 +139,7 @@ __device__ __forceinline__ int64_t step_pairs(const int64_t* npairs, int64_t s, 
 // (bit 2)} (a like pair also lands on 2, and any outcome leaves it unchanged),
 // and i beats j iff ui - uj is 1 or -2.  Species outside {1, 2, 3} never
 // interact.
-__device__ __forceinline__ void play_pair(int& si, int& sj, uint32_t bits) {
+__host__ __device__ constexpr __forceinline__ void play_pair(int& si, int& sj, uint32_t bits) {
     const uint32_t ui = (uint32_t)(si - 1), uj = (uint32_t)(sj - 1);
     const bool valid = (ui < 3u) & (uj < 3u);
     const uint32_t k = (0x2010u >> (4u * ((ui + uj) & 7u))) & 3u;
@@ -161,22 +152,38 @@ __device__ __forceinline__ void play_pair(int& si, int& sj, uint32_t bits) {
     sj = nj;
 }
 
-// A pair's outcome as a table: bit 3 (si - 1) + (sj - 1), for si, sj in
-// {1, 2, 3}, is set when play_pair leaves both particles with si (i wins, or
-// a like pair).  Levelled records carry it (slot_j | table << 16), so that a
-// row of the replay, whose chain of dependent operations sets the time of a
-// level, decides by one table lookup.
-__device__ __forceinline__ uint32_t win_table(uint32_t bits) {
+// A pair's outcome as two tables over species indices (species - 1, or 3 for
+// any code that never interacts): two bits at 2 (4 ui + uj), i's new index in
+// x and j's in y, so that a step of a replay, a chain of dependent operations,
+// is two shifts.
+constexpr uint32_t outcome_table(uint32_t bits, int side) {
     uint32_t t = 0;
-#pragma unroll
-    for (int si = 1; si <= 3; ++si)
-#pragma unroll
-        for (int sj = 1; sj <= 3; ++sj) {
-            int a = si, b = sj;
-            play_pair(a, b, bits);
-            if (a == si && b == si) t |= 1u << (3 * (si - 1) + (sj - 1));
+    for (int ui = 0; ui < 4; ++ui)
+        for (int uj = 0; uj < 4; ++uj) {
+            int si = ui + 1, sj = uj + 1;  // 4 is outside {1, 2, 3}
+            play_pair(si, sj, bits);
+            t |= (uint32_t)((side ? sj : si) - 1) << (2 * (4 * ui + uj));
         }
     return t;
+}
+
+// Each outcome bit decides entries of its own, so the tables of any bits are
+// those of 0 with the bits' differences.
+constexpr uint32_t table_change(int k, int side) { return outcome_table(1u << k, side) ^ outcome_table(0u, side); }
+
+__device__ __forceinline__ uint2 outcome_tables(uint32_t bits) {
+    constexpr uint32_t x0 = outcome_table(0, 0), y0 = outcome_table(0, 1);
+    constexpr uint32_t xa = table_change(0, 0), xb = table_change(1, 0), xc = table_change(2, 0);
+    constexpr uint32_t ya = table_change(0, 1), yb = table_change(1, 1), yc = table_change(2, 1);
+    static_assert((x0 ^ xa ^ xb ^ xc) == outcome_table(7, 0) && (y0 ^ ya ^ yb ^ yc) == outcome_table(7, 1), "");
+    const uint32_t a = 0u - (bits & 1u), b = 0u - (bits >> 1 & 1u), c = 0u - (bits >> 2 & 1u);
+    return make_uint2(x0 ^ (xa & a) ^ (xb & b) ^ (xc & c), y0 ^ (ya & a) ^ (yb & b) ^ (yc & c));
+}
+
+// Species code -> index and back (raw: the code of an index 3).
+__device__ __forceinline__ uint32_t species_index(int code) {
+    const uint32_t u = (uint32_t)(code - 1);
+    return u < 3u ? u : 3u;
 }
 
 // Wavefront-aggregated append of v to list (one atomic per wavefront); every
@@ -717,25 +724,27 @@ rps_fill_kernel(int64_t n, const int32_t* __restrict__ pi_all, const int32_t* __
 }
 
 // 64-lane blocks, one wavefront per wide component: for each window of 64
-// pairs, the bitmask of earlier lanes that share a particle slot.  For a
-// component of up to kDepsTable particles, an LDS table of one 64-bit mask
-// per slot: every lane ORs its bit into the masks of its two slots, then
-// reads them back and keeps the earlier lanes' bits, then clears them (the
-// wavefront's LDS operations complete in program order, and every window
-// leaves the table zero).  Larger components compare each lane with the 63
-// before it by shuffles.  Split like the levels pass below: for a batch of
-// many steps, components of up to kDepsSmallPairs pairs with a table of
-// kDepsSmallTable slots (2 KB of LDS, so that many blocks stay resident),
+// pairs, every pair's links: for each of its slots, the lane and side of the
+// pair before it in the window that has the slot, and whether it is the last
+// that does.  For a component of up to TABLE particles, an LDS table of one
+// 64-bit mask per slot: every lane ORs its bit into the masks of its two
+// slots, reads them back and clears them (the wavefront's LDS operations
+// complete in program order, and every window leaves the table zero).  Larger
+// components compare each lane with the others by shuffles.  For a batch of
+// many steps, components of up to kLinksSmallPairs pairs with a table of
+// kLinksSmallTable slots (2 KB of LDS, so that many blocks stay resident),
 // then the larger ones; for a few steps, one launch takes every component.
-constexpr int32_t kSplitSteps = 24;  // batches of at least this many steps split the deps and levels passes
+// link byte of a slot: lane | side << 6 | has << 7; links: i's byte, j's << 8,
+// last at i << 16, last at j << 17.
+constexpr int32_t kSplitSteps = 24;  // batches of at least this many steps split the links pass
 enum SizeClass { kAllComponents, kSmallComponents, kLargeComponents };
-constexpr uint32_t kDepsTable = 2048;
-constexpr uint32_t kDepsSmallPairs = 256;  // the first launch's components: 2 KB of table, more blocks resident
-constexpr uint32_t kDepsSmallTable = kDepsSmallPairs + 8;
+constexpr uint32_t kLinksTable = 2048;
+constexpr uint32_t kLinksSmallPairs = 256;
+constexpr uint32_t kLinksSmallTable = kLinksSmallPairs + 8;
 
 template <uint32_t TABLE, int CLASS>
 __global__ void __launch_bounds__(64)
-rps_deps_kernel(int64_t n, RpsArrays A, RpsStrides st) {
+rps_links_kernel(int64_t n, RpsArrays A, RpsStrides st) {
     uint32_t bx, by;
     xcd_block(&bx, &by);  // an XCD works through a contiguous range of steps: one step's arrays in its L2
     __shared__ unsigned long long mask[TABLE];
@@ -744,14 +753,14 @@ rps_deps_kernel(int64_t n, RpsArrays A, RpsStrides st) {
     const uint32_t cnt = A.lists[4 * s + 1];
     if (bx >= cnt) return;  // uniform: no component for this block
     const uint2* rec = A.rec + po;
-    unsigned long long* deps = A.deps + po;
+    uint32_t* links = A.links + po;
     for (uint32_t t = lane; t < TABLE; t += 64) mask[t] = 0ull;
     __syncthreads();
     const unsigned long long bit = 1ull << lane;
     for (uint32_t c = bx; c < cnt; c += gridDim.x) {
         const uint4 dsc = A.wide[ro + c];
         const uint32_t qb = dsc.x, np = dsc.y, psz = dsc.w;
-        if ((CLASS == kSmallComponents && np > kDepsSmallPairs) || (CLASS == kLargeComponents && np <= kDepsSmallPairs))
+        if ((CLASS == kSmallComponents && np > kLinksSmallPairs) || (CLASS == kLargeComponents && np <= kLinksSmallPairs))
             continue;  // the other launch's component
         const bool table = psz <= TABLE;  // uniform over the wavefront
         if (np == 0) continue;
@@ -761,9 +770,8 @@ rps_deps_kernel(int64_t n, RpsArrays A, RpsStrides st) {
             const bool live = w + lane < np;
             const uint2 r_cur = r_next;
             r_next = rec[qb + min(w + 64u + lane, np - 1u)];
-            const uint2 r = live ? r_cur : make_uint2(kUnset, kUnset - 1u);
-            const uint32_t a = live ? (r.x & kSlotMask) : kUnset, b = live ? r.y : kUnset - 1u;
-            unsigned long long d = 0ull;
+            const uint32_t a = live ? (r_cur.x & kSlotMask) : kUnset, b = live ? r_cur.y : kUnset;
+            unsigned long long ma = 0ull, mb = 0ull;  // lanes with my slots
             if (table) {
                 // slots are < psz <= TABLE; the clamp only keeps a bad record inside the table
                 const uint32_t ta = min(a, TABLE - 1u), tb = min(b, TABLE - 1u);
@@ -772,7 +780,10 @@ rps_deps_kernel(int64_t n, RpsArrays A, RpsStrides st) {
                     atomicOr(&mask[tb], bit);
                 }
                 __builtin_amdgcn_wave_barrier();
-                if (live) d = (mask[ta] | mask[tb]) & (bit - 1ull);
+                if (live) {
+                    ma = mask[ta];
+                    mb = mask[tb];
+                }
                 __builtin_amdgcn_wave_barrier();
                 if (live) {
                     mask[ta] = 0ull;
@@ -780,142 +791,23 @@ rps_deps_kernel(int64_t n, RpsArrays A, RpsStrides st) {
                 }
                 __builtin_amdgcn_wave_barrier();
             } else {
-                for (uint32_t e = 1; e < 64; ++e) {
-                    const uint32_t src = lane >= e ? lane - e : lane;
-                    const uint32_t a2 = __shfl(a, src, 64), b2 = __shfl(b, src, 64);
-                    if (live && lane >= e && (a2 == a || a2 == b || b2 == a || b2 == b)) d |= 1ull << (lane - e);
+                for (uint32_t e = 0; e < 64; ++e) {
+                    const uint32_t a2 = __shfl(a, e, 64), b2 = __shfl(b, e, 64);
+                    if (a2 == a || b2 == a) ma |= 1ull << e;
+                    if (a2 == b || b2 == b) mb |= 1ull << e;
                 }
             }
-            if (live) deps[qb + w + lane] = d;
+            auto link = [&](unsigned long long m, uint32_t slot) {
+                const unsigned long long before = m & (bit - 1ull);
+                const uint32_t prev = before ? 63u - (uint32_t)__clzll((long long)before) : lane;
+                const uint32_t at_i = __shfl(a, prev, 64);
+                return before ? prev | (at_i == slot ? 0u : 64u) | 128u : 0u;
+            };
+            const uint32_t la = link(ma, a), lb = link(mb, b);
+            const unsigned long long above = ~(bit | (bit - 1ull));
+            if (live)
+                links[qb + w + lane] = la | lb << 8 | ((ma & above) ? 0u : 1u << 16) | ((mb & above) ? 0u : 1u << 17);
         }
-    }
-}
-
-// 64-lane blocks, one wavefront per wide component of at most kLevelPairs
-// pairs: the level of every pair in the dependency order (1 + the largest
-// level of an earlier pair sharing a particle; replayed window by window with
-// the masks of rps_deps, so it is exactly the longest-path depth), then the
-// pairs counting-sorted by level.  Pairs of one level share no particle, so a
-// replay may run each level in parallel, levels in order.
-//
-// For a batch of many steps, two launches of one kernel: components of up
-// to kLevelSmallPairs pairs with 1 KB of LDS per block, so that many blocks
-// stay resident, then the larger ones with 16 KB; for a few steps, one
-// launch takes every component (the larger components' long chains then
-// overlap the small ones instead of following them).  The per-slot last level (uint16) is dead once the
-// levels are known, so its words then hold the per-level counts and cursors
-// as packed uint16 pairs (level l in the (l & 1)-th half of word l >> 1;
-// every count and cursor is <= PAIRS, so an add never carries into the
-// other half).
-__device__ __forceinline__ uint32_t half_of(uint32_t word, uint32_t l) { return (word >> (16u * (l & 1u))) & 0xffffu; }
-
-constexpr uint32_t kLevelSmallPairs = 256;
-
-template <uint32_t PAIRS, int CLASS>
-__global__ void __launch_bounds__(64)
-rps_levels_kernel(int64_t n, RpsArrays A, RpsStrides st) {
-    uint32_t bx, by;
-    xcd_block(&bx, &by);  // an XCD works through a contiguous range of steps: one step's arrays in its L2
-    static_assert(PAIRS < 65536u && PAIRS <= kLevelPairs, "level counts must fit 16 bits");
-    __shared__ uint32_t words[(PAIRS + 2) / 2];  // last[] during the level phase, then the packed counts
-    __shared__ uint16_t lvl[PAIRS];
-    uint16_t* last = reinterpret_cast<uint16_t*>(words);
-    const int64_t s = by, ro = s * st.row, po = s * st.pair;
-    const uint32_t lane = threadIdx.x;
-    const uint32_t ncomp = A.lists[4 * s + 1];
-    const uint2* rec = A.rec + po;
-    const unsigned long long* deps = A.deps + po;
-    for (uint32_t c = bx; c < ncomp; c += gridDim.x) {
-        const uint4 dsc = A.wide[ro + c];
-        const uint32_t qb = dsc.x, np = dsc.y, psz = dsc.w;
-        if ((CLASS == kSmallComponents && np > PAIRS) || (CLASS == kLargeComponents && np <= kLevelSmallPairs))
-            continue;  // the other launch's component
-        if (np > PAIRS || psz > PAIRS + 1 || psz == 0) {
-            if (lane == 0) A.depth[ro + c] = 0;  // windowed replay
-            continue;
-        }
-        for (uint32_t t = lane; t < psz; t += 64) last[t] = 0;
-        __syncthreads();
-        uint32_t dmax = 0;
-        // the next window's records and masks load while this one resolves
-        // (np >= 1: a listed component has pairs)
-        uint2 r_next = rec[qb + min(lane, np - 1u)];
-        unsigned long long d_next = deps[qb + min(lane, np - 1u)];
-        for (uint32_t w = 0; w < np; w += 64) {
-            const bool live = w + lane < np;
-            const uint2 r_cur = r_next;
-            const unsigned long long d_cur = d_next;
-            r_next = rec[qb + min(w + 64u + lane, np - 1u)];
-            d_next = deps[qb + min(w + 64u + lane, np - 1u)];
-            const uint2 r = live ? r_cur : make_uint2(0u, 0u);
-            const unsigned long long dep = live ? d_cur : 0ull;
-            const uint32_t a = min(r.x & kSlotMask, psz - 1), b = min(r.y, psz - 1);
-            const unsigned long long all = __ballot(live);
-            unsigned long long done = 0ull;
-            bool mine = live;
-            while (done != all) {
-                const bool ready = mine && (dep & ~done) == 0ull;
-                if (ready) {
-                    const uint32_t lv = (uint32_t)max(last[a], last[b]) + 1u;
-                    last[a] = (uint16_t)lv;
-                    last[b] = (uint16_t)lv;
-                    lvl[w + lane] = (uint16_t)lv;
-                    dmax = max(dmax, lv);
-                    mine = false;
-                }
-                done |= __ballot(ready);
-                __builtin_amdgcn_wave_barrier();
-            }
-        }
-#pragma unroll
-        for (int d = 32; d >= 1; d >>= 1) dmax = max(dmax, (uint32_t)__shfl_xor(dmax, d, 64));
-        __syncthreads();
-        // last[] is dead: its words become the per-level counts (dmax <= np <= PAIRS levels)
-        for (uint32_t t = lane; t < (dmax + 1u) / 2u; t += 64) words[t] = 0u;
-        __syncthreads();
-        for (uint32_t q = lane; q < np; q += 64) {
-            const uint32_t l = lvl[q] - 1u;
-            atomicAdd(&words[l >> 1], 1u << (16u * (l & 1u)));
-        }
-        __syncthreads();
-        // exclusive offsets per level (kept as cursors in the same halves) and level ends
-        uint32_t carry = 0;
-        for (uint32_t l0 = 0; l0 < dmax; l0 += 64) {
-            const uint32_t l = l0 + lane;
-            const bool in = l < dmax;
-            const uint32_t v = in ? half_of(words[l >> 1], l) : 0u;
-            const uint32_t inc = wave_inclusive_scan(v);
-            __builtin_amdgcn_wave_barrier();  // every lane has read its half before any half is rewritten
-            if (in) {
-                last[l] = (uint16_t)(carry + inc - v);
-                A.lend[po + qb + l] = carry + inc;
-            }
-            carry += __shfl(inc, 63, 64);
-        }
-        __syncthreads();
-        // records into level order, four per lane at once (their loads in flight together)
-        for (uint32_t q0 = lane; q0 < np; q0 += 256) {
-            uint2 rv[4];
-            uint32_t pos[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) rv[u] = rec[qb + min(q0 + 64u * u, np - 1u)];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const uint32_t q = q0 + 64u * u;
-                pos[u] = kUnset;
-                if (q < np) {
-                    const uint32_t l = lvl[q] - 1u;
-                    pos[u] = half_of(atomicAdd(&words[l >> 1], 1u << (16u * (l & 1u))), l);
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                if (pos[u] < np)
-                    A.lrec[po + qb + pos[u]] =
-                        make_uint2(rv[u].x & kSlotMask, min(rv[u].y, 0xffffu) | (win_table(rv[u].x >> 29) << 16));
-        }
-        if (lane == 0) A.depth[ro + c] = dmax;
-        __syncthreads();
     }
 }
 
@@ -924,13 +816,12 @@ rps_levels_kernel(int64_t n, RpsArrays A, RpsStrides st) {
 // ---------------------------------------------------------------------------
 // One launch per step, blocks of one wavefront in three roles, ordered so
 // the longest work starts first:
-//   [0, nwide)                 one wavefront per wide component (levels, or
-//                              windows of dependency rounds past kLevelPairs)
+//   [0, nwide)                 one wavefront per wide component
 //   [nwide, nwide + nnarrow)   one lane per small component
 //   the rest                   particles without pairs keep their species
 // A wavefront's LDS operations complete in program order, so no role needs
 // a barrier between its LDS writes and later reads by other lanes.
-constexpr uint32_t kWaveSlots = (kLevelSlots + 15u) & ~15u;   // LDS species slots of a wide component
+constexpr uint32_t kWaveSlots = 4112;                         // LDS species slots of a wide component
 constexpr unsigned kPlayWideBlocks = 2048;
 constexpr unsigned kPlayNarrowBlocks = 2048;
 constexpr int kCopyItems = 8;                                 // particles per thread in the copy role
@@ -942,72 +833,6 @@ __device__ __forceinline__ void play_slots(int8_t* slots, uint2 r, uint32_t top)
     play_pair(si, sj, r.x >> 29);
     slots[a] = (int8_t)si;
     slots[b] = (int8_t)sj;
-}
-
-// play_slots on a levelled record {slot_i, slot_j | table << 16}: the same
-// result as play_pair (species outside {1, 2, 3} never interact).
-__device__ __forceinline__ void play_slots_table(int8_t* slots, uint2 r, uint32_t top) {
-    const uint32_t a = min(r.x, top), b = min(r.y & 0xffffu, top);
-    const int si = slots[a], sj = slots[b];
-    const uint32_t ui = (uint32_t)(si - 1), uj = (uint32_t)(sj - 1);
-    const bool valid = (ui < 3u) & (uj < 3u);
-    const uint32_t i_wins = (r.y >> (16u + ((3u * ui + uj) & 15u))) & 1u;  // read only when valid
-    const int w = i_wins ? si : sj;
-    slots[a] = (int8_t)(valid ? w : si);
-    slots[b] = (int8_t)(valid ? w : sj);
-}
-
-// Levelled component: species in LDS by slot; the pairs of a level share no
-// particle, so a level plays at once, in rows of at most 64 pairs (a wider
-// level is several rows, which are independent of each other).  The records
-// of kRowBatch rows go straight from memory into registers, the next batch
-// loading while the current one plays, so a row costs one LDS round trip
-// (its slots) on the critical path; the wavefront's LDS operations complete
-// in program order, so a row reads what the rows before it wrote.
-constexpr int kRowBatch = 16;
-
-struct RowCursor {
-    uint32_t l, lb, lstart, off;  // level, first level held in `ends`, level start, next row within it
-};
-
-// Row descriptors of the next kRowBatch rows (count 0 past the end) and their
-// records, one per lane.  `ends` holds the ends of levels lb .. lb + 63; it is
-// refilled, if needed, before any record load of the batch is issued (a batch
-// advances at most kRowBatch levels), and the loads are unconditional
-// (clamped), so no wait for them is placed before the batch plays.
-__device__ __forceinline__ void next_rows(RowCursor& rc, uint32_t& ends, const uint2* __restrict__ lrec,
-                                          const uint32_t* __restrict__ lend, uint32_t np, uint32_t depth,
-                                          uint32_t (&cnt)[kRowBatch], uint2 (&rr)[kRowBatch]) {
-    const uint32_t lane = threadIdx.x;
-    if (rc.l - rc.lb + kRowBatch > 64) {
-        rc.lb = rc.l;
-        ends = rc.lb + lane < depth ? lend[rc.lb + lane] : np;
-    }
-    uint32_t pos[kRowBatch];
-#pragma unroll
-    for (int q = 0; q < kRowBatch; ++q) {
-        const uint32_t at = rc.lstart + rc.off;
-        const uint32_t le = max(min((uint32_t)__builtin_amdgcn_readlane((int)ends, (int)(rc.l - rc.lb)), np), at + 1u);
-        const bool live = at < np;
-        pos[q] = live ? at : 0u;
-        cnt[q] = live ? min(64u, le - at) : 0u;
-        const bool level_done = live && at + cnt[q] >= le;
-        rc.off = level_done ? 0u : (live ? rc.off + 64u : rc.off);
-        rc.lstart = level_done ? le : rc.lstart;
-        rc.l += level_done ? 1u : 0u;
-    }
-#pragma unroll
-    for (int q = 0; q < kRowBatch; ++q) rr[q] = lrec[min(pos[q] + lane, np - 1u)];
-}
-
-__device__ __forceinline__ void play_rows(int8_t* slots, const uint32_t (&cnt)[kRowBatch],
-                                          const uint2 (&rr)[kRowBatch], uint32_t top) {
-    const uint32_t lane = threadIdx.x;
-#pragma unroll
-    for (int q = 0; q < kRowBatch; ++q) {
-        if (lane < cnt[q]) play_slots_table(slots, rr[q], top);
-        __builtin_amdgcn_wave_barrier();
-    }
 }
 
 // A wavefront stages the species of particles ids[0 .. psz) (psz >= 1) into
@@ -1052,38 +877,52 @@ __device__ __forceinline__ void stage_out(int64_t n, const uint32_t* __restrict_
     }
 }
 
-__device__ void play_levels(int64_t n, const uint32_t* __restrict__ ids, uint32_t psz,
-                            const uint2* __restrict__ lrec, const uint32_t* __restrict__ lend, uint32_t np,
-                            uint32_t depth, const int8_t* __restrict__ sp_in, int8_t* __restrict__ sp_out,
-                            int8_t* slots) {
-    const uint32_t lane = threadIdx.x;
-    const uint32_t top = psz - 1;  // 1 <= psz <= kLevelSlots
-    uint32_t ends = lane < depth ? lend[lane] : np;  // ends of levels lb .. lb + 63
-    RowCursor rc{0u, 0u, 0u, 0u};
-    uint32_t ca[kRowBatch], cb[kRowBatch];
-    uint2 ra[kRowBatch], rb[kRowBatch];
-    next_rows(rc, ends, lrec, lend, np, depth, ca, ra);
-    stage_in(n, ids, psz, sp_in, slots);
-    __builtin_amdgcn_wave_barrier();
-    while (ca[0] > 0) {
-        next_rows(rc, ends, lrec, lend, np, depth, cb, rb);
-        play_rows(slots, ca, ra, top);
-        if (cb[0] == 0) break;
-        next_rows(rc, ends, lrec, lend, np, depth, ca, ra);
-        play_rows(slots, cb, rb, top);
+// One window of up to 64 pairs of a wide component, a pair per lane, given the
+// species indices (ui, uj) its slots hold before the window: the indices after
+// it, packed i | j << 2.  A pair that follows another of the window at a slot
+// takes that one's result, which is the fixed point of playing all lanes from
+// each other's last results: from "nobody loses" as the first guess, until no
+// lane's result changes (a wavefront vote; the links point to earlier lanes, so
+// at most 64 rounds).  Results rarely change far along a chain: about five
+// rounds of ~70 ns for a window whose pairs hang together in chains of twenty.
+__device__ __forceinline__ uint32_t solve_window(uint32_t bits, uint32_t link, uint32_t ui, uint32_t uj) {
+    const uint2 tab = outcome_tables(bits);
+    const bool has_i = (link & 0x80u) != 0u, has_j = (link & 0x8000u) != 0u;
+    const int from_i = (int)((link & 63u) << 2), from_j = (int)((link >> 8 & 63u) << 2);
+    const uint32_t sh_i = link >> 5 & 2u, sh_j = link >> 13 & 2u;  // 2 * side
+    uint32_t res = ui | uj << 2;
+    for (int round = 0; round <= 64; ++round) {
+        const uint32_t at = ui << 3 | uj << 1;
+        const uint32_t now = (tab.x >> at & 3u) | (tab.y >> at & 3u) << 2;
+        const bool changed = now != res;
+        res = now;
+        if (__ballot(changed) == 0ull) break;
+        const uint32_t ri = (uint32_t)__builtin_amdgcn_ds_bpermute(from_i, (int)res);
+        const uint32_t rj = (uint32_t)__builtin_amdgcn_ds_bpermute(from_j, (int)res);
+        ui = has_i ? ri >> sh_i & 3u : ui;
+        uj = has_j ? rj >> sh_j & 3u : uj;
     }
-    __builtin_amdgcn_wave_barrier();
-    stage_out(n, ids, psz, slots, sp_out);
+    return res;
 }
 
-// Component past the level limits: windows of 64 pairs, each replayed in
-// dependency rounds (a pair fires once every earlier pair of its window that
-// shares a slot has fired); species in LDS when they fit, else in sp_out.
-__device__ void play_windows(int64_t n, const uint32_t* __restrict__ ids, uint32_t psz,
-                             const uint2* __restrict__ rec, const unsigned long long* __restrict__ deps,
-                             uint32_t np, const int8_t* __restrict__ sp_in, int8_t* __restrict__ sp_out,
-                             int8_t* slots) {
+// A wide component, window by window, by one wavefront: the records and links
+// of the next kAhead windows in flight, the species indices in LDS by slot
+// when they fit, else the species in sp_out.
+constexpr int kAhead = 4;
+
+__device__ void play_wide(int64_t n, const uint32_t* __restrict__ ids, uint32_t psz, const uint2* __restrict__ rec,
+                          const uint32_t* __restrict__ links, uint32_t np, const int8_t* __restrict__ sp_in,
+                          int8_t* __restrict__ sp_out, int8_t* slots) {
     const uint32_t lane = threadIdx.x;
+    if (np == 0) return;
+    uint2 r[kAhead];
+    uint32_t l[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+        const uint32_t k = min(64u * u + lane, np - 1u);
+        r[u] = rec[k];
+        l[u] = links[k];
+    }
     const bool in_lds = psz <= kWaveSlots;
     if (in_lds) {
         stage_in(n, ids, psz, sp_in, slots);
@@ -1094,45 +933,32 @@ __device__ void play_windows(int64_t n, const uint32_t* __restrict__ ids, uint32
         }
     }
     __syncthreads();  // (one wavefront) the copies above are visible to every lane
-    uint2 r_next = lane < np ? rec[lane] : make_uint2(0u, 0u);
-    unsigned long long d_next = lane < np ? deps[lane] : 0ull;
-    for (uint32_t w = 0; w < np; w += 64) {
-        const bool live = w + lane < np;
-        const uint2 r = r_next;
-        const unsigned long long dep = d_next;
-        if (w + 64 + lane < np) {  // next window's records, while this one replays
-            r_next = rec[w + 64 + lane];
-            d_next = deps[w + 64 + lane];
-        }
-        const uint32_t fb = r.x >> 29;
-        const uint32_t a = min(r.x & kSlotMask, psz - 1), b = min(r.y, psz - 1);  // slots are < psz
-        const unsigned long long all = __ballot(live);
-        unsigned long long done = 0ull;
-        bool mine = live;
-        while (done != all) {
-            const bool ready = mine && (dep & ~done) == 0ull;
-            if (ready) {
-                if (in_lds) {
-                    int si = slots[a], sj = slots[b];
-                    play_pair(si, sj, fb);
-                    slots[a] = (int8_t)si;
-                    slots[b] = (int8_t)sj;
-                } else {
-                    const uint32_t xa = ids[a], xb = ids[b];
-                    if (xa < (uint64_t)n && xb < (uint64_t)n) {
-                        int si = sp_out[xa], sj = sp_out[xb];
-                        play_pair(si, sj, fb);
-                        sp_out[xa] = (int8_t)si;
-                        sp_out[xb] = (int8_t)sj;
-                    }
-                }
-                mine = false;
-            }
-            done |= __ballot(ready);
-            if (in_lds)
+    for (uint32_t w0 = 0; w0 < np; w0 += 64u * kAhead) {
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const uint32_t w = w0 + 64u * u;
+            if (w >= np) break;  // uniform
+            const bool live = w + lane < np;
+            const uint32_t a = min(r[u].x & kSlotMask, psz - 1u), b = min(r[u].y, psz - 1u);  // slots are < psz
+            const uint32_t bits = r[u].x >> 29, link = live ? l[u] : 0u;
+            const uint32_t k = min(w + 64u * kAhead + lane, np - 1u);
+            r[u] = rec[k];
+            l[u] = links[k];
+            if (in_lds) {
+                const uint32_t out = solve_window(bits, link, species_index(slots[a]), species_index(slots[b]));
+                // an index 3 stands for a code that stays
+                if ((link >> 16 & 1u) && (out & 3u) != 3u) slots[a] = (int8_t)((out & 3u) + 1u);
+                if ((link >> 17 & 1u) && (out >> 2) != 3u) slots[b] = (int8_t)((out >> 2) + 1u);
                 __builtin_amdgcn_wave_barrier();
-            else
-                __syncthreads();  // this round's global stores before the next round's loads
+            } else {
+                const uint32_t xa = ids[a], xb = ids[b];
+                const bool ok = live && xa < (uint64_t)n && xb < (uint64_t)n;
+                const uint32_t ui = species_index(ok ? sp_out[xa] : 0), uj = species_index(ok ? sp_out[xb] : 0);
+                const uint32_t out = solve_window(bits, link, ui, uj);
+                if (ok && (link >> 16 & 1u) && (out & 3u) != 3u) sp_out[xa] = (int8_t)((out & 3u) + 1u);
+                if (ok && (link >> 17 & 1u) && (out >> 2) != 3u) sp_out[xb] = (int8_t)((out >> 2) + 1u);
+                __syncthreads();  // this window's global stores before the next one's loads
+            }
         }
     }
     if (in_lds) {
@@ -1202,12 +1028,8 @@ rps_play_kernel(int64_t n, int64_t s, RpsArrays A, RpsStrides st, const int8_t* 
         for (uint32_t c = bid; c < cnt; c += nwide) {
             const uint4 dsc = A.wide[ro + c];
             const uint32_t qb = dsc.x, np = dsc.y, pb = dsc.z, psz = dsc.w;
-            const uint32_t depth = A.depth[ro + c];
-            if (depth > 0 && psz >= 1 && psz <= kLevelSlots)
-                play_levels(n, A.ids + ro + pb, psz, A.lrec + po + qb, A.lend + po + qb, np, depth, sp_in, sp_out,
-                            slots);
-            else if (psz >= 1)
-                play_windows(n, A.ids + ro + pb, psz, A.rec + po + qb, A.deps + po + qb, np, sp_in, sp_out, slots);
+            if (psz >= 1)
+                play_wide(n, A.ids + ro + pb, psz, A.rec + po + qb, A.links + po + qb, np, sp_in, sp_out, slots);
             __syncthreads();  // (one wavefront) LDS free for the next component
         }
         return;
@@ -1269,7 +1091,7 @@ rps_play_kernel(int64_t n, int64_t s, RpsArrays A, RpsStrides st, const int8_t* 
 // rec: x = source at i | source at j << 16, y = next at i | next at j << 14 |
 // outcome bits << 28 | kSmallNoop; source = 2 * (pair in the window) + side,
 // or kSmallSpecies + particle; next = pair in the window or kSmallNone.
-// lend: i | j << 14 | kSmallValid.
+// links: i | j << 14 | kSmallValid.
 constexpr uint32_t kSmallValid = 0x80000000u, kSmallNoop = 0x80000000u;
 constexpr int kSmallPairs = 8;  // pairs per thread in a window
 constexpr uint32_t kSmallWindow = kSmallBlock * kSmallPairs;
@@ -1291,7 +1113,7 @@ rps_small_kernel(uint32_t n, const int32_t* __restrict__ pi_all, const int32_t* 
     if (t == 0) A.plen[s] = P;
     const int32_t* pi = pi_all + po;
     const int32_t* pj = pj_all + po;
-    uint32_t* list = reinterpret_cast<uint32_t*>(A.deps + po);  // pairs by j
+    uint32_t* list = A.list + po;
     for (uint32_t v = t; v < n; v += kSmallBlock) ends[v] = rbeg[v] = rend[v] = 0u;
     __syncthreads();
     for (uint32_t k = t; k < P; k += kSmallBlock) {
@@ -1359,23 +1181,8 @@ rps_small_kernel(uint32_t n, const int32_t* __restrict__ pi_all, const int32_t* 
             who = a | (two ? b : a) << 14 | kSmallValid;
         }
         A.rec[po + k] = r;
-        A.lend[po + k] = who;
+        A.links[po + k] = who;
     }
-}
-
-// play_pair for every pair of species indices (species - 1, or 3 for any code
-// that never interacts): two bits per pair at 2 * (4 ui + uj) for i's new
-// index (x) and j's (y).
-__device__ __forceinline__ uint2 small_table(uint32_t bits, bool two) {
-    uint2 t = make_uint2(0u, 0u);
-    for (int ui = 0; ui < 4; ++ui)
-        for (int uj = 0; uj < 4; ++uj) {
-            int si = ui + 1, sj = uj + 1;  // 4 is outside {1, 2, 3}
-            if (two) play_pair(si, sj, bits);
-            t.x |= (uint32_t)(si - 1) << (2 * (4 * ui + uj));
-            t.y |= (uint32_t)(sj - 1) << (2 * (4 * ui + uj));
-        }
-    return t;
 }
 
 // A barrier that waits for this wavefront's LDS operations only: records on
@@ -1394,24 +1201,24 @@ rps_play_small_kernel(uint32_t n, int64_t s0, int nsteps, RpsArrays A, RpsStride
     uint8_t* sp = val + kSmallSpecies;
     uint16_t* res = reinterpret_cast<uint16_t*>(val);
     const uint32_t t = threadIdx.x;
-    if (t < 9) tables[t] = small_table(t & 7u, t < 8u);
+    // (the last one changes nothing)
+    if (t < 9) tables[t] = t < 8u ? outcome_tables(t) : make_uint2(0xffaa5500u, 0xe4e4e4e4u);
     if (t < 3) queued[t] = 0u;
     for (uint32_t v = t; v < n; v += kSmallBlock) {
-        const uint32_t u = (uint32_t)(sp_in[v] - 1);
-        sp[v] = (uint8_t)(u < 3u ? u : 3u);
+        sp[v] = (uint8_t)species_index(sp_in[v]);
     }
     uint2 next_rec[kSmallPairs];
     uint32_t next_who[kSmallPairs];
     auto load = [&](int64_t s, uint32_t w, uint32_t P) {
         const uint2* rec = A.rec + s * st.pair + w;  // uniform
-        const uint32_t* lend = A.lend + s * st.pair + w;
+        const uint32_t* links = A.links + s * st.pair + w;
         const uint32_t left = P - w;
 #pragma unroll
         for (int q = 0; q < kSmallPairs; ++q) {
             const uint32_t k = q * kSmallBlock + t;
             const uint32_t kc = k < left ? k : 0u;
             next_rec[q] = rec[kc];
-            next_who[q] = k < left ? lend[kc] : 0u;
+            next_who[q] = k < left ? links[kc] : 0u;
         }
     };
     // plays pair p from the results in LDS; true if its result changed
@@ -1494,7 +1301,7 @@ rps_play_small_kernel(uint32_t n, int64_t s0, int nsteps, RpsArrays A, RpsStride
                     }
                 } else {  // more than the queue holds: every pair
                     for (uint32_t k0 = 0; k0 < most; k0 += kSmallBlock) {
-                        const bool live = k0 + t < most && (A.lend[(s0 + s) * st.pair + w + k0 + t] & kSmallValid) != 0u;
+                        const bool live = k0 + t < most && (A.links[(s0 + s) * st.pair + w + k0 + t] & kSmallValid) != 0u;
                         const uint32_t p = live ? k0 + t : 0u;
                         const uint2 r = recs[p];
                         push_after(live && play(p, r), r.y, queue[(round + 1) & 1u], &queued[then]);
@@ -1542,7 +1349,7 @@ rps_small_stats_kernel(uint32_t n, int64_t s, RpsArrays A, RpsStrides st, int64_
     }
     __syncthreads();
     for (uint32_t k = t; k < P; k += kSmallBlock) {
-        const uint32_t r = A.lend[s * st.pair + k];
+        const uint32_t r = A.links[s * st.pair + k];
         const uint32_t a = r & 0x3fffu, b = (r >> 14) & 0x3fffu;
         if (!(r & kSmallValid)) continue;
         cs[a] = cs[b] = 1u;  // has pairs
@@ -1550,7 +1357,7 @@ rps_small_stats_kernel(uint32_t n, int64_t s, RpsArrays A, RpsStrides st, int64_
     }
     __syncthreads();
     for (uint32_t k = t; k < P; k += kSmallBlock) {
-        const uint32_t r = A.lend[s * st.pair + k];
+        const uint32_t r = A.links[s * st.pair + k];
         if (r & kSmallValid) atomicAdd(&cp[lds_find(par, r & 0x3fffu)], 1u);
     }
     __syncthreads();
@@ -1659,14 +1466,12 @@ static void rps_free_pairs(lm_rps_ws* w) {
     lm::RpsArrays& A = w->A;
     (void)hipFree(A.bits);
     (void)hipFree(A.rec);
-    (void)hipFree(A.deps);
-    (void)hipFree(A.lrec);
-    (void)hipFree(A.lend);
+    (void)hipFree(A.links);
+    (void)hipFree(A.list);
     A.bits = nullptr;
     A.rec = nullptr;
-    A.deps = nullptr;
-    A.lrec = nullptr;
-    A.lend = nullptr;
+    A.links = nullptr;
+    A.list = nullptr;
     w->bytes -= w->pair_bytes;
     w->pair_bytes = 0;
     w->pair_cap = 0;
@@ -1684,7 +1489,6 @@ static void rps_ws_free(lm_rps_ws* w) {
     (void)hipFree(A.narrow);
     (void)hipFree(A.wide);
     (void)hipFree(A.plen);
-    (void)hipFree(A.depth);
     lm::sort_scratch_free(&w->sort);
     (void)hipFree(w->run_off);
     (void)hipFree(w->tile_off);
@@ -1702,8 +1506,8 @@ static int rps_ensure_pairs(lm_rps_ws* w, int64_t cap, hipStream_t s) {
     int64_t b = 0;
     int rc;
     if ((rc = rws_alloc(&A.bits, S * c, &b)) || (rc = rws_alloc(&A.rec, S * c, &b)) ||
-        (rc = rws_alloc(&A.deps, S * c, &b)) || (rc = rws_alloc(&A.lrec, S * c, &b)) ||
-        (rc = rws_alloc(&A.lend, S * c, &b))) {
+        (rc = rws_alloc(&A.links, S * c, &b)) ||
+        (rc = rws_alloc(&A.list, w->n_max <= lm::kSmallMax ? S * c : 1, &b))) {
         w->bytes += b;
         w->pair_bytes = b;
         rps_free_pairs(w);
@@ -1745,7 +1549,7 @@ int lm_rps_ws_create(int64_t n_max, int32_t steps_max, lm_rps_ws** out) {
         (rc = rws_alloc(&A.pval, R, &w->bytes)) || (rc = rws_alloc(&A.ptk, R, &w->bytes)) ||
         (rc = rws_alloc(&A.ptv, R, &w->bytes)) || (rc = rws_alloc(&A.narrow, R, &w->bytes)) ||
         (rc = rws_alloc(&A.wide, R, &w->bytes)) || (rc = rws_alloc(&A.lists, 4 * S, &w->bytes)) ||
-        (rc = rws_alloc(&A.plen, S, &w->bytes)) || (rc = rws_alloc(&A.depth, R, &w->bytes)) ||
+        (rc = rws_alloc(&A.plen, S, &w->bytes)) ||
         (rc = rws_alloc(&w->scan_tmp, S * lm::scan_num_blocks(n_max), &w->bytes)) ||
         (rc = rws_alloc(&w->tile_off, S * w->tiles1, &w->bytes)) ||
         (rc = lm::sort_scratch_alloc(&w->sort, n_max, steps_max))) {
@@ -1770,7 +1574,7 @@ int64_t lm_rps_ws_bytes(const lm_rps_ws* ws) { return ws ? ws->bytes : 0; }
 
 // The tail of a prepare, once the particles are grouped by component: row
 // offsets in grouped order, the component lists, the pair records at their
-// run positions, the wide components' dependency masks and levels.
+// run positions, the wide components' links.
 static int rps_prepare_tail(lm_rps_ws* ws, int64_t n, unsigned S, const int32_t* pair_i, const int32_t* pair_j,
                             int64_t pair_stride, hipStream_t s) {
     const lm::RpsStrides sp{ws->row, pair_stride};
@@ -1785,25 +1589,14 @@ static int rps_prepare_tail(lm_rps_ws* ws, int64_t n, unsigned S, const int32_t*
     LM_LAUNCH(lm::K_RPS_FILL, lm::rps_fill_kernel, dim3(npb, S), dim3(lm::kBlock), 0, s, n, pair_i, pair_j, A, sp);
     LM_LAUNCH_CHECK();
     if ((int32_t)S >= lm::kSplitSteps) {
-        LM_LAUNCH(lm::K_RPS_DEPS, (lm::rps_deps_kernel<lm::kDepsSmallTable, lm::kSmallComponents>), dim3(1024, S),
+        LM_LAUNCH(lm::K_RPS_LINKS, (lm::rps_links_kernel<lm::kLinksSmallTable, lm::kSmallComponents>), dim3(1024, S),
                   dim3(64), 0, s, n, A, sp);
         LM_LAUNCH_CHECK();
-        LM_LAUNCH(lm::K_RPS_DEPS, (lm::rps_deps_kernel<lm::kDepsTable, lm::kLargeComponents>), dim3(256, S),
+        LM_LAUNCH(lm::K_RPS_LINKS, (lm::rps_links_kernel<lm::kLinksTable, lm::kLargeComponents>), dim3(256, S),
                   dim3(64), 0, s, n, A, sp);
     } else {
-        LM_LAUNCH(lm::K_RPS_DEPS, (lm::rps_deps_kernel<lm::kDepsTable, lm::kAllComponents>), dim3(1024, S), dim3(64),
+        LM_LAUNCH(lm::K_RPS_LINKS, (lm::rps_links_kernel<lm::kLinksTable, lm::kAllComponents>), dim3(1024, S), dim3(64),
                   0, s, n, A, sp);
-    }
-    LM_LAUNCH_CHECK();
-    if ((int32_t)S >= lm::kSplitSteps) {
-        LM_LAUNCH(lm::K_RPS_LEVELS, (lm::rps_levels_kernel<lm::kLevelSmallPairs, lm::kSmallComponents>),
-                  dim3(1024, S), dim3(64), 0, s, n, A, sp);
-        LM_LAUNCH_CHECK();
-        LM_LAUNCH(lm::K_RPS_LEVELS, (lm::rps_levels_kernel<lm::kLevelPairs, lm::kLargeComponents>), dim3(256, S),
-                  dim3(64), 0, s, n, A, sp);
-    } else {
-        LM_LAUNCH(lm::K_RPS_LEVELS, (lm::rps_levels_kernel<lm::kLevelPairs, lm::kAllComponents>), dim3(1024, S),
-                  dim3(64), 0, s, n, A, sp);
     }
     LM_LAUNCH_CHECK();
     return LM_OK;
@@ -1836,7 +1629,7 @@ static int rps_prepare_impl(lm_rps_ws* ws, int32_t nsteps, int64_t n, const int3
     const unsigned S = (unsigned)nsteps;
     // one workgroup holds a small step; without pairs the general replay's
     // copy is all there is to do, and an ensemble's runs have keys of their own
-    ws->small = n <= lm::kSmallMax && run == nullptr && pair_stride > 0;
+    ws->small = ws->n_max <= lm::kSmallMax && run == nullptr && pair_stride > 0;
     if (ws->small) {
         LM_LAUNCH(lm::K_RPS_SMALL, lm::rps_small_kernel, dim3(S), dim3(lm::kSmallBlock), 0, s, (uint32_t)n, pair_i,
                   pair_j, npairs, A, sp, pRS, pPR, pSP, key0, key1, step0);

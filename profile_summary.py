@@ -52,8 +52,8 @@ TIMER_NAMES = {
     "scan_reduce_kernel": "scan_reduce", "scan_apply_kernel": "scan_apply", "rps_init_kernel": "rps_init",
     "rps_tile_union_kernel": "rps_tile",
     "rps_union_kernel": "rps_union", "rps_keys_kernel": "rps_keys", "rps_group_blk_kernel": "rps_group",
-    "rps_comps_kernel": "rps_comps", "rps_fill_kernel": "rps_fill", "rps_deps_kernel": "rps_deps",
-    "rps_levels_kernel": "rps_levels", "rps_play_kernel": "rps_play", "copy16_kernel": "copy16",
+    "rps_comps_kernel": "rps_comps", "rps_fill_kernel": "rps_fill", "rps_links_kernel": "rps_links",
+    "rps_play_kernel": "rps_play", "copy16_kernel": "copy16",
     "philox_kernel": "philox", "seg_copy_kernel": "copy16",
     "advect_rk4_f32_kernel": "advect_rk4_f32", "field_blend_f32_kernel": "field_blend_f32",
     "adj_forward_kernel": "adj_forward", "adj_recompute_kernel": "adj_recompute",
