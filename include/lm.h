@@ -356,6 +356,19 @@ int lm_adjoint_backward(int64_t n, const double* checkpoints, const float* field
                         int32_t ckpt, void* scratch, int64_t scratch_bytes, double* glon, double* glat, float* gfield,
                         void* stream);
 
+/* *loss (device double) = the mean squared great-circle distance of the n >= 1
+ * positions to their targets (degrees; haversine on a sphere of the given
+ * radius; the loss in the units of radius^2), summed in a fixed order, and with
+ * ngrad = 2 (4) its gradients to lon, lat (and lon_t, lat_t) as consecutive
+ * rows of grad ([ngrad][n] doubles).  partial: LM_LOSS_PARTIALS doubles of
+ * scratch.  No reference counterpart (the reference fits nothing). */
+#define LM_LOSS_PARTIALS 2048
+int lm_trajectory_loss(int64_t n, const double* lon, const double* lat, const double* lon_t, const double* lat_t,
+                       double radius, int32_t ngrad, double* grad, double* partial, double* loss, void* stream);
+/* out[k] = grad[k] * *by, k < count (*by a device double): the loss's
+ * gradients times the gradient that reaches it. */
+int lm_scale_by(int64_t count, const double* grad, const double* by, double* out, void* stream);
+
 /* ------------------------------------------------------------------------ */
 /* Plain streaming copy, used to calibrate hardware byte counters.          */
 /* No reference counterpart.                                                */

@@ -69,6 +69,8 @@ _SIGNATURES = {
     "lm_adjoint_scratch_bytes": (c_i64, [c_i64, c_i32, ctypes.POINTER(LmGrid), c_i32]),
     "lm_adjoint_backward": (ctypes.c_int, [c_i64, c_vp, c_vp, c_i32, ctypes.POINTER(LmGrid), c_vp, c_vp, c_vp,
                                            c_i32, c_dbl, c_i32, c_vp, c_i64, c_vp, c_vp, c_vp, c_vp]),
+    "lm_trajectory_loss": (ctypes.c_int, [c_i64, c_vp, c_vp, c_vp, c_vp, c_dbl, c_i32, c_vp, c_vp, c_vp, c_vp]),
+    "lm_scale_by": (ctypes.c_int, [c_i64, c_vp, c_vp, c_vp, c_vp]),
     "lm_copy_bytes": (ctypes.c_int, [c_vp, c_vp, c_i64, c_vp]),
     "lm_sort_pairs_u32": (ctypes.c_int, [c_i32, c_vp, c_i64, c_i64, c_i64, c_i32, c_vp, c_vp, c_vp, c_vp, c_vp]),
     "lm_timing_enable": (ctypes.c_int, [ctypes.c_int]),
@@ -77,6 +79,8 @@ _SIGNATURES = {
 }
 
 EXPORTED = tuple(_SIGNATURES)
+
+LOSS_PARTIALS = 2048  # LM_LOSS_PARTIALS
 
 _lib = None
 

@@ -163,9 +163,75 @@ def great_circle_sq(lon, lat, lon_t, lat_t, radius=SPHERE_RADIUS_M):
     return (radius * ang) ** 2
 
 
+def _mean_great_circle_sq(lon, lat, lon_t, lat_t):
+    return great_circle_sq(lon, lat, lon_t, lat_t, radius=SPHERE_RADIUS_M / 1e3).mean()
+
+
+class TrajectoryLoss(torch.autograd.Function):
+    """trajectory_loss of contiguous float64 GPU tensors of one shape, with its
+    gradients from the same pass (lm_trajectory_loss)."""
+
+    @staticmethod
+    def forward(ctx, lon, lat, lon_t, lat_t):
+        need = ctx.needs_input_grad
+        ngrad = 4 if need[2] or need[3] else 2 if need[0] or need[1] else 0
+        n = lon.numel()
+        # one block: the loss, the scratch sums and the gradients
+        buf = torch.empty(1 + _lib.LOSS_PARTIALS + ngrad * n, dtype=torch.float64, device=lon.device)
+        grad = buf[1 + _lib.LOSS_PARTIALS:]
+        loss = torch.empty((), dtype=torch.float64, device=lon.device)
+        check(_lib.load().lm_trajectory_loss(n, ptr(lon), ptr(lat), ptr(lon_t), ptr(lat_t), SPHERE_RADIUS_M / 1e3, ngrad,
+                                             ptr(grad), ptr(buf[1:]), ptr(loss), stream_ptr()))
+        ctx.save_for_backward(grad)
+        # the inputs serve a second differentiation only: they may be changed
+        # in place before the backward, as under the single operations
+        ctx.inputs = (lon, lat, lon_t, lat_t)
+        ctx.versions = tuple(t._version for t in ctx.inputs)
+        return loss
+
+    @staticmethod
+    def backward(ctx, by):
+        grad, = ctx.saved_tensors
+        inputs, need = ctx.inputs, ctx.needs_input_grad
+        if torch.is_grad_enabled():  # a gradient that is to be differentiated again
+            if any(t._version != v for t, v in zip(inputs, ctx.versions)):
+                raise RuntimeError("a position or target of trajectory_loss was modified by an inplace operation "
+                                   "before its gradient was differentiated")
+            loss = _mean_great_circle_sq(*inputs)
+            wanted = [t for t, w in zip(inputs, need) if w]
+            got = iter(torch.autograd.grad(loss, wanted, by, create_graph=True))
+            return tuple(next(got) if w else None for w in need)
+        n = inputs[0].numel()
+        out = torch.empty_like(grad)
+        by = by.to(torch.float64).contiguous()
+        check(_lib.load().lm_scale_by(out.numel(), ptr(grad), ptr(by), ptr(out), stream_ptr()))
+        return tuple(out[k * n:(k + 1) * n].view(inputs[0].shape) if w else None for k, w in enumerate(need))
+
+
+def _plain_f64(tensors):
+    """Plain contiguous float64 tensors of one shape on the current GPU, with no
+    tracing, transform, mode or forward-mode tangent that would have to see the
+    single operations."""
+    t0 = tensors[0]
+    if not all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float64 and t.device == t0.device
+               and t.shape == t0.shape and t.is_contiguous() for t in tensors):
+        return False
+    if t0.device.type != "cuda" or t0.device.index != torch.cuda.current_device() or t0.numel() == 0:
+        return False
+    if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._functorch.peek_interpreter_stack() is not None:
+        return False
+    if torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack():
+        return False
+    return not any(torch.autograd.forward_ad.unpack_dual(t).tangent is not None for t in tensors) \
+        if torch.autograd.forward_ad._current_level >= 0 else True
+
+
 def trajectory_loss(lon, lat, lon_t, lat_t):
     """Mean squared great-circle distance to the targets, in km^2."""
-    return great_circle_sq(lon, lat, lon_t, lat_t, radius=SPHERE_RADIUS_M / 1e3).mean()
+    args = (lon, lat, lon_t, lat_t)
+    if all(isinstance(t, torch.Tensor) for t in args) and _plain_f64(args):
+        return TrajectoryLoss.apply(*args)
+    return _mean_great_circle_sq(*args)
 
 
 def interact_final(lon, lat, species, radius, params, key, step, bbox, norm=2.0):

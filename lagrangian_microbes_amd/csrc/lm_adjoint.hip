@@ -689,6 +689,71 @@ adj_slab_kernel(const float* __restrict__ slab, int nlev, lm_grid g, float* __re
     if (acc != 0.0f) gfield[t] += acc;
 }
 
+// ----------------------------------------------------------------------------
+// Trajectory loss: the mean squared great-circle distance of n positions to
+// their targets, and its gradients.  Per particle, with p = lat pi / 180:
+//   a = sin^2((p_t - p) / 2) + cos p cos p_t sin^2((lon_t - lon) pi / 360),
+//   d = radius 2 asin(sqrt(clamp(a, 1e-300, 1))),   loss = mean d^2,
+// dd^2/da = 2 radius^2 ang / (sqrt(a) sqrt(1 - a)), zero where the clamp holds a.
+// One pass computes both (the gradients are unscaled by the loss's own: a
+// second kernel multiplies): as separate operations the loss and its gradient
+// were 60 launches, 0.5 ms of a 0.75 ms fitting step of 10,000 particles.
+// ----------------------------------------------------------------------------
+__global__ void __launch_bounds__(kAdjBlock)
+traj_loss_kernel(int64_t n, const double* __restrict__ lon, const double* __restrict__ lat,
+                 const double* __restrict__ lon_t, const double* __restrict__ lat_t, double radius,
+                 double* __restrict__ grad, int ngrad, double* __restrict__ partial) {
+    __shared__ double lds[kAdjBlock / 64];
+    double sum = 0.0;
+    for (int64_t i = (int64_t)blockIdx.x * kAdjBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kAdjBlock) {
+        const double p1 = lat[i] * LM_DEG2RAD, p2 = lat_t[i] * LM_DEG2RAD;
+        double s1, c1, s2, c2, sp1, cp1, sp2, cp2;
+        sincos(0.5 * (p2 - p1), &s1, &c1);
+        sincos(0.5 * (lon_t[i] - lon[i]) * LM_DEG2RAD, &s2, &c2);
+        sincos(p1, &sp1, &cp1);
+        sincos(p2, &sp2, &cp2);
+        const double a = s1 * s1 + cp1 * cp2 * (s2 * s2);
+        const double ac = a < 1e-300 ? 1e-300 : a > 1.0 ? 1.0 : a;  // (a NaN stays)
+        const double r = sqrt(ac), ang = 2.0 * asin(r);
+        sum += (radius * ang) * (radius * ang);
+        if (ngrad > 0) {
+            const double g = a < 1e-300 || a > 1.0 ? 0.0 : 2.0 * radius * radius * ang / (r * sqrt(1.0 - ac)) / (double)n;
+            const double glon = -(g * LM_DEG2RAD) * (cp1 * cp2 * (s2 * c2));
+            grad[i] = glon;
+            grad[n + i] = -(g * LM_DEG2RAD) * (s1 * c1 + sp1 * cp2 * (s2 * s2));
+            if (ngrad > 2) {
+                grad[2 * n + i] = -glon;
+                grad[3 * n + i] = (g * LM_DEG2RAD) * (s1 * c1 - cp1 * sp2 * (s2 * s2));
+            }
+        }
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) partial[blockIdx.x] = (lds[0] + lds[1]) + (lds[2] + lds[3]);
+}
+
+// loss = sum of the workgroups' sums / n, in a fixed order.
+__global__ void __launch_bounds__(kAdjBlock)
+traj_loss_sum_kernel(int64_t n, const double* __restrict__ partial, int count, double* __restrict__ loss) {
+    __shared__ double lds[kAdjBlock / 64];
+    double sum = 0.0;
+    for (int k = threadIdx.x; k < count; k += kAdjBlock) sum += partial[k];
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = sum;
+    __syncthreads();
+    if (threadIdx.x == 0) *loss = ((lds[0] + lds[1]) + (lds[2] + lds[3])) / (double)n;
+}
+
+__global__ void __launch_bounds__(kAdjBlock)
+traj_scale_kernel(int64_t count, const double* __restrict__ grad, const double* __restrict__ by,
+                  double* __restrict__ out) {
+    const int64_t i = (int64_t)blockIdx.x * kAdjBlock + threadIdx.x;
+    if (i < count) out[i] = grad[i] * *by;
+}
+
 }  // namespace lm
 
 namespace {
@@ -900,6 +965,33 @@ int lm_adjoint_backward(int64_t n, const double* checkpoints, const float* field
     }
     LM_LAUNCH(lm::K_ADJ_SLAB, lm::adj_slab_kernel, dim3(lm::grid_for((int64_t)nlev * level_len_of(grid) * 2, lm::kAdjBlock)),
               dim3(lm::kAdjBlock), 0, s, slab, (int)nlev, *grid, gfield);
+    LM_LAUNCH_CHECK();
+    return LM_OK;
+}
+
+int lm_trajectory_loss(int64_t n, const double* lon, const double* lat, const double* lon_t, const double* lat_t,
+                       double radius, int32_t ngrad, double* grad, double* partial, double* loss, void* stream) {
+    LM_REQUIRE(n >= 1, LM_ERR_ARG, "the loss needs at least one particle");
+    LM_REQUIRE(ngrad == 0 || ngrad == 2 || ngrad == 4, LM_ERR_ARG, "0, 2 or 4 gradients");
+    LM_REQUIRE(lon && lat && lon_t && lat_t && partial && loss && (ngrad == 0 || grad), LM_ERR_ARG, "NULL pointer");
+    int64_t blocks = (n + lm::kAdjBlock - 1) / lm::kAdjBlock;
+    blocks = blocks < LM_LOSS_PARTIALS ? blocks : LM_LOSS_PARTIALS;
+    hipStream_t s = (hipStream_t)stream;
+    LM_LAUNCH(lm::K_TRAJ_LOSS, lm::traj_loss_kernel, dim3((unsigned)blocks), dim3(lm::kAdjBlock), 0, s, n, lon, lat,
+              lon_t, lat_t, radius, grad, (int)ngrad, partial);
+    LM_LAUNCH_CHECK();
+    LM_LAUNCH(lm::K_TRAJ_LOSS, lm::traj_loss_sum_kernel, dim3(1), dim3(lm::kAdjBlock), 0, s, n,
+              (const double*)partial, (int)blocks, loss);
+    LM_LAUNCH_CHECK();
+    return LM_OK;
+}
+
+int lm_scale_by(int64_t count, const double* grad, const double* by, double* out, void* stream) {
+    LM_REQUIRE(count >= 0, LM_ERR_ARG, "negative size");
+    if (count == 0) return LM_OK;
+    LM_REQUIRE(grad && by && out, LM_ERR_ARG, "NULL pointer");
+    LM_LAUNCH(lm::K_TRAJ_LOSS, lm::traj_scale_kernel, dim3(lm::grid_for(count, lm::kAdjBlock)), dim3(lm::kAdjBlock), 0,
+              (hipStream_t)stream, count, grad, by, out);
     LM_LAUNCH_CHECK();
     return LM_OK;
 }

@@ -89,6 +89,7 @@ enum KernelId {
     K_EMIT_SMALL,
     K_RPS_SMALL,
     K_PLAY_SMALL,
+    K_TRAJ_LOSS,
     K_NUM_KERNELS
 };
 bool timing_on();

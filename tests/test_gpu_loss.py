@@ -1,0 +1,70 @@
+"""The one-pass trajectory loss against the single torch operations it stands for."""
+import pytest
+import torch
+
+from lagrangian_microbes_amd import adjoint
+
+pytestmark = pytest.mark.gpu
+
+
+def inputs(n, seed, need):
+    g = torch.Generator().manual_seed(seed)
+    lon, lat = 360.0 * torch.rand(n, generator=g), 178.0 * torch.rand(n, generator=g) - 89.0
+    d = torch.randn(2, n, generator=g) * 10.0 ** torch.randint(-7, 1, (n,), generator=g)
+    t = [lon, lat, lon + d[0], (lat + d[1]).clamp(-89.5, 89.5)]
+    t = [v.double() for v in t]
+    t[2][:1], t[3][:1] = t[0][:1], t[1][:1]  # a particle on its target
+    return [v.cuda().requires_grad_(bool(w)) for v, w in zip(t, need)]
+
+
+@pytest.mark.parametrize("n", [1, 2, 255, 257, 4097, 600_001])
+@pytest.mark.parametrize("need", [(1, 1, 0, 0), (1, 0, 0, 1), (0, 0, 1, 1)])
+def test_loss_and_gradients(gpu, n, need):
+    args = inputs(n, n, need)
+    wanted = [t for t in args if t.requires_grad]
+    loss, ref = adjoint.trajectory_loss(*args), adjoint._mean_great_circle_sq(*args)
+    assert type(loss.grad_fn).__name__ == "TrajectoryLossBackward" and loss.shape == ref.shape
+    # a handful of roundings per term, and the order of the sum
+    torch.testing.assert_close(loss, ref, rtol=1e-13, atol=0.0)
+    by = torch.tensor(0.7, dtype=torch.float64, device="cuda")
+    for a, b in zip(torch.autograd.grad(loss, wanted, by), torch.autograd.grad(ref, wanted, by)):
+        # the angle's sine and a = sin^2 ... round alike; 1 / sqrt(a) and the quotients once more each
+        torch.testing.assert_close(a, b, rtol=1e-12, atol=1e-16 * float(b.abs().max()))
+
+
+def test_second_derivatives(gpu):
+    args = inputs(50, 3, (1, 1, 1, 1))
+    for f in (adjoint.trajectory_loss, adjoint._mean_great_circle_sq):
+        g = torch.autograd.grad(f(*args), args, create_graph=True)
+        got = torch.autograd.grad(sum((v[1:] ** 2).sum() for v in g), args)
+        if f is adjoint.trajectory_loss:
+            first = got
+    for a, b in zip(first, got):
+        torch.testing.assert_close(a, b, rtol=1e-12, atol=0.0, equal_nan=True)
+
+
+def test_other_calls_take_the_single_operations(gpu):
+    lon, lat, lon_t, lat_t = (t.detach() for t in inputs(40, 5, (0, 0, 0, 0)))
+    ref = adjoint._mean_great_circle_sq(lon, lat, lon_t, lat_t)
+    # broadcast targets, float32, strided, on the CPU
+    assert torch.isfinite(adjoint.trajectory_loss(lon, lat, lon_t[:1], lat_t[:1]))
+    assert adjoint.trajectory_loss(*(t.float() for t in (lon, lat, lon_t, lat_t))).dtype == torch.float32
+    both = torch.stack((lon, lat), 1)
+    torch.testing.assert_close(adjoint.trajectory_loss(both[:, 0], both[:, 1], lon_t, lat_t), ref)
+    torch.testing.assert_close(adjoint.trajectory_loss(*(t.cpu() for t in (lon, lat, lon_t, lat_t))).cuda(), ref)
+    # a transform, forward-mode, an input changed in place before the backward
+    each = torch.func.vmap(lambda a, b: adjoint.trajectory_loss(a, b, lon_t, lat_t))(lon[None], lat[None])
+    torch.testing.assert_close(each[0], ref)
+    _, tangent = torch.func.jvp(lambda a: adjoint.trajectory_loss(a, lat, lon_t, lat_t), (lon,), (torch.ones_like(lon),))
+    x = lon.clone().requires_grad_()
+    g, = torch.autograd.grad(adjoint.trajectory_loss(x, lat, lon_t, lat_t), x)
+    torch.testing.assert_close(tangent, g.sum())
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(lon, torch.ones_like(lon))
+        out = torch.autograd.forward_ad.unpack_dual(adjoint.trajectory_loss(dual, lat, lon_t, lat_t))
+        torch.testing.assert_close(out.tangent, tangent)
+    y = x * 1.0
+    loss = adjoint.trajectory_loss(y, lat, lon_t, lat_t)
+    with torch.no_grad():
+        y.add_(1.0)
+    torch.testing.assert_close(torch.autograd.grad(loss, x)[0], g)
