@@ -7,64 +7,61 @@
 // blended node-wise beforehand (lm_field_blend_f64), so a stage reads four
 // interleaved (u,v) nodes = 2 x 32 contiguous bytes, which stay in L2/MALL:
 // a 0.25 degree field over 20 x 20 degrees is 0.1 MB per stage time.
-//
-// Operation order (mirrored operation by operation in oracle/lm_oracle.c):
-//   fx  = (x - x0) * inv_dx,          i = trunc(fx) clamped to nx-2, xi  = fx - i
-//   fy  = (y - y0) * inv_dy,          j = trunc(fy) clamped to ny-2, eta = fy - j
-//   u_b = fma(xi, u10 - u00, u00),   u_t = fma(xi, u11 - u01, u01)
-//   u   = fma(eta, u_t - u_b, u_b)   (same for v)
-//   u_deg = (u * (1/111120)) / cos_deg(y),   v_deg = v * (1/111120)
-//   x1 = fma(u1, dt/2, x) ... x3 = fma(u3, dt, x)
-//   x += fma(2, u2 + u3, u1 + u4) * (dt/6) as fma(., dt/6, x)
+// The sample and its operation order are in lm_rk4.h.
 #include "lm_common.h"
+#include "lm_rk4.h"
 
 namespace lm {
 
-__device__ __forceinline__ bool sample_uv(const double* __restrict__ f, const lm_grid& g, double x,
-                                          double y, double* ud, double* vd) {
-    const double fx = (x - g.x0) * g.inv_dx;
-    const double fy = (y - g.y0) * g.inv_dy;
-    if (!(fx >= 0.0 && fx <= (double)(g.nx - 1) && fy >= 0.0 && fy <= (double)(g.ny - 1)))
-        return false;  // outside the grid (or NaN)
-    int i = (int)fx;
-    int j = (int)fy;
-    i = i > g.nx - 2 ? g.nx - 2 : i;
-    j = j > g.ny - 2 ? g.ny - 2 : j;
-    const double xi = fx - (double)i;
-    const double eta = fy - (double)j;
-    // node index in 32 bits (the entry points require nx * ny < 2^31): one
-    // integer multiply-add instead of a 64-bit product per sample
-    const double2* r0 = reinterpret_cast<const double2*>(f) + ((uint32_t)j * (uint32_t)g.nx + (uint32_t)i);
-    const double2* r1 = r0 + g.nx;
-    const double2 a = r0[0], b = r0[1], c = r1[0], d = r1[1];
-    const double ub = fma(xi, b.x - a.x, a.x);
-    const double ut = fma(xi, d.x - c.x, c.x);
-    const double u = fma(eta, ut - ub, ub);
-    const double vb = fma(xi, b.y - a.y, a.y);
-    const double vt = fma(xi, d.y - c.y, c.y);
-    const double v = fma(eta, vt - vb, vb);
-    *ud = (u * LM_INV_M_PER_DEG) / cos_deg(y);
-    *vd = v * LM_INV_M_PER_DEG;
-    return true;
+LM_DEFINE_COS_COEFS(advect_cos)
+
+// A step's random-walk increments of particle i: philox4x64_10 at (i, step, 1,
+// 0).  The first rounds' products that do not see the step leave the loop; the
+// later rounds' keys are made opaque in it, because all twenty of them kept in
+// scalar registers spill the rest.
+__device__ __forceinline__ void walk_step(uint64_t i, uint64_t step, uint64_t k0, uint64_t k1, double amp, double* x,
+                                          double* y) {
+    constexpr uint64_t M0 = 0xD2E7470EE14C6C93ull, M1 = 0xCA5A826395121157ull;
+    constexpr uint64_t W0 = 0x9E3779B97F4A7C15ull, W1 = 0xBB67AE8584CAA73Bull;
+    uint64_t c0 = i, c1 = step, c2 = kStreamWalk, c3 = 0;
+#pragma unroll
+    for (int r = 0; r < 10; ++r) {
+        if (r == 3) asm volatile("" : "+s"(k0), "+s"(k1));
+        uint64_t hi0, lo0, hi1, lo1;
+        mulhilo64(M0, c0, &hi0, &lo0);
+        mulhilo64(M1, c2, &hi1, &lo1);
+        c0 = hi1 ^ c1 ^ k0;
+        c2 = hi0 ^ c3 ^ k1;
+        c1 = lo1;
+        c3 = lo0;
+        k0 += W0;
+        k1 += W1;
+    }
+    *y = fma(fma(2.0, u01_from_u64(c0), -1.0), amp, *y);
+    *x = fma(fma(2.0, u01_from_u64(c1), -1.0), amp, *x);
 }
 
 // One RK4 step; returns false (position untouched) if any stage leaves the grid.
+template <bool BIG>
 __device__ __forceinline__ bool rk4_step(const double* __restrict__ f0, const double* __restrict__ fh,
-                                         const double* __restrict__ f1, const lm_grid& g,
+                                         const double* __restrict__ f1, const lm_grid& g, const CosCoefs& K,
                                          double hh, double h, double h6, double* x, double* y) {
     double u1, v1, u2, v2, u3, v3, u4, v4;
     const double x0 = *x, y0 = *y;
-    if (!sample_uv(f0, g, x0, y0, &u1, &v1)) return false;
-    if (!sample_uv(fh, g, fma(u1, hh, x0), fma(v1, hh, y0), &u2, &v2)) return false;
-    if (!sample_uv(fh, g, fma(u2, hh, x0), fma(v2, hh, y0), &u3, &v3)) return false;
-    if (!sample_uv(f1, g, fma(u3, h, x0), fma(v3, h, y0), &u4, &v4)) return false;
+    uint32_t ci, cj;
+    lanes_t in = sample_uv<BIG>(f0, g, K, x0, y0, &u1, &v1, &ci, &cj);
+    in &= sample_uv<BIG>(fh, g, K, fma(u1, hh, x0), fma(v1, hh, y0), &u2, &v2, &ci, &cj);
+    in &= sample_uv<BIG>(fh, g, K, fma(u2, hh, x0), fma(v2, hh, y0), &u3, &v3, &ci, &cj);
+    in &= sample_uv<BIG>(f1, g, K, fma(u3, h, x0), fma(v3, h, y0), &u4, &v4, &ci, &cj);
+    const bool inside = __builtin_amdgcn_inverse_ballot_w64(in);
     const double su = fma(2.0, u2 + u3, u1 + u4);
     const double sv = fma(2.0, v2 + v3, v1 + v4);
-    *x = fma(su, h6, x0);
-    *y = fma(sv, h6, y0);
-    return true;
+    *x = inside ? fma(su, h6, x0) : x0;
+    *y = inside ? fma(sv, h6, y0) : y0;
+    return inside;
 }
 
+template <bool WALK, bool BIG>
 __global__ void __launch_bounds__(kBlock)
 advect_rk4_f64_kernel(int64_t n, double* __restrict__ lon, double* __restrict__ lat,
                       const double* __restrict__ fields, int64_t stage_stride, lm_grid g,
@@ -75,19 +72,16 @@ advect_rk4_f64_kernel(int64_t n, double* __restrict__ lon, double* __restrict__ 
     const int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
     double x = lon[i], y = lat[i];
+    const CosCoefs K = load_advect_cos();
     for (int s = 0; s < nsteps; ++s) {
         const double* f0 = fields + (int64_t)(2 * s) * stage_stride;
-        if (!rk4_step(f0, f0 + stage_stride, f0 + 2 * stage_stride, g, hh, h, h6, &x, &y))
+        if (!rk4_step<BIG>(f0, f0 + stage_stride, f0 + 2 * stage_stride, g, K, hh, h, h6, &x, &y))
             atomicAdd(oob_count, 1u);
         if (rec_lon) {
             rec_lon[(int64_t)s * rec_stride + i] = (float)x;
             rec_lat[(int64_t)s * rec_stride + i] = (float)y;
         }
-        if (walk_amp > 0.0) {
-            const philox4x64 r = philox4x64_10((uint64_t)i, step0 + (uint64_t)s, kStreamWalk, 0, k0, k1);
-            y = fma(fma(2.0, u01_from_u64(r.v[0]), -1.0), walk_amp, y);
-            x = fma(fma(2.0, u01_from_u64(r.v[1]), -1.0), walk_amp, x);
-        }
+        if constexpr (WALK) walk_step((uint64_t)i, step0 + (uint64_t)s, k0, k1, walk_amp, &x, &y);
     }
     lon[i] = x;
     lat[i] = y;
@@ -132,20 +126,28 @@ __device__ __forceinline__ float cos_deg_f32(float lat_deg) {
     return fmaf(p, z, 1.0f);
 }
 
-__device__ __forceinline__ bool sample_uv_f32(const float* __restrict__ f, const lm_grid& g, double x, double y,
+// divide_near_one in float32.
+__device__ __forceinline__ float divide_near_one_f32(float n, float d) {
+    float r = __builtin_amdgcn_rcpf(d);
+    r = fmaf(fmaf(-d, r, 1.0f), r, r);
+    float q = n * r;
+    q = fmaf(fmaf(-d, q, n), r, q);
+    return __builtin_amdgcn_div_fixupf(fmaf(fmaf(-d, q, n), r, q), d, n);
+}
+
+// sample_uv in float32.
+template <bool BIG>
+__device__ __forceinline__ lanes_t sample_uv_f32(const float* __restrict__ f, const lm_grid& g, double x, double y,
                                               float* ud, float* vd) {
-    const double fx = (x - g.x0) * g.inv_dx;
-    const double fy = (y - g.y0) * g.inv_dy;
-    if (!(fx >= 0.0 && fx <= (double)(g.nx - 1) && fy >= 0.0 && fy <= (double)(g.ny - 1)))
-        return false;  // outside the grid (or NaN)
-    int i = (int)fx;
-    int j = (int)fy;
-    i = i > g.nx - 2 ? g.nx - 2 : i;
-    j = j > g.ny - 2 ? g.ny - 2 : j;
-    const float xi = (float)(fx - (double)i);
-    const float eta = (float)(fy - (double)j);
-    const float2* r0 = reinterpret_cast<const float2*>(f) + ((uint32_t)j * (uint32_t)g.nx + (uint32_t)i);
-    const float2* r1 = r0 + g.nx;
+    uint32_t i, j;
+    double fx, fy;
+    const lanes_t in_x = locate_axis(x, g.x0, g.inv_dx, g.nx, &i, &fx);
+    const lanes_t in_y = locate_axis(y, g.y0, g.inv_dy, g.ny, &j, &fy);
+    const float xi = (float)fx, eta = (float)fy;
+    const auto off = node_offset<8, BIG>(g, i, j);
+    const char* row = reinterpret_cast<const char*>(f);
+    const float2* r0 = reinterpret_cast<const float2*>(row + off);
+    const float2* r1 = reinterpret_cast<const float2*>(row + 8 * (int64_t)g.nx + off);
     const float2 a = r0[0], b = r0[1], c = r1[0], d = r1[1];
     const float ub = fmaf(xi, b.x - a.x, a.x);
     const float ut = fmaf(xi, d.x - c.x, c.x);
@@ -153,27 +155,30 @@ __device__ __forceinline__ bool sample_uv_f32(const float* __restrict__ f, const
     const float vb = fmaf(xi, b.y - a.y, a.y);
     const float vt = fmaf(xi, d.y - c.y, c.y);
     const float v = fmaf(eta, vt - vb, vb);
-    *ud = (u * LM_INV_M_PER_DEG_F) / cos_deg_f32((float)y);
+    *ud = divide_near_one_f32(u * LM_INV_M_PER_DEG_F, cos_deg_f32((float)y));
     *vd = v * LM_INV_M_PER_DEG_F;
-    return true;
+    return in_x & in_y;
 }
 
+template <bool BIG>
 __device__ __forceinline__ bool rk4_step_f32(const float* __restrict__ f0, const float* __restrict__ fh,
                                              const float* __restrict__ f1, const lm_grid& g, double hh, double h,
                                              double h6, double* x, double* y) {
     float u1, v1, u2, v2, u3, v3, u4, v4;
     const double x0 = *x, y0 = *y;
-    if (!sample_uv_f32(f0, g, x0, y0, &u1, &v1)) return false;
-    if (!sample_uv_f32(fh, g, fma((double)u1, hh, x0), fma((double)v1, hh, y0), &u2, &v2)) return false;
-    if (!sample_uv_f32(fh, g, fma((double)u2, hh, x0), fma((double)v2, hh, y0), &u3, &v3)) return false;
-    if (!sample_uv_f32(f1, g, fma((double)u3, h, x0), fma((double)v3, h, y0), &u4, &v4)) return false;
+    lanes_t in = sample_uv_f32<BIG>(f0, g, x0, y0, &u1, &v1);
+    in &= sample_uv_f32<BIG>(fh, g, fma((double)u1, hh, x0), fma((double)v1, hh, y0), &u2, &v2);
+    in &= sample_uv_f32<BIG>(fh, g, fma((double)u2, hh, x0), fma((double)v2, hh, y0), &u3, &v3);
+    in &= sample_uv_f32<BIG>(f1, g, fma((double)u3, h, x0), fma((double)v3, h, y0), &u4, &v4);
+    const bool inside = __builtin_amdgcn_inverse_ballot_w64(in);
     const float su = fmaf(2.0f, u2 + u3, u1 + u4);
     const float sv = fmaf(2.0f, v2 + v3, v1 + v4);
-    *x = fma((double)su, h6, x0);
-    *y = fma((double)sv, h6, y0);
-    return true;
+    *x = inside ? fma((double)su, h6, x0) : x0;
+    *y = inside ? fma((double)sv, h6, y0) : y0;
+    return inside;
 }
 
+template <bool WALK, bool BIG>
 __global__ void __launch_bounds__(kBlock)
 advect_rk4_f32_kernel(int64_t n, double* __restrict__ lon, double* __restrict__ lat,
                       const float* __restrict__ fields, int64_t stage_stride, lm_grid g, int nsteps, double hh,
@@ -185,17 +190,13 @@ advect_rk4_f32_kernel(int64_t n, double* __restrict__ lon, double* __restrict__ 
     double x = lon[i], y = lat[i];
     for (int s = 0; s < nsteps; ++s) {
         const float* f0 = fields + (int64_t)(2 * s) * stage_stride;
-        if (!rk4_step_f32(f0, f0 + stage_stride, f0 + 2 * stage_stride, g, hh, h, h6, &x, &y))
+        if (!rk4_step_f32<BIG>(f0, f0 + stage_stride, f0 + 2 * stage_stride, g, hh, h, h6, &x, &y))
             atomicAdd(oob_count, 1u);
         if (rec_lon) {
             rec_lon[(int64_t)s * rec_stride + i] = (float)x;
             rec_lat[(int64_t)s * rec_stride + i] = (float)y;
         }
-        if (walk_amp > 0.0) {
-            const philox4x64 r = philox4x64_10((uint64_t)i, step0 + (uint64_t)s, kStreamWalk, 0, k0, k1);
-            y = fma(fma(2.0, u01_from_u64(r.v[0]), -1.0), walk_amp, y);
-            x = fma(fma(2.0, u01_from_u64(r.v[1]), -1.0), walk_amp, x);
-        }
+        if constexpr (WALK) walk_step((uint64_t)i, step0 + (uint64_t)s, k0, k1, walk_amp, &x, &y);
     }
     lon[i] = x;
     lat[i] = y;
@@ -251,9 +252,17 @@ int lm_advect_rk4_f64(int64_t n, double* lon, double* lat, const double* stage_f
     LM_REQUIRE(((uintptr_t)stage_fields & 15) == 0 && (stage_stride % 2) == 0, LM_ERR_ARG,
                "stage fields must be 16-byte aligned");
     const double hh = 0.5 * dt, h6 = dt / 6.0;
-    LM_LAUNCH(lm::K_ADVECT, lm::advect_rk4_f64_kernel, dim3(lm::grid_for(n)), dim3(lm::kBlock), 0,
-              (hipStream_t)stream, n, lon, lat, stage_fields, stage_stride, *grid, (int)nsteps, hh, dt, h6,
-              rec_lon, rec_lat, rec_stride, walk_amp, key0, key1, step0, oob_count);
+    // the walk's generator takes a kernel of its own (its keys and products
+    // would cost every run a third of the scalar registers), and so do fields
+    // past 32-bit offsets
+    const bool walk = walk_amp > 0.0, big = !lm::fits_offset32(*grid, 16);
+    auto launch = [&](auto kernel) {
+        LM_LAUNCH(lm::K_ADVECT, kernel, dim3(lm::grid_for(n)), dim3(lm::kBlock), 0, (hipStream_t)stream, n, lon, lat, stage_fields, stage_stride, *grid, (int)nsteps, hh, dt, h6, rec_lon, rec_lat, rec_stride, walk_amp, key0, key1, step0, oob_count);
+    };
+    if (walk && big) launch(lm::advect_rk4_f64_kernel<true, true>);
+    else if (walk) launch(lm::advect_rk4_f64_kernel<true, false>);
+    else if (big) launch(lm::advect_rk4_f64_kernel<false, true>);
+    else launch(lm::advect_rk4_f64_kernel<false, false>);
     LM_LAUNCH_CHECK();
     return LM_OK;
 }
@@ -292,9 +301,17 @@ int lm_advect_rk4_f32(int64_t n, double* lon, double* lat, const float* stage_fi
     LM_REQUIRE(((uintptr_t)stage_fields & 7) == 0 && (stage_stride % 2) == 0, LM_ERR_ARG,
                "stage fields must be 8-byte aligned");
     const double hh = 0.5 * dt, h6 = dt / 6.0;
-    LM_LAUNCH(lm::K_ADVECT_F32, lm::advect_rk4_f32_kernel, dim3(lm::grid_for(n)), dim3(lm::kBlock), 0,
-              (hipStream_t)stream, n, lon, lat, stage_fields, stage_stride, *grid, (int)nsteps, hh, dt, h6,
-              rec_lon, rec_lat, rec_stride, walk_amp, key0, key1, step0, oob_count);
+    // the walk's generator takes a kernel of its own (its keys and products
+    // would cost every run a third of the scalar registers), and so do fields
+    // past 32-bit offsets
+    const bool walk = walk_amp > 0.0, big = !lm::fits_offset32(*grid, 8);
+    auto launch = [&](auto kernel) {
+        LM_LAUNCH(lm::K_ADVECT_F32, kernel, dim3(lm::grid_for(n)), dim3(lm::kBlock), 0, (hipStream_t)stream, n, lon, lat, stage_fields, stage_stride, *grid, (int)nsteps, hh, dt, h6, rec_lon, rec_lat, rec_stride, walk_amp, key0, key1, step0, oob_count);
+    };
+    if (walk && big) launch(lm::advect_rk4_f32_kernel<true, true>);
+    else if (walk) launch(lm::advect_rk4_f32_kernel<true, false>);
+    else if (big) launch(lm::advect_rk4_f32_kernel<false, true>);
+    else launch(lm::advect_rk4_f32_kernel<false, false>);
     LM_LAUNCH_CHECK();
     return LM_OK;
 }

@@ -130,14 +130,9 @@ struct philox4x64 {
 };
 
 __host__ __device__ inline void mulhilo64(uint64_t a, uint64_t b, uint64_t* hi, uint64_t* lo) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    *lo = a * b;
-    *hi = __umul64hi(a, b);
-#else
-    unsigned __int128 p = (unsigned __int128)a * (unsigned __int128)b;
+    const unsigned __int128 p = (unsigned __int128)a * (unsigned __int128)b;
     *lo = (uint64_t)p;
     *hi = (uint64_t)(p >> 64);
-#endif
 }
 
 __host__ __device__ inline philox4x64 philox4x64_10(uint64_t c0, uint64_t c1, uint64_t c2,
