@@ -49,12 +49,15 @@
 // launched with adds its moments to a global slab, turned into node values
 // at the end.
 #include "lm_common.h"
+#include "lm_rk4.h"
 
 #include <mutex>
 
 namespace lm {
 
 constexpr int kAdjBlock = 256;
+
+LM_DEFINE_COS_COEFS(adjoint_cos)
 
 // 1 / c by two Newton steps from the hardware reciprocal estimate.
 __device__ __forceinline__ double recip(double c) {
@@ -84,69 +87,35 @@ struct AdjStage {
 // Cell and fractional position as the FP64 path computes them; false outside.
 __device__ __forceinline__ bool adj_locate(const lm_grid& g, double x, double y, int* i, int* j, double* xi,
                                            double* eta) {
-    const double fx = (x - g.x0) * g.inv_dx;
-    const double fy = (y - g.y0) * g.inv_dy;
-    if (!(fx >= 0.0 && fx <= (double)(g.nx - 1) && fy >= 0.0 && fy <= (double)(g.ny - 1))) return false;
-    int ii = (int)fx, jj = (int)fy;
-    ii = ii > g.nx - 2 ? g.nx - 2 : ii;
-    jj = jj > g.ny - 2 ? g.ny - 2 : jj;
-    *i = ii;
-    *j = jj;
-    *xi = fx - (double)ii;
-    *eta = fy - (double)jj;
-    return true;
+    uint32_t ci, cj;
+    const lanes_t in = locate_axis(x, g.x0, g.inv_dx, g.nx, &ci, xi) & locate_axis(y, g.y0, g.inv_dy, g.ny, &cj, eta);
+    *i = (int)ci;
+    *j = (int)cj;
+    return __builtin_amdgcn_inverse_ballot_w64(in);
 }
 
-// Corners (j,i), (j,i+1), (j+1,i), (j+1,i+1) of stage time s.
-__device__ __forceinline__ void adj_corners(const AdjField& F, int s, int i, int j, double2 q[4]) {
-    const double2* r0 = F.st + (int64_t)(s - F.k0) * F.sstride + (int64_t)j * F.g.nx + i;
-    const double2* r1 = r0 + F.g.nx;
-    q[0] = r0[0];
-    q[1] = r0[1];
-    q[2] = r1[0];
-    q[3] = r1[1];
-}
-
-// The FP64 path's sample, bit for bit; also returns the cell.
-__device__ __forceinline__ bool adj_sample(const AdjField& F, int s, double x, double y, double* ud, double* vd,
-                                           int* ci, int* cj) {
-    int i, j;
+// sample_uv with 1/cos(lat) from recip(): within rounding of it.
+template <bool BIG>
+__device__ __forceinline__ lanes_t sample_uv_fast(const double* __restrict__ f, const lm_grid& g, const CosCoefs& K,
+                                                  double x, double y, double* ud, double* vd, uint32_t* ci,
+                                                  uint32_t* cj) {
     double xi, eta;
-    if (!adj_locate(F.g, x, y, &i, &j, &xi, &eta)) return false;
-    double2 q[4];
-    adj_corners(F, s, i, j, q);
-    const double ub = fma(xi, q[1].x - q[0].x, q[0].x);
-    const double ut = fma(xi, q[3].x - q[2].x, q[2].x);
+    const lanes_t in_x = locate_axis(x, g.x0, g.inv_dx, g.nx, ci, &xi);
+    const lanes_t in_y = locate_axis(y, g.y0, g.inv_dy, g.ny, cj, &eta);
+    const auto off = node_offset<16, BIG>(g, *ci, *cj);
+    const char* row = reinterpret_cast<const char*>(f);
+    const double2* r0 = reinterpret_cast<const double2*>(row + off);
+    const double2* r1 = reinterpret_cast<const double2*>(row + 16 * (int64_t)g.nx + off);
+    const double2 a = r0[0], b = r0[1], c = r1[0], d = r1[1];
+    const double ub = fma(xi, b.x - a.x, a.x);
+    const double ut = fma(xi, d.x - c.x, c.x);
     const double u = fma(eta, ut - ub, ub);
-    const double vb = fma(xi, q[1].y - q[0].y, q[0].y);
-    const double vt = fma(xi, q[3].y - q[2].y, q[2].y);
+    const double vb = fma(xi, b.y - a.y, a.y);
+    const double vt = fma(xi, d.y - c.y, c.y);
     const double v = fma(eta, vt - vb, vb);
-    *ud = (u * LM_INV_M_PER_DEG) / cos_deg(y);
+    *ud = u * (LM_INV_M_PER_DEG * recip(cos_deg_from(K, y)));
     *vd = v * LM_INV_M_PER_DEG;
-    *ci = i;
-    *cj = j;
-    return true;
-}
-
-// The same with 1/cos(lat) from recip(): within rounding of adj_sample.
-__device__ __forceinline__ bool adj_sample_fast(const AdjField& F, int s, double x, double y, double* ud,
-                                                double* vd, int* ci, int* cj) {
-    int i, j;
-    double xi, eta;
-    if (!adj_locate(F.g, x, y, &i, &j, &xi, &eta)) return false;
-    double2 q[4];
-    adj_corners(F, s, i, j, q);
-    const double ub = fma(xi, q[1].x - q[0].x, q[0].x);
-    const double ut = fma(xi, q[3].x - q[2].x, q[2].x);
-    const double u = fma(eta, ut - ub, ub);
-    const double vb = fma(xi, q[1].y - q[0].y, q[0].y);
-    const double vt = fma(xi, q[3].y - q[2].y, q[2].y);
-    const double v = fma(eta, vt - vb, vb);
-    *ud = u * (LM_INV_M_PER_DEG * recip(cos_deg(y)));
-    *vd = v * LM_INV_M_PER_DEG;
-    *ci = i;
-    *cj = j;
-    return true;
+    return in_x & in_y;
 }
 
 // Cell bounding box of one lane's stage samples.
@@ -165,30 +134,34 @@ struct CellBox {
 };
 
 // One RK4 step in the FP64 path's operation order (FAST: with
-// adj_sample_fast); false (position kept) if a stage leaves the grid.  With
+// sample_uv_fast); false (position kept) if a stage leaves the grid.  With
 // box != NULL the stage cells of a completed step are added to it.
-template <bool FAST>
-__device__ __forceinline__ bool adj_rk4(const AdjField& F, int s, double hh, double h, double h6, double* x,
-                                       double* y, CellBox* box) {
+template <bool FAST, bool BIG>
+__device__ __forceinline__ bool adj_rk4(const AdjField& F, const CosCoefs& K, int s, double hh, double h, double h6,
+                                        double* x, double* y, CellBox* box) {
     double u1, v1, u2, v2, u3, v3, u4, v4;
-    int i1, j1, i2, j2, i3, j3, i4, j4;
+    uint32_t i1, j1, i2, j2, i3, j3, i4, j4;
     const double x0 = *x, y0 = *y;
-    auto sample = [&](int st, double px, double py, double* ud, double* vd, int* ci, int* cj) {
-        return FAST ? adj_sample_fast(F, st, px, py, ud, vd, ci, cj) : adj_sample(F, st, px, py, ud, vd, ci, cj);
+    s = __builtin_amdgcn_readfirstlane(s);  // uniform: the stage fields' pointers stay in scalar registers
+    auto sample = [&](int st, double px, double py, double* ud, double* vd, uint32_t* ci, uint32_t* cj) {
+        const double* f = reinterpret_cast<const double*>(F.st + (int64_t)(st - F.k0) * F.sstride);
+        if constexpr (FAST) return sample_uv_fast<BIG>(f, F.g, K, px, py, ud, vd, ci, cj);
+        else return sample_uv<BIG>(f, F.g, K, px, py, ud, vd, ci, cj);
     };
-    if (!sample(2 * s, x0, y0, &u1, &v1, &i1, &j1)) return false;
-    if (!sample(2 * s + 1, fma(u1, hh, x0), fma(v1, hh, y0), &u2, &v2, &i2, &j2)) return false;
-    if (!sample(2 * s + 1, fma(u2, hh, x0), fma(v2, hh, y0), &u3, &v3, &i3, &j3)) return false;
-    if (!sample(2 * s + 2, fma(u3, h, x0), fma(v3, h, y0), &u4, &v4, &i4, &j4)) return false;
+    lanes_t in = sample(2 * s, x0, y0, &u1, &v1, &i1, &j1);
+    in &= sample(2 * s + 1, fma(u1, hh, x0), fma(v1, hh, y0), &u2, &v2, &i2, &j2);
+    in &= sample(2 * s + 1, fma(u2, hh, x0), fma(v2, hh, y0), &u3, &v3, &i3, &j3);
+    in &= sample(2 * s + 2, fma(u3, h, x0), fma(v3, h, y0), &u4, &v4, &i4, &j4);
+    if (!__builtin_amdgcn_inverse_ballot_w64(in)) return false;
     const double su = fma(2.0, u2 + u3, u1 + u4);
     const double sv = fma(2.0, v2 + v3, v1 + v4);
     *x = fma(su, h6, x0);
     *y = fma(sv, h6, y0);
     if (box) {
-        box->add(j1, i1);
-        box->add(j2, i2);
-        box->add(j3, i3);
-        box->add(j4, i4);
+        box->add((int)j1, (int)i1);
+        box->add((int)j2, (int)i2);
+        box->add((int)j3, (int)i3);
+        box->add((int)j4, (int)i4);
     }
     return true;
 }
@@ -490,6 +463,7 @@ adj_blend_kernel(const float2* __restrict__ lev, int64_t level_len, int64_t lstr
 
 // Steps [s_begin, s_end) of the run; the positions at the start of each
 // step s with s % ckpt == 0 go to checkpoint s / ckpt.
+template <bool BIG>
 __global__ void __launch_bounds__(kAdjBlock)
 adj_forward_kernel(int64_t n, double* __restrict__ lon, double* __restrict__ lat, AdjField F, int s_begin, int s_end,
                    double hh, double h, double h6, int ckpt, double2* __restrict__ ck, uint32_t* __restrict__ oob) {
@@ -499,9 +473,10 @@ adj_forward_kernel(int64_t n, double* __restrict__ lon, double* __restrict__ lat
     if (i >= n) return;
     double x = lon[i], y = lat[i];
     uint32_t out = 0;
+    const CosCoefs K = load_adjoint_cos();
     for (int s = s_begin; s < s_end; ++s) {
         if (s % ckpt == 0) ck[(int64_t)(s / ckpt) * n + i] = make_double2(x, y);
-        if (!adj_rk4<false>(F, s, hh, h, h6, &x, &y, nullptr)) ++out;
+        if (!adj_rk4<false, BIG>(F, K, s, hh, h, h6, &x, &y, nullptr)) ++out;
     }
     lon[i] = x;
     lat[i] = y;
@@ -510,6 +485,7 @@ adj_forward_kernel(int64_t n, double* __restrict__ lon, double* __restrict__ lat
 
 // Steps s0 .. s0 + m - 1 from the checkpoint ck: the start position of step
 // s0 + k into pos[k * n + i]; the block's cell box into box[block].
+template <bool BIG>
 __global__ void __launch_bounds__(kAdjBlock)
 adj_recompute_kernel(int64_t n, const double2* __restrict__ ck, AdjField F, int s0, int m, double hh, double h,
                      double h6, double2* __restrict__ pos, int4* __restrict__ box) {
@@ -527,9 +503,10 @@ adj_recompute_kernel(int64_t n, const double2* __restrict__ ck, AdjField F, int 
     if (i < n) {
         const double2 p = ck[i];
         double x = p.x, y = p.y;
+        const CosCoefs K = load_adjoint_cos();
         for (int k = 0; k < m; ++k) {
             pos[(int64_t)k * n + i] = make_double2(x, y);
-            adj_rk4<true>(F, s0 + k, hh, h, h6, &x, &y, &cb);
+            adj_rk4<true, BIG>(F, K, s0 + k, hh, h, h6, &x, &y, &cb);
         }
     }
     if (cb.jmax >= 0) {
@@ -884,9 +861,13 @@ int lm_adjoint_forward(int64_t n, double* lon, double* lat, const float* field, 
         lm::AdjField F;
         rc = adj_blend(field, nlev, grid, lev0, w, 2 * a, 2 * (b - a) + 1, buf, s, &F);
         if (rc) return rc;
-        LM_LAUNCH(lm::K_ADJ_FORWARD, lm::adj_forward_kernel, dim3(lm::grid_for(n, lm::kAdjBlock)),
-                  dim3(lm::kAdjBlock), 0, s, n, lon, lat, F, a, b, 0.5 * dt, dt, dt / 6.0, (int)ckpt,
-                  reinterpret_cast<double2*>(checkpoints), oob_count);
+        auto launch = [&](auto kernel) {
+            LM_LAUNCH(lm::K_ADJ_FORWARD, kernel, dim3(lm::grid_for(n, lm::kAdjBlock)), dim3(lm::kAdjBlock), 0, s, n,
+                      lon, lat, F, a, b, 0.5 * dt, dt, dt / 6.0, (int)ckpt, reinterpret_cast<double2*>(checkpoints),
+                      oob_count);
+        };
+        if (lm::fits_offset32(*grid, 16)) launch(lm::adj_forward_kernel<false>);
+        else launch(lm::adj_forward_kernel<true>);
         LM_LAUNCH_CHECK();
     }
     return LM_OK;
@@ -955,8 +936,12 @@ int lm_adjoint_backward(int64_t n, const double* checkpoints, const float* field
         lm::AdjField F;
         rc = adj_blend(field, nlev, grid, lev0, w, 2 * s0, 2 * m + 1, stage, s, &F);
         if (rc) return rc;
-        LM_LAUNCH(lm::K_ADJ_RECOMPUTE, lm::adj_recompute_kernel, dim3(nb), dim3(lm::kAdjBlock), 0, s, n,
-                  ck + (int64_t)seg * n, F, s0, m, hh, dt, h6, pos, box);
+        auto recompute = [&](auto kernel) {
+            LM_LAUNCH(lm::K_ADJ_RECOMPUTE, kernel, dim3(nb), dim3(lm::kAdjBlock), 0, s, n, ck + (int64_t)seg * n, F, s0,
+                      m, hh, dt, h6, pos, box);
+        };
+        if (lm::fits_offset32(*grid, 16)) recompute(lm::adj_recompute_kernel<false>);
+        else recompute(lm::adj_recompute_kernel<true>);
         LM_LAUNCH_CHECK();
         LM_LAUNCH(lm::K_ADJ_BACKWARD, lm::adj_backward_kernel, dim3(nb), dim3(lm::kAdjBlock),
                   (unsigned)kAdjWindowBytes, s, n, V, lev0, w, (int)nlev, s0, m, hh, dt, h6, pos, box, glon, glat,
