@@ -356,10 +356,21 @@ struct GradSink {
     int cx, cy;   // cells along x, y
 };
 
+// A lane's register k holds counter k ^ kswap(lane) of the slot: neighbouring
+// lanes sit in the same few cells, and where a wavefront flushes together
+// (a segment's end, a change of level pair) its lanes would meet at one
+// counter, one add per cycle, 16 counters in turn.  With the counters
+// permuted, 16 neighbouring lanes add to 16 different ones.  The permutation
+// is applied to the factors of the moments (eight selects per sample, and no
+// moving of registers: rotating the sums at each flush was slower than the
+// conflicts).  Sweep back of 1,000,000 particles: 8.10 -> 7.22 ms; with only
+// the two high bits permuted 7.81; with slots padded to 17 floats alone 8.04.
 struct GradCache {
     int l, cell;  // l < 0: empty; cell = (j << 16) | i
-    float m[16];  // [comp][S, W][moment]
+    float m[16];  // [comp][S, W][moment], permuted
 };
+
+__device__ __forceinline__ int kswap() { return (int)(threadIdx.x & 15u); }
 
 __device__ __forceinline__ float corner_of(const float* m, int dj, int di) {
     const float m3 = m[3];
@@ -372,7 +383,7 @@ __device__ __forceinline__ float corner_of(const float* m, int dj, int di) {
 // win: the block's window in LDS (read only when B.win).
 __device__ __forceinline__ void cache_flush(GradCache& gc, const BlockBox& B, float* win, const GradSink& sk) {
     if (gc.l < 0) return;
-    const int cj = gc.cell >> 16, ci = gc.cell & 0xffff;
+    const int cj = (int)((uint32_t)gc.cell >> 16), ci = gc.cell & 0xffff, x = kswap();
     const int t = B.win ? box_index(B, gc.l, ci, cj) : -1;
     if (t >= 0) {
         // workgroup scope, unlike the slab's device-scope atomics: the two
@@ -381,11 +392,11 @@ __device__ __forceinline__ void cache_flush(GradCache& gc, const BlockBox& B, fl
         float* slot = win + t * 16;
 #pragma unroll
         for (int k = 0; k < 16; ++k)
-            __hip_atomic_fetch_add(slot + k, gc.m[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            __hip_atomic_fetch_add(slot + (k ^ x), gc.m[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     } else {
         float* slot = sk.slab + (((int64_t)gc.l * sk.cy + cj) * sk.cx + ci) * 16;
 #pragma unroll
-        for (int k = 0; k < 16; ++k) atomicAdd(slot + k, gc.m[k]);
+        for (int k = 0; k < 16; ++k) atomicAdd(slot + (k ^ x), gc.m[k]);
     }
     gc.l = -1;
 }
@@ -419,17 +430,20 @@ __device__ __forceinline__ float node_from_slots(int lv, int nj, int ni, bool st
 
 // Adds one stage sample to the cache's moments: velocity adjoints (gu, gv)
 // already scaled to m/s, time weight w, fractional position (xi, eta).
+// Counter k = (comp, S/W, eta, xi) is the product of four factors, one chosen
+// by each bit of k; a lane's permutation swaps the two choices of a bit.
 __device__ __forceinline__ void cache_accumulate(GradCache& gc, float w, float xi, float eta, float gu, float gv) {
-    const float b[4] = {1.0f, xi, eta, xi * eta};
-    const float g[2] = {gu, gv};
+    const int x = kswap();
+    const float g[2] = {x & 8 ? gv : gu, x & 8 ? gu : gv};
+    const float f[2] = {x & 4 ? w : 1.0f, x & 4 ? 1.0f : w};
+    const float e[2] = {x & 2 ? eta : 1.0f, x & 2 ? 1.0f : eta};
+    const float q[2] = {x & 1 ? xi : 1.0f, x & 1 ? 1.0f : xi};
+    const float b[4] = {e[0] * q[0], e[0] * q[1], e[1] * q[0], e[1] * q[1]};
 #pragma unroll
-    for (int comp = 0; comp < 2; ++comp) {
-        const float gw = g[comp] * w;
+    for (int c = 0; c < 4; ++c) {
+        const float gf = g[c >> 1] * f[c & 1];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            gc.m[comp * 8 + k] = fmaf(g[comp], b[k], gc.m[comp * 8 + k]);
-            gc.m[comp * 8 + 4 + k] = fmaf(gw, b[k], gc.m[comp * 8 + 4 + k]);
-        }
+        for (int k = 0; k < 4; ++k) gc.m[c * 4 + k] = fmaf(gf, b[k], gc.m[c * 4 + k]);
     }
 }
 
