@@ -202,10 +202,20 @@ class TrajectoryLoss(torch.autograd.Function):
             got = iter(torch.autograd.grad(loss, wanted, by, create_graph=True))
             return tuple(next(got) if w else None for w in need)
         n = inputs[0].numel()
-        out = torch.empty_like(grad)
-        by = by.to(torch.float64).contiguous()
-        check(_lib.load().lm_scale_by(out.numel(), ptr(grad), ptr(by), ptr(out), stream_ptr()))
+        if _watched() or type(by) is not torch.Tensor or not torch._C._has_storage(by):
+            out = grad * by  # a batch of gradients (vectorised Jacobians), or a mode that has to see the operation
+        else:
+            out = torch.empty_like(grad)
+            by = by.to(torch.float64).contiguous()
+            check(_lib.load().lm_scale_by(out.numel(), ptr(grad), ptr(by), ptr(out), stream_ptr()))
         return tuple(out[k * n:(k + 1) * n].view(inputs[0].shape) if w else None for k, w in enumerate(need))
+
+
+def _watched():
+    """Whether a trace, a transform or a mode has to see the single operations."""
+    return (torch.compiler.is_compiling() or torch.jit.is_tracing()
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0)
 
 
 def _plain_f64(tensors):
@@ -218,9 +228,7 @@ def _plain_f64(tensors):
         return False
     if t0.device.type != "cuda" or t0.device.index != torch.cuda.current_device() or t0.numel() == 0:
         return False
-    if torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._functorch.peek_interpreter_stack() is not None:
-        return False
-    if torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack():
+    if _watched():
         return False
     return not any(torch.autograd.forward_ad.unpack_dual(t).tangent is not None for t in tensors) \
         if torch.autograd.forward_ad._current_level >= 0 else True

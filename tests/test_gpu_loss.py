@@ -68,3 +68,18 @@ def test_other_calls_take_the_single_operations(gpu):
     with torch.no_grad():
         y.add_(1.0)
     torch.testing.assert_close(torch.autograd.grad(loss, x)[0], g)
+
+
+@pytest.mark.parametrize("need", [(1, 1, 0, 0), (0, 1, 1, 0)])
+def test_a_batch_of_gradients_at_once(gpu, need):
+    args = inputs(40, 7, need)
+    wanted = [t for t in args if t.requires_grad]
+    by = torch.tensor([0.5, -2.0, 1.0], dtype=torch.float64, device="cuda")
+    got = torch.autograd.grad(adjoint.trajectory_loss(*args), wanted, by, is_grads_batched=True)
+    for k in range(3):
+        one = torch.autograd.grad(adjoint.trajectory_loss(*args), wanted, by[k])
+        for a, b in zip(got, one):
+            torch.testing.assert_close(a[k], b, rtol=1e-15, atol=0.0)
+    got = torch.autograd.functional.jacobian(lambda t: adjoint.trajectory_loss(args[0], t, args[2], args[3]),
+                                             args[1].detach(), vectorize=True)
+    torch.testing.assert_close(got, one[need[0]], rtol=1e-15, atol=0.0)
