@@ -36,7 +36,7 @@
 //                        places every component's pairs in one run, in order
 //           7. comps     per particle its slot (position minus its root's) and
 //                        the shift from pair rank to run position; each
-//                        component listed once, as small (<= 32 pairs) or wide
+//                        component listed once, as small (<= 16 or 32 pairs) or wide
 //           8. fill      pair records (slot_i | bits << 29, slot_j) at their
 //                        run positions
 //           9. links     for the wide components, per 64-pair window, the pair
@@ -46,7 +46,7 @@
 // Only the replay itself runs per step, in one launch of one-wavefront blocks:
 //   wide     one wavefront per larger component, species in LDS, a window of
 //            64 pairs at a time, each solved as a fixed point
-//   small    one lane per component of <= 32 pairs, replayed in order
+//   small    one lane per component of <= 16 or 32 pairs, replayed in order
 //   copy     particles without pairs keep their species
 //
 // Small populations (workspaces of kSmallMax particles, no runs) take two kernels instead,
@@ -60,7 +60,15 @@
 namespace lm {
 
 constexpr uint32_t kUnset = 0xffffffffu;
-constexpr uint32_t kNarrowPairs = 32;
+// A component of up to 32 pairs is small: one lane replays it, pair after pair
+// (about 100 ns each); a larger one takes a wavefront.  Up to kFewParticles
+// particles the limit is 16: a step's replay then waits for its longest serial
+// chain, and the components between the limits find wavefronts free.  124,000
+// particles, 60 steps: 1,748 us with 32, 1,572 with 16; 30,000: 990 and 880;
+// but 242,000 dense ones, 100 steps: 6.50 and 6.74 ms, and 4,000,000, 96
+// steps: 81.9 and 87.2 ms, where these components are thousands.
+constexpr uint32_t kNarrowPairs = 32, kNarrowPairsFew = 16;
+constexpr int64_t kFewParticles = 1 << 17;
 constexpr uint32_t kNarrowSlots = kNarrowPairs + 1;  // a component of P pairs has <= P + 1 particles
 constexpr uint32_t kSlotMask = (1u << 29) - 1u;
 constexpr int kCompItems = 4;                        // sorted positions per thread when listing components
@@ -629,7 +637,7 @@ rps_group_blk_kernel(int64_t n, RpsArrays A, RpsStrides st, const uint32_t* __re
 // lists its component.  A block takes kCompItems positions per thread and
 // reserves its list entries with one global add per list.
 __global__ void __launch_bounds__(kBlock)
-rps_comps_kernel(int64_t n, RpsArrays A, RpsStrides st) {
+rps_comps_kernel(int64_t n, RpsArrays A, RpsStrides st, uint32_t narrow) {
     uint32_t bx, by;
     xcd_block(&bx, &by);  // an XCD works through a contiguous range of steps: one step's arrays in its L2
     __shared__ uint32_t cnt[2], base[2];
@@ -681,7 +689,7 @@ rps_comps_kernel(int64_t n, RpsArrays A, RpsStrides st) {
             const uint32_t pe = A.pend[ro + L[r]];
             const uint32_t qb = min(ro_e[r], P), qe = min(roff[pe], P);
             d[r] = make_uint4(qb, qe > qb ? qe - qb : 0u, (uint32_t)e, pe - (uint32_t)e);
-            const uint32_t wide = d[r].y > kNarrowPairs ? 1u : 0u;
+            const uint32_t wide = d[r].y > narrow ? 1u : 0u;
             at[r] = (wide << 31) | atomicAdd(&cnt[wide], 1u);
         }
     }
@@ -977,21 +985,30 @@ __device__ __forceinline__ void play_narrow(int64_t n, const uint32_t* __restric
     if (psz == 0) return;
     // every load is clamped inside the component rather than guarded, so
     // none waits behind a branch: the species of kStage slots at a time are
-    // gathered together, and the records of the next 8 pairs load while the
-    // current 8 play
+    // gathered together, while the indices of the next kStage load, and the
+    // records of the next 8 pairs load while the current 8 play
     uint2 r[8];
+    uint32_t x[kStage], first[kStage];
+#pragma unroll
+    for (int q = 0; q < kStage; ++q) x[q] = first[q] = ids[pb + min((uint32_t)q, psz - 1u)];
 #pragma unroll
     for (uint32_t q = 0; q < 8; ++q) r[q] = np > 0 ? rec[qb + min(q, np - 1u)] : make_uint2(0u, 0u);
     for (uint32_t t0 = 0; t0 < psz; t0 += kStage) {
-        uint32_t x[kStage];
+        uint32_t xn[kStage];
         int8_t v[kStage];
-#pragma unroll
-        for (int q = 0; q < kStage; ++q) x[q] = ids[pb + min(t0 + q, psz - 1u)];
 #pragma unroll
         for (int q = 0; q < kStage; ++q) v[q] = sp_in[x[q] < (uint64_t)n ? x[q] : 0u];
 #pragma unroll
+        for (int q = 0; q < kStage; ++q) xn[q] = 0u;
+        if (t0 + kStage < psz) {
+#pragma unroll
+            for (int q = 0; q < kStage; ++q) xn[q] = ids[pb + min(t0 + kStage + q, psz - 1u)];
+        }
+#pragma unroll
         for (int q = 0; q < kStage; ++q)
             if (t0 + q < psz) my[t0 + q] = x[q] < (uint64_t)n ? v[q] : (int8_t)0;
+#pragma unroll
+        for (int q = 0; q < kStage; ++q) x[q] = xn[q];
     }
     for (uint32_t q0 = 0; q0 < np; q0 += 8) {
         uint2 rn[8];
@@ -1003,16 +1020,23 @@ __device__ __forceinline__ void play_narrow(int64_t n, const uint32_t* __restric
 #pragma unroll
         for (uint32_t q = 0; q < 8; ++q) r[q] = rn[q];
     }
+    // back: the first kStage indices are still here, the next load ahead
     for (uint32_t t0 = 0; t0 < psz; t0 += kStage) {
-        uint32_t x[kStage];
+        uint32_t xn[kStage];
         int8_t v[kStage];
 #pragma unroll
-        for (int q = 0; q < kStage; ++q) x[q] = ids[pb + min(t0 + q, psz - 1u)];
+        for (int q = 0; q < kStage; ++q) xn[q] = 0u;
+        if (t0 + kStage < psz) {
+#pragma unroll
+            for (int q = 0; q < kStage; ++q) xn[q] = ids[pb + min(t0 + kStage + q, psz - 1u)];
+        }
 #pragma unroll
         for (int q = 0; q < kStage; ++q) v[q] = my[min(t0 + q, psz - 1u)];
 #pragma unroll
         for (int q = 0; q < kStage; ++q)
-            if (t0 + q < psz && x[q] < (uint64_t)n) sp_out[x[q]] = v[q];
+            if (t0 + q < psz && first[q] < (uint64_t)n) sp_out[first[q]] = v[q];
+#pragma unroll
+        for (int q = 0; q < kStage; ++q) first[q] = xn[q];
     }
 }
 
@@ -1024,9 +1048,11 @@ rps_play_kernel(int64_t n, int64_t s, RpsArrays A, RpsStrides st, const int8_t* 
     const uint32_t lane = threadIdx.x;
     const uint32_t bid = blockIdx.x;
     if (bid < nwide) {
+        uint4 dsc = A.wide[ro + min((int64_t)bid, st.row - 1)];  // loads beside the count
         const uint32_t cnt = A.lists[4 * s + 1];
+        lm_pin(dsc.x, dsc.y, dsc.z, dsc.w);
         for (uint32_t c = bid; c < cnt; c += nwide) {
-            const uint4 dsc = A.wide[ro + c];
+            if (c != bid) dsc = A.wide[ro + c];
             const uint32_t qb = dsc.x, np = dsc.y, pb = dsc.z, psz = dsc.w;
             if (psz >= 1)
                 play_wide(n, A.ids + ro + pb, psz, A.rec + po + qb, A.links + po + qb, np, sp_in, sp_out, slots);
@@ -1035,10 +1061,17 @@ rps_play_kernel(int64_t n, int64_t s, RpsArrays A, RpsStrides st, const int8_t* 
         return;
     }
     if (bid < nwide + nnarrow) {
+        // the count and the lane's first descriptor load together
+        uint32_t c = (bid - nwide) * 64 + lane;
+        uint4 dsc = A.narrow[ro + min((int64_t)c, st.row - 1)];
         const uint32_t cnt = A.lists[4 * s + 0];
+        lm_pin(dsc.x, dsc.y, dsc.z, dsc.w);
         int8_t* my = slots + lane * kNarrowSlots;
-        for (uint32_t c = (bid - nwide) * 64 + lane; c < cnt; c += nnarrow * 64)
-            play_narrow(n, A.ids + ro, A.rec + po, A.narrow[ro + c], sp_in, sp_out, my);
+        while (c < cnt) {
+            play_narrow(n, A.ids + ro, A.rec + po, dsc, sp_in, sp_out, my);
+            c += nnarrow * 64;
+            if (c < cnt) dsc = A.narrow[ro + c];
+        }
         return;
     }
     // particles without pairs (touched 0) keep their species; the others
@@ -1394,8 +1427,8 @@ rps_stats_kernel(int64_t s, RpsArrays A, RpsStrides st, int64_t* __restrict__ st
     const uint32_t c0 = A.lists[4 * s + 0], c1 = A.lists[4 * s + 1];
     uint64_t v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     for (uint32_t c = blockIdx.x * kBlock + threadIdx.x; c < c0 + c1; c += gridDim.x * kBlock) {
-        const bool wide = c >= c0;
-        const uint4 d = wide ? A.wide[ro + (c - c0)] : A.narrow[ro + c];
+        const uint4 d = c >= c0 ? A.wide[ro + (c - c0)] : A.narrow[ro + c];
+        const bool wide = d.y > kNarrowPairs;
         v[0] += 1;
         v[1] = v[1] > d.y ? v[1] : d.y;
         v[2] = v[2] > d.w ? v[2] : d.w;
@@ -1584,7 +1617,8 @@ static int rps_prepare_tail(lm_rps_ws* ws, int64_t n, unsigned S, const int32_t*
     int rc = lm::exclusive_scan_u32_batched(A.rcnt, n, ws->row, A.roff, ws->row, (int32_t)S, ws->scan_tmp, nullptr, s);
     if (rc) return rc;
     LM_LAUNCH(lm::K_RPS_COMPS, lm::rps_comps_kernel, dim3((nbp + lm::kCompItems - 1) / lm::kCompItems, S),
-              dim3(lm::kBlock), 0, s, n, A, sp);
+              dim3(lm::kBlock), 0, s, n, A, sp,
+              n <= lm::kFewParticles ? lm::kNarrowPairsFew : lm::kNarrowPairs);
     LM_LAUNCH_CHECK();
     LM_LAUNCH(lm::K_RPS_FILL, lm::rps_fill_kernel, dim3(npb, S), dim3(lm::kBlock), 0, s, n, pair_i, pair_j, A, sp);
     LM_LAUNCH_CHECK();

@@ -1,0 +1,41 @@
+"""The replay's component classes on both sides of their limits, for populations on both sides of
+the size where the small class changes, against the sequential oracle."""
+import numpy as np
+import pytest
+
+import oracle
+from test_gpu_kernels import gpu_rps
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n", [12_289, 131_072, 131_073])
+def test_component_classes(gpu, n):
+    rng = np.random.default_rng(n)
+    # particles and pairs beyond a spanning tree, per component: 16, 17, 32, 33 pairs, one window and
+    # two, the links pass's classes, more slots than the LDS holds
+    sizes = [(s, e) for s in (2, 3, 9, 16, 17, 18, 32, 33, 34) for e in (0, 1, 2)] * 8
+    sizes += [(12, 20), (12, 21), (20, 46), (40, 26), (250, 7), (250, 8), (300, 200), (2049, 100), (4200, 300)]
+    perm, pairs, at, npairs = rng.permutation(n), set(), 0, []
+    for size, extra in sizes:
+        ids = perm[at:at + size]
+        at += size
+        mine = set()
+        for a in range(1, size):
+            b = int(rng.integers(max(0, a - 3), a))
+            mine.add((min(ids[a], ids[b]), max(ids[a], ids[b])))
+        want = min(len(mine) + extra, size * (size - 1) // 2)
+        while len(mine) < want:
+            a, b = rng.choice(ids, 2, replace=False)
+            mine.add((min(a, b), max(a, b)))
+        npairs.append(len(mine))
+        pairs |= mine
+    assert at <= n
+    arr = np.array(sorted(pairs), dtype=np.int32)
+    species = rng.integers(0, 5, n).astype(np.int8)  # 0 and 4 never interact
+    args = (0.5, 0.6, 0.4, (n, 9), 3)
+    got, up = gpu_rps(species, arr[:, 0], arr[:, 1], *args)
+    assert np.array_equal(got, oracle.rps_sequential(species, arr[:, 0], arr[:, 1], *args))
+    st, wide = up.component_stats(), [p for p in npairs if p > 32]
+    assert st.components == len(sizes) and st.pairs == len(arr) and st.max_pairs == max(npairs)
+    assert st.wide_components == len(wide) and st.wide_pairs == sum(wide)
