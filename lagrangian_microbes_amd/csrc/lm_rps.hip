@@ -501,8 +501,13 @@ rps_keys_kernel(int64_t n, RpsArrays A, RpsStrides st, bool write_vals) {
 // 10 bits covers the rest: 9 at 490k particles, whose per-tile digit
 // counters cost half the 10-bit pass's; R = 2, as a super-bucket holds
 // ~2^10 particles),
-// 12 up to 2^22, 14 up to 2^24 (ensembles; 64 KB of counters).
+// 11 up to 2^21 (half the counters to clear and scan and one bit less to rank
+// by than with 12, for a 10-bit radix pass in place of a 9-bit one: sixteen
+// runs of 1,280,000 particles, 96 steps, 21.95 -> 21.30 ms; 1,950,000, 30
+// steps, 13.46 -> 13.14), 12 up to 2^22, 14 up to 2^24 (ensembles; 64 KB of
+// counters).
 constexpr uint32_t kGroupFineBits = 10;
+constexpr uint32_t kGroupFineBitsMid = 11;
 constexpr uint32_t kGroupFineBitsWide = 12;
 constexpr uint32_t kGroupFineBitsHuge = 14;
 constexpr uint32_t kGroupRounds = 8;
@@ -1715,6 +1720,7 @@ static int rps_prepare_impl(lm_rps_ws* ws, int32_t nsteps, int64_t n, const int3
         // bits, then a block per super-bucket counts its roots in LDS
         const int kb = key_bits_for(n);
         const int fb = kb - (int)lm::kGroupFineBits <= lm::kMaxDigitBits ? (int)lm::kGroupFineBits
+                       : kb - (int)lm::kGroupFineBitsMid <= lm::kMaxDigitBits ? (int)lm::kGroupFineBitsMid
                        : kb - (int)lm::kGroupFineBitsWide <= lm::kMaxDigitBits ? (int)lm::kGroupFineBitsWide
                                                                                : (int)lm::kGroupFineBitsHuge;
         const int fine_bits = kb < fb ? kb : fb;
@@ -1737,6 +1743,10 @@ static int rps_prepare_impl(lm_rps_ws* ws, int32_t nsteps, int64_t n, const int3
         }
         if (fb == (int)lm::kGroupFineBits) {
             LM_LAUNCH(lm::K_RPS_GROUP, (lm::rps_group_blk_kernel<lm::kGroupFineBits, 4>), dim3(1u << super_bits, S),
+                      dim3(64 * lm::kGroupWaves), 0, s, n, A, sp, (const uint32_t*)pk[in], (const uint32_t*)pv[in],
+                      pk[1 - in], pv[1 - in], dstart, ws->sort.row, dstride, 1u << fine_bits);
+        } else if (fb == (int)lm::kGroupFineBitsMid) {
+            LM_LAUNCH(lm::K_RPS_GROUP, lm::rps_group_blk_kernel<lm::kGroupFineBitsMid>, dim3(1u << super_bits, S),
                       dim3(64 * lm::kGroupWaves), 0, s, n, A, sp, (const uint32_t*)pk[in], (const uint32_t*)pv[in],
                       pk[1 - in], pv[1 - in], dstart, ws->sort.row, dstride, 1u << fine_bits);
         } else if (fb == (int)lm::kGroupFineBitsWide) {

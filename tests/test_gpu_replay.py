@@ -1,5 +1,5 @@
 """The replay's component classes on both sides of their limits, for populations on both sides of
-the size where the small class changes, against the sequential oracle."""
+the sizes where the small class and the grouping change, against the sequential oracle."""
 import numpy as np
 import pytest
 
@@ -9,7 +9,7 @@ from test_gpu_kernels import gpu_rps
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [12_289, 131_072, 131_073])
+@pytest.mark.parametrize("n", [12_289, 131_072, 131_073, 1 << 20, (1 << 20) + 1, 1 << 21, (1 << 21) + 1])
 def test_component_classes(gpu, n):
     rng = np.random.default_rng(n)
     # particles and pairs beyond a spanning tree, per component: 16, 17, 32, 33 pairs, one window and
