@@ -97,9 +97,14 @@ class FusedRunner:
 
     def reset(self):
         """Back to the initial state, step 0 and the field's first time level."""
-        self.lon = torch.from_numpy(self.lon0.copy()).to(self.device)
-        self.lat = torch.from_numpy(self.lat0.copy()).to(self.device)
-        self.species = torch.from_numpy(self.species0.copy()).to(self.device)
+        def upload(a):
+            # .to() has read the array when it returns, so no copy of it is
+            # made before but for what from_numpy does not take as it is
+            if a.flags.writeable and a.flags.c_contiguous and self.device.type != "cpu":
+                return torch.from_numpy(a).to(self.device)
+            return torch.from_numpy(a.copy()).to(self.device)
+
+        self.lon, self.lat, self.species = upload(self.lon0), upload(self.lat0), upload(self.species0)
         self.step = 0          # global step index: keys the uniforms
         self.clock_steps = 0   # steps since the field's first time level
         self.oob.zero_()

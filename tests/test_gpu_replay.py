@@ -39,3 +39,31 @@ def test_component_classes(gpu, n):
     st, wide = up.component_stats(), [p for p in npairs if p > 32]
     assert st.components == len(sizes) and st.pairs == len(arr) and st.max_pairs == max(npairs)
     assert st.wide_components == len(wide) and st.wide_pairs == sum(wide)
+
+
+@pytest.mark.parametrize("form", ["plain", "read-only", "strided", "reversed"])
+def test_reset_takes_any_array(gpu, form):
+    from lagrangian_microbes_amd import FusedRunner, VelocityField
+    rng = np.random.default_rng(4)
+    lon, lat = 200.0 + rng.random(300), 20.0 + rng.random(300)
+    species = rng.integers(1, 4, 300).astype(np.int8)
+    host = [lon, lat, species]
+    if form == "strided":
+        host = [np.repeat(a, 2)[::2] for a in host]
+    elif form == "reversed":
+        host = [a[::-1].copy()[::-1] for a in host]
+    elif form == "read-only":
+        for a in host:
+            a.flags.writeable = False
+    f = VelocityField(np.array([199.0, 202.0]), np.array([19.0, 22.0]), np.zeros((1, 2, 2)), np.zeros((1, 2, 2)), None)
+    r = FusedRunner(*host, f, 0.01, {"pRS": 0.5, "pPR": 0.5, "pSP": 0.5}, (1, 0), 3600.0, chunk=2)
+    for got, want in zip((r.lon, r.lat, r.species), (lon, lat, species)):
+        assert np.array_equal(got.cpu().numpy(), want)
+    if form == "plain":  # what the arrays hold at the reset counts, and only then
+        before = lon.copy()
+        lon += 0.25
+        assert np.array_equal(r.lon.cpu().numpy(), before)
+        r.reset()
+        assert np.array_equal(r.lon.cpu().numpy(), lon)
+    r.run(2)
+    assert r.step == 2
