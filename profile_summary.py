@@ -51,6 +51,7 @@ TIMER_NAMES = {
     "pair_emit_kernel": "pair_emit", "radix_hist_kernel": "sort_hist", "radix_scatter_kernel": "sort_scatter",
     "scan_reduce_kernel": "scan_reduce", "scan_apply_kernel": "scan_apply", "rps_init_kernel": "rps_init",
     "rps_tile_union_kernel": "rps_tile",
+    "traj_loss_kernel": "traj_loss", "traj_loss_sum_kernel": "traj_loss", "traj_scale_kernel": "traj_loss",
     "rps_union_kernel": "rps_union", "rps_keys_kernel": "rps_keys", "rps_group_blk_kernel": "rps_group",
     "rps_comps_kernel": "rps_comps", "rps_fill_kernel": "rps_fill", "rps_links_kernel": "rps_links",
     "rps_play_kernel": "rps_play", "copy16_kernel": "copy16",
