@@ -133,8 +133,9 @@ class FusedRunner:
         Three streams, three sets of chunk buffers (set c % 3 for chunk c):
         the advection of chunk c + 2 (FP64 arithmetic) runs on its own stream
         beside the pair search and grouping of chunk c + 1 (memory-latency
-        bound) on a side stream, while chunk c replays the species on the
-        caller's stream.  The advection of a chunk waits for the replay that
+        bound) on a side stream, while chunk c replays the species on a
+        stream of its own (a small population's on the caller's), which the
+        caller's waits for before the callback.  The advection of a chunk waits for the replay that
         last used its set; the grouping waits for its advection.  After each
         chunk, ``on_chunk(k, rec_x, rec_y, rec_s, npairs)`` receives that
         chunk's records (device views, valid until the callback returns; if
