@@ -64,9 +64,9 @@ constexpr uint32_t kUnset = 0xffffffffu;
 // (about 100 ns each); a larger one takes a wavefront.  Up to kFewParticles
 // particles the limit is 16: a step's replay then waits for its longest serial
 // chain, and the components between the limits find wavefronts free.  124,000
-// particles, 60 steps: 1,748 us with 32, 1,572 with 16; 30,000: 990 and 880;
-// but 242,000 dense ones, 100 steps: 6.50 and 6.74 ms, and 4,000,000, 96
-// steps: 81.9 and 87.2 ms, where these components are thousands.
+// particles, 60 steps: 1,748 us with 32, 1,572 with 16; but 242,000 dense
+// ones, 100 steps: 6.54 and 6.74 ms, and 4,000,000, 96 steps: 81.9 and 87.2
+// ms, where these components are thousands.
 constexpr uint32_t kNarrowPairs = 32, kNarrowPairsFew = 16;
 constexpr int64_t kFewParticles = 1 << 17;
 constexpr uint32_t kNarrowSlots = kNarrowPairs + 1;  // a component of P pairs has <= P + 1 particles
