@@ -197,8 +197,12 @@ class TrajectoryLoss(torch.autograd.Function):
             if any(t._version != v for t, v in zip(inputs, ctx.versions)):
                 raise RuntimeError("a position or target of trajectory_loss was modified by an inplace operation "
                                    "before its gradient was differentiated")
-            loss = _mean_great_circle_sq(*inputs)
-            wanted = [t for t, w in zip(inputs, need) if w]
+            # by views of the arguments, a node of its own for each: an argument
+            # that another one is made from, or that is passed twice, gets its
+            # partial derivative, and the hooks on it wait for the caller's pass
+            views = [t.view_as(t) for t in inputs]
+            loss = _mean_great_circle_sq(*views)
+            wanted = [t for t, w in zip(views, need) if w]
             got = iter(torch.autograd.grad(loss, wanted, by, create_graph=True))
             return tuple(next(got) if w else None for w in need)
         n = inputs[0].numel()

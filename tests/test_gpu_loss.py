@@ -43,6 +43,43 @@ def test_second_derivatives(gpu):
         torch.testing.assert_close(a, b, rtol=1e-12, atol=0.0, equal_nan=True)
 
 
+def related_arguments(how, lon, lat, lon_t, lat_t):
+    """Leaves, and the arguments made from them."""
+    if how == "displacement":  # a trajectory's end against its own start: the start's gradient is zero
+        return [lon, lat, lon_t, lat_t], lambda x, y, s, t: (x + s, y + t, x, y)
+    if how == "chained":
+        return [lon, lat, lat_t], lambda x, y, t: (x, y, 1.5 * x - 99.0, t)
+    if how == "repeated":
+        return [lon, lat, lon_t], lambda x, y, t: (x, y, t, y)
+    assert how == "hook"
+    def args(x, y, s, t):
+        out = (x * 1.0, y, s, t * 1.0)
+        out[0].register_hook(lambda g: 10.0 * g)
+        out[3].register_hook(lambda g: g - 1.0)
+        return out
+    return [lon, lat, lon_t, lat_t], args
+
+
+@pytest.mark.parametrize("how", ["displacement", "chained", "repeated", "hook"])
+def test_arguments_that_share_a_graph(gpu, how):
+    # bounds: the roundings of a term's gradient (test_loss_and_gradients), where terms cancel
+    # relative to the gradients that cancel
+    leaves, args = related_arguments(how, *(t.detach() for t in inputs(60, 11, (0, 0, 0, 0))))
+    if how == "displacement":
+        leaves[2], leaves[3] = leaves[2] * 1e-3, leaves[3] * 1e-3
+    leaves = [t.requires_grad_() for t in leaves]
+    got = []
+    for f in (adjoint.trajectory_loss, adjoint._mean_great_circle_sq):
+        plain = torch.autograd.grad(f(*args(*leaves)), leaves)
+        first = torch.autograd.grad(f(*args(*leaves)), leaves, create_graph=True)
+        second = torch.autograd.grad(sum((v[1:] ** 2).sum() for v in first), leaves, allow_unused=True)
+        got.append((*plain, *first, *(torch.zeros_like(t) if g is None else g for g, t in zip(second, leaves))))
+    scale = [max(float(v[1:].abs().max()) for v in got[1][k:k + len(leaves)]) for k in (0, 0, 2 * len(leaves))]
+    for k, (a, b) in enumerate(zip(*got)):
+        torch.testing.assert_close(a[1:], b[1:], rtol=1e-11, atol=1e-12 * scale[k // len(leaves)])
+        torch.testing.assert_close(a[:1].isnan(), b[:1].isnan())
+
+
 def test_other_calls_take_the_single_operations(gpu):
     lon, lat, lon_t, lat_t = (t.detach() for t in inputs(40, 5, (0, 0, 0, 0)))
     ref = adjoint._mean_great_circle_sq(lon, lat, lon_t, lat_t)
