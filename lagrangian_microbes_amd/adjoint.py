@@ -167,52 +167,47 @@ def _mean_great_circle_sq(lon, lat, lon_t, lat_t):
     return great_circle_sq(lon, lat, lon_t, lat_t, radius=SPHERE_RADIUS_M / 1e3).mean()
 
 
+def _loss_and_gradients(n, rows, grad, device):
+    """The loss of n positions and targets at four addresses (float64) and,
+    unless grad is None, its gradients to them, [4, n] (lm_trajectory_loss)."""
+    partial = torch.empty(_lib.LOSS_PARTIALS, dtype=torch.float64, device=device)
+    loss = torch.empty((), dtype=torch.float64, device=device)
+    check(_lib.load().lm_trajectory_loss(n, *rows, SPHERE_RADIUS_M / 1e3, 0 if grad is None else 4, ptr(grad),
+                                         ptr(partial), ptr(loss), stream_ptr()))
+    return loss
+
+
 class TrajectoryLoss(torch.autograd.Function):
-    """trajectory_loss of contiguous float64 GPU tensors of one shape, with its
-    gradients from the same pass (lm_trajectory_loss)."""
+    """trajectory_loss of the rows of a [4, ...] tensor, with its gradients from
+    the same pass.
+
+    The four arguments come stacked: the node then owns what it differentiates
+    again, so the arguments may be changed in place or freed before the
+    backward, as under the single operations, and each has an edge of its own
+    whatever else it is made from or used as.  What it keeps is saved as any
+    operation saves it: seen by saved-tensor hooks, freed by the backward."""
 
     @staticmethod
-    def forward(ctx, lon, lat, lon_t, lat_t):
-        need = ctx.needs_input_grad
-        ngrad = 4 if need[2] or need[3] else 2 if need[0] or need[1] else 0
-        n = lon.numel()
-        # one block: the loss, the scratch sums and the gradients
-        buf = torch.empty(1 + _lib.LOSS_PARTIALS + ngrad * n, dtype=torch.float64, device=lon.device)
-        grad = buf[1 + _lib.LOSS_PARTIALS:]
-        loss = torch.empty((), dtype=torch.float64, device=lon.device)
-        check(_lib.load().lm_trajectory_loss(n, ptr(lon), ptr(lat), ptr(lon_t), ptr(lat_t), SPHERE_RADIUS_M / 1e3, ngrad,
-                                             ptr(grad), ptr(buf[1:]), ptr(loss), stream_ptr()))
-        ctx.save_for_backward(grad)
-        # the inputs serve a second differentiation only: they may be changed
-        # in place before the backward, as under the single operations
-        ctx.inputs = (lon, lat, lon_t, lat_t)
-        ctx.versions = tuple(t._version for t in ctx.inputs)
+    def forward(ctx, packed):
+        n, at, grad = packed.numel() // 4, packed.data_ptr(), torch.empty_like(packed)
+        loss = _loss_and_gradients(n, [at + 8 * k * n for k in range(4)], grad, packed.device)
+        ctx.save_for_backward(packed, grad)
         return loss
 
     @staticmethod
     def backward(ctx, by):
-        grad, = ctx.saved_tensors
-        inputs, need = ctx.inputs, ctx.needs_input_grad
+        packed, grad = ctx.saved_tensors
         if torch.is_grad_enabled():  # a gradient that is to be differentiated again
-            if any(t._version != v for t, v in zip(inputs, ctx.versions)):
-                raise RuntimeError("a position or target of trajectory_loss was modified by an inplace operation "
-                                   "before its gradient was differentiated")
-            # by views of the arguments, a node of its own for each: an argument
-            # that another one is made from, or that is passed twice, gets its
-            # partial derivative, and the hooks on it wait for the caller's pass
-            views = [t.view_as(t) for t in inputs]
-            loss = _mean_great_circle_sq(*views)
-            wanted = [t for t, w in zip(views, need) if w]
-            got = iter(torch.autograd.grad(loss, wanted, by, create_graph=True))
-            return tuple(next(got) if w else None for w in need)
-        n = inputs[0].numel()
-        if _watched() or type(by) is not torch.Tensor or not torch._C._has_storage(by):
-            out = grad * by  # a batch of gradients (vectorised Jacobians), or a mode that has to see the operation
-        else:
-            out = torch.empty_like(grad)
-            by = by.to(torch.float64).contiguous()
-            check(_lib.load().lm_scale_by(out.numel(), ptr(grad), ptr(by), ptr(out), stream_ptr()))
-        return tuple(out[k * n:(k + 1) * n].view(inputs[0].shape) if w else None for k, w in enumerate(need))
+            return torch.autograd.grad(_mean_great_circle_sq(*packed), packed, by, create_graph=True)[0]
+        if (_watched() or type(by) is not torch.Tensor or not torch._C._has_storage(by) or _dual(by)
+                or grad.dtype != torch.float64 or not grad.is_contiguous() or grad.device != by.device):
+            # a batch of gradients (vectorised Jacobians), a mode that has to see
+            # the operation, or what a hook made of the saved gradients
+            return grad * by
+        out = torch.empty_like(grad)
+        by = by.to(torch.float64).contiguous()
+        check(_lib.load().lm_scale_by(out.numel(), ptr(grad), ptr(by), ptr(out), stream_ptr()))
+        return out
 
 
 def _watched():
@@ -220,6 +215,11 @@ def _watched():
     return (torch.compiler.is_compiling() or torch.jit.is_tracing()
             or torch._C._functorch.peek_interpreter_stack() is not None
             or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0)
+
+
+def _dual(t):
+    """Whether t carries a forward-mode tangent."""
+    return torch.autograd.forward_ad._current_level >= 0 and torch.autograd.forward_ad.unpack_dual(t).tangent is not None
 
 
 def _plain_f64(tensors):
@@ -232,18 +232,17 @@ def _plain_f64(tensors):
         return False
     if t0.device.type != "cuda" or t0.device.index != torch.cuda.current_device() or t0.numel() == 0:
         return False
-    if _watched():
-        return False
-    return not any(torch.autograd.forward_ad.unpack_dual(t).tangent is not None for t in tensors) \
-        if torch.autograd.forward_ad._current_level >= 0 else True
+    return not _watched() and not any(_dual(t) for t in tensors)
 
 
 def trajectory_loss(lon, lat, lon_t, lat_t):
     """Mean squared great-circle distance to the targets, in km^2."""
     args = (lon, lat, lon_t, lat_t)
-    if all(isinstance(t, torch.Tensor) for t in args) and _plain_f64(args):
-        return TrajectoryLoss.apply(*args)
-    return _mean_great_circle_sq(*args)
+    if not (all(isinstance(t, torch.Tensor) for t in args) and _plain_f64(args)):
+        return _mean_great_circle_sq(*args)
+    if torch.is_grad_enabled() and any(t.requires_grad for t in args):
+        return TrajectoryLoss.apply(torch.stack(args))
+    return _loss_and_gradients(lon.numel(), [ptr(t) for t in args], None, lon.device)
 
 
 def interact_final(lon, lat, species, radius, params, key, step, bbox, norm=2.0):

@@ -1,4 +1,6 @@
 """The one-pass trajectory loss against the single torch operations it stands for."""
+import weakref
+
 import pytest
 import torch
 
@@ -78,6 +80,48 @@ def test_arguments_that_share_a_graph(gpu, how):
     for k, (a, b) in enumerate(zip(*got)):
         torch.testing.assert_close(a[1:], b[1:], rtol=1e-11, atol=1e-12 * scale[k // len(leaves)])
         torch.testing.assert_close(a[:1].isnan(), b[:1].isnan())
+
+
+def test_arguments_changed_in_place_before_a_second_differentiation(gpu):
+    got = []
+    for f in (adjoint.trajectory_loss, adjoint._mean_great_circle_sq):
+        leaves = inputs(50, 13, (1, 1, 1, 0))
+        args = [leaves[0] * 1.0, leaves[1] * 1.0, leaves[2] * 1.0, leaves[3]]
+        loss = f(*args)
+        with torch.no_grad():
+            for t in args:
+                t.add_(1.0)
+        first = torch.autograd.grad(loss, leaves[:3], create_graph=True)
+        got.append((*first, *torch.autograd.grad(sum((v[1:] ** 2).sum() for v in first), leaves[:3])))
+    for a, b in zip(*got):
+        # rtol: as in test_second_derivatives; atol: entries that cancel to near zero
+        torch.testing.assert_close(a[1:], b[1:], rtol=1e-12, atol=1e-16 * float(b[1:].abs().max()))
+
+
+def test_what_the_loss_keeps(gpu):
+    n = 1 << 20
+    base = inputs(n, 17, (0, 0, 0, 0))
+    x = [t.detach().requires_grad_() for t in base]
+    ref = torch.autograd.grad(adjoint._mean_great_circle_sq(*x), x)
+    # after the backward the loss holds no argument
+    args = [t * 1.0 for t in x]
+    kept = [weakref.ref(t) for t in args]
+    loss = adjoint.trajectory_loss(*args)
+    loss.backward()
+    del args
+    assert all(r() is None for r in kept) and loss.grad_fn is not None
+    # hooks on saved tensors see all of it: with a copy on the host nothing of n entries stays on the GPU
+    before = torch.cuda.memory_allocated()
+    with torch.autograd.graph.save_on_cpu():
+        loss = adjoint.trajectory_loss(*(t * 1.0 for t in x))
+    assert torch.cuda.memory_allocated() - before < 8 * n
+    for a, b in zip(torch.autograd.grad(loss, x), ref):  # (bounds as in test_loss_and_gradients)
+        torch.testing.assert_close(a, b, rtol=1e-12, atol=1e-16 * float(b.abs().max()))
+    # and may give it back in another precision
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t.float(), lambda t: t):
+        loss = adjoint.trajectory_loss(*x)
+    for a, b in zip(torch.autograd.grad(loss, x), ref):
+        torch.testing.assert_close(a, b, rtol=1e-6, atol=1e-7 * float(b.abs().max()))
 
 
 def test_other_calls_take_the_single_operations(gpu):
