@@ -1137,13 +1137,81 @@ constexpr uint32_t kSmallSpecies = 2 * kSmallWindow;
 constexpr uint32_t kSmallNone = kSmallWindow;
 static_assert(kSmallMax <= 1 << 14 && kSmallSpecies + kSmallMax <= 1 << 16 && kSmallNone < 1 << 14, "record fields");
 
+// The pairs at a particle as their j come from its list.  While no list holds
+// more than kSmallScan pairs, they are filled in any order and a pair's
+// neighbours are found by reading the whole list.  That is quadratic in a list,
+// so a step with a longer one has all of them filled in order, which keeps the
+// work linear in the pairs but for a search at the ends of a row: a crowd of
+// 1,000 particles in one radius (500,000 pairs) 144 -> 2.9 ms, 12,287 pairs
+// with one j 17.3 ms -> 77 us.  12,288 particles with one partner above each:
+// 67 us in any order, 81 in order; with four (lists up to 16 or so) 296 and
+// 261.
+constexpr uint32_t kSmallScan = 16;
+constexpr int kSmallRounds = 4;
+
+// list = the pairs by j, each j's in order from its cursor ends[j] on, which
+// ends at the list's end; rec[k].x = pair k's place.  A wavefront ranks its
+// kSmallRounds x 64 consecutive pairs among those of the same j (a ballot per
+// bit of j); then the wavefronts read and advance the cursors in turn.
+__device__ void small_place_in_order(uint32_t n, uint32_t P, const int32_t* __restrict__ pi,
+                                     const int32_t* __restrict__ pj, uint32_t* ends, uint32_t* __restrict__ list,
+                                     uint2* __restrict__ rec) {
+    constexpr uint32_t R = kSmallRounds, kWaves = kSmallBlock / 64;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const unsigned long long below = (1ull << lane) - 1ull;
+    for (uint32_t c0 = 0; c0 < P; c0 += kSmallBlock * R) {  // uniform over the workgroup
+        const uint32_t w0 = c0 + 64u * R * wave;
+        uint32_t j[R], rank[R], tot[R], start[R];
+#pragma unroll
+        for (uint32_t r = 0; r < R; ++r) {
+            const uint32_t k = w0 + 64u * r + lane;
+            const uint32_t a = k < P ? (uint32_t)pi[k] : kUnset, b = k < P ? (uint32_t)pj[k] : kUnset;
+            j[r] = a < n && b < n && b != a ? b : kUnset;
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < R; ++r) {
+            const bool valid = j[r] != kUnset;
+            unsigned long long m = __ballot(valid);
+#pragma unroll
+            for (uint32_t bit = 0; (kSmallMax - 1) >> bit != 0; ++bit) {
+                const bool on = (j[r] >> bit) & 1u;
+                const unsigned long long bm = __ballot(valid && on);
+                m &= on ? bm : ~bm;
+            }
+            rank[r] = (uint32_t)__popcll(m & below);
+            tot[r] = (uint32_t)__popcll(m);
+        }
+        for (uint32_t w = 0; w < kWaves; ++w) {
+            if (wave == w) {
+#pragma unroll
+                for (uint32_t r = 0; r < R; ++r) {
+                    const bool valid = j[r] != kUnset;
+                    start[r] = valid ? ends[j[r]] : 0u;
+                    // every lane has read the cursor before its first one advances it
+                    // (the wavefront's LDS operations complete in program order)
+                    if (valid && rank[r] == 0u) ends[j[r]] = start[r] + tot[r];
+                    __builtin_amdgcn_wave_barrier();
+                }
+            }
+            __syncthreads();
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < R; ++r) {
+            if (j[r] == kUnset) continue;
+            const uint32_t k = w0 + 64u * r + lane, at = start[r] + rank[r];
+            list[at] = k;
+            rec[k].x = at;
+        }
+    }
+}
+
 __global__ void __launch_bounds__(kSmallBlock)
 rps_small_kernel(uint32_t n, const int32_t* __restrict__ pi_all, const int32_t* __restrict__ pj_all,
                  const int64_t* __restrict__ npairs, RpsArrays A, RpsStrides st, double pRS, double pPR, double pSP,
                  uint64_t k0, uint64_t k1, uint64_t step0) {
     __shared__ uint32_t ends[kSmallMax];                   // counts, then ends of the lists of pairs by j
     __shared__ uint32_t rbeg[kSmallMax], rend[kSmallMax];  // rows: the pairs by i
-    __shared__ uint32_t scan_lds[kSmallBlock / 64];
+    __shared__ uint32_t scan_lds[kSmallBlock / 64], longest;
     const int64_t s = blockIdx.x, po = s * st.pair;
     const uint32_t t = threadIdx.x;
     const int64_t P64 = step_pairs(npairs, s, st.pair);
@@ -1153,20 +1221,28 @@ rps_small_kernel(uint32_t n, const int32_t* __restrict__ pi_all, const int32_t* 
     const int32_t* pj = pj_all + po;
     uint32_t* list = A.list + po;
     for (uint32_t v = t; v < n; v += kSmallBlock) ends[v] = rbeg[v] = rend[v] = 0u;
+    if (t == 0) longest = 0u;
     __syncthreads();
+    uint32_t most = 0u;
     for (uint32_t k = t; k < P; k += kSmallBlock) {
         const uint32_t a = (uint32_t)pi[k], b = (uint32_t)pj[k];
         const uint32_t before = (uint32_t)pi[k > 0 ? k - 1 : 0], after = (uint32_t)pi[k + 1 < P ? k + 1 : k];
         if (a >= n) continue;
         if (k == 0 || before != a) rbeg[a] = k;
         if (k + 1 == P || after != a) rend[a] = k + 1;
-        if (b < n && b != a) atomicAdd(&ends[b], 1u);
+        if (b < n && b != a) most = max(most, atomicAdd(&ends[b], 1u) + 1u);
     }
+    if (most > kSmallScan) atomicMax(&longest, most);
     __syncthreads();
     small_scan_array(ends, n, scan_lds);
-    for (uint32_t k = t; k < P; k += kSmallBlock) {
-        const uint32_t a = (uint32_t)pi[k], b = (uint32_t)pj[k];
-        if (a < n && b < n && b != a) list[atomicAdd(&ends[b], 1u)] = k;  // the cursor ends at the list's end
+    const bool ordered = longest > kSmallScan;  // uniform
+    if (!ordered) {
+        for (uint32_t k = t; k < P; k += kSmallBlock) {
+            const uint32_t a = (uint32_t)pi[k], b = (uint32_t)pj[k];
+            if (a < n && b < n && b != a) list[atomicAdd(&ends[b], 1u)] = k;  // the cursor ends at the list's end
+        }
+    } else {
+        small_place_in_order(n, P, pi, pj, ends, list, A.rec + po);
     }
     __threadfence_block();
     __syncthreads();
@@ -1174,13 +1250,31 @@ rps_small_kernel(uint32_t n, const int32_t* __restrict__ pi_all, const int32_t* 
     // of those whose j is v
     auto around = [&](uint32_t v, uint32_t k, uint32_t* prev, uint32_t* next) {
         uint32_t lo = kUnset, hi = kUnset;
-        for (uint32_t q = v > 0 ? ends[v - 1] : 0u; q < ends[v]; ++q) {
-            const uint32_t e = list[q];
-            if (e < k) lo = lo == kUnset ? e : max(lo, e);
-            else if (e > k) hi = min(hi, e);
+        const uint32_t q0 = v > 0 ? ends[v - 1] : 0u, q1 = ends[v];
+        if (!ordered) {
+            for (uint32_t q = q0; q < q1; ++q) {
+                const uint32_t e = list[q];
+                if (e < k) lo = lo == kUnset ? e : max(lo, e);
+                else if (e > k) hi = min(hi, e);
+            }
+        } else {
+            uint32_t b0 = q0, b1 = q1;  // the first entry above k
+            while (b0 < b1) {
+                const uint32_t mid = (b0 + b1) >> 1;
+                if (list[mid] < k) b0 = mid + 1u;
+                else b1 = mid;
+            }
+            if (b0 > q0) lo = list[b0 - 1u];
+            if (b0 < q1) hi = list[b0];
         }
         *prev = lo == kUnset ? kUnset : 2u * lo + 1u;
         *next = hi == kUnset ? kUnset : 2u * hi + 1u;
+    };
+    // the same at k's own j, b, in an ordered list: the entries beside k's
+    auto beside = [&](uint32_t b, uint32_t k, uint32_t* prev, uint32_t* next) {
+        const uint32_t at = A.rec[po + k].x;
+        *prev = at > (b > 0 ? ends[b - 1] : 0u) ? 2u * list[at - 1u] + 1u : kUnset;
+        *next = at + 1u < ends[b] ? 2u * list[at + 1u] + 1u : kUnset;
     };
     auto source = [&](uint32_t prev, uint32_t k, uint32_t v) {
         const bool here = prev != kUnset && (prev >> 1) / kSmallWindow == k / kSmallWindow;
@@ -1198,14 +1292,15 @@ rps_small_kernel(uint32_t n, const int32_t* __restrict__ pi_all, const int32_t* 
             const double u = u01_from_u64(philox4x64_10(k, step0 + (uint64_t)s, kStreamPairs, 0, k0, k1).v[0]);
             const uint32_t bits = (u < pRS ? 1u : 0u) | (u < pPR ? 2u : 0u) | (u < pSP ? 4u : 0u);
             const bool two = b < n && b != a;
-            uint32_t prev, next;
-            around(a, k, &prev, &next);
+            uint32_t prev = kUnset, next = kUnset;
+            if (!ordered || k <= rbeg[a] || k + 1u >= rend[a]) around(a, k, &prev, &next);
             if (k > rbeg[a]) prev = 2u * (k - 1u);  // i's row is one run of pairs
             if (k + 1u < rend[a]) next = 2u * (k + 1u);
             r.x = source(prev, k, a);
             r.y = after_it(next, k) | bits << 28;
             if (two) {
-                around(b, k, &prev, &next);
+                if (ordered) beside(b, k, &prev, &next);
+                else around(b, k, &prev, &next);
                 if (rend[b] > rbeg[b]) {  // j's own row, all of it before or after k
                     if (rend[b] <= k && (prev == kUnset || 2u * (rend[b] - 1u) > prev)) prev = 2u * (rend[b] - 1u);
                     if (rbeg[b] > k && (next == kUnset || 2u * rbeg[b] < next)) next = 2u * rbeg[b];

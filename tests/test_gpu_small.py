@@ -80,6 +80,59 @@ def test_rps_pairs_in_any_direction(gpu, n):
     assert np.array_equal(g, ref)
 
 
+def crowded(kind, n, rng):
+    """Sorted pair lists with many pairs of one j."""
+    ids = np.arange(n)
+    if kind == "hub last":
+        pairs = [(k, n - 1) for k in range(n - 1)]
+    elif kind == "hub between":  # its pairs have it as i, as j, and as j below i
+        h = n // 2
+        pairs = [(k, h) for k in range(n) if k != h] + [(h, k) for k in range(0, n, 3) if k != h]
+    elif kind == "crowd":
+        m = np.sort(rng.permutation(n)[:n // 8])
+        pairs = np.stack([m[a] for a in np.triu_indices(len(m), 1)], 1)
+    elif kind == "lists of 16":
+        pairs = [(k, j) for j in range(16, n, 16) for k in range(j - 16, j)]
+    else:
+        assert kind == "one list of 17"
+        pairs = [(k, j) for j in range(16, n, 16) for k in range(j - 16, j)] + [(0, 32)]
+    return np.unique(np.array(pairs, dtype=np.int32), axis=0)
+
+
+@pytest.mark.parametrize("n", [66, 2500, 12288])
+@pytest.mark.parametrize("kind", ["hub last", "hub between", "crowd", "lists of 16", "one list of 17"])
+def test_rps_many_pairs_of_one_j(gpu, kind, n):
+    rng = np.random.default_rng(n)
+    arr = crowded(kind, n, rng)
+    sp = rng.integers(0, 5, n).astype(np.int8)
+    args = (0.5, 0.6, 0.4, (n, 2), 5)
+    g, _ = gpu_rps(sp, arr[:, 0], arr[:, 1], *args)
+    assert np.array_equal(g, oracle.rps_sequential(sp, arr[:, 0], arr[:, 1], *args))
+
+
+def prepare_us(n, arr):
+    pi, pj = T(arr[None, :, 0].copy()), T(arr[None, :, 1].copy())
+    count, up, best = T(np.array([len(arr)])), dev.RPSUpdater(n), np.inf
+    for _ in range(4):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        up.prepare(n, pi, pj, count, 0.5, 0.5, 0.5, (1, 2), 0)
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, 1e3 * a.elapsed_time(b))
+    return best
+
+
+def test_prepare_is_linear_in_the_pairs(gpu):
+    # wide bounds: quadratic lists took 360 times the hub with the lowest index, and 40 times the
+    # general kernels on the crowd
+    n, rng = 12288, np.random.default_rng(1)
+    first = np.array([(0, k) for k in range(1, n)], dtype=np.int32)
+    assert prepare_us(n, crowded("hub last", n, rng)) < 20 * prepare_us(n, first)
+    crowd = crowded("crowd", 8 * 1000, rng)
+    assert prepare_us(n, crowd) < 8 * prepare_us(n + 1, crowd)
+
+
 @pytest.mark.parametrize("n,out", [(9001, 9001), (9000, 9016), (15000, 15000)])
 def test_play_steps_matches_single_steps(gpu, n, out):
     rng = np.random.default_rng(n)
