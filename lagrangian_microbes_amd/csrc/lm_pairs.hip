@@ -493,15 +493,31 @@ pair_emit_kernel(int64_t n, const float* __restrict__ x_all, const float* __rest
 //          and searching its own 1024 / LPP particles, LPP lanes each (with
 //          4, three lanes take a stencil row each): partners above each
 //          particle, counted, the first kSmallNbr kept
-//   emit   every workgroup sums the counts before its 1024 rows, scans its
-//          own and writes them sorted; a row of more than kSmallNbr partners
-//          is found again by its wavefront, 64 particles at a time in index
-//          order
+//   emit   every workgroup sums the counts before its ROWS rows, scans its
+//          own and writes them sorted; its rows of more than kSmallNbr
+//          partners are found again by a wavefront each, from the bucket order
+//          that the count left in memory, or, with hundreds of partners,
+//          among all particles in index order
 // The cells wrap onto a torus of 2^LWX x 2^LWY buckets (a stencil's nine cells
 // always fall into nine buckets: the sides are at least 64; cells further
 // apart may share one, and the distance test drops what the stencil does not
 // reach), so the table fits LDS whatever the box.
 constexpr int kSmallNbr = 16;  // 16-bit partners kept per particle, in the bytes of kNbr 32-bit ones
+constexpr int kSmallTab = (1 << 13) + 4;  // bucket table entries per step in memory (>= 2^(LWX + LWY) + 1)
+
+// A crowded row's partners are gathered from its buckets and ranked against
+// each other (the work grows with their square) up to 128 + n / 48 of them, and
+// found among all particles in index order (the work grows with n, and there
+// is nothing to rank) above.  2,500 particles with a mean of 150 partners: 514
+// us with the line at 512, 294 at 180; 12,288 with 200: 899 at 384, 1,042 at 256.
+constexpr uint32_t kSmallGather = 128 + (uint32_t)kSmallMax / 48;
+
+__device__ __forceinline__ uint32_t lane_of(uint32_t v, int lane) {  // lane: uniform
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, lane);
+}
+__device__ __forceinline__ float lane_of(float v, int lane) {
+    return __uint_as_float(lane_of(__float_as_uint(v), lane));
+}
 
 template <int LWX, int LWY, typename F>
 __device__ __forceinline__ void small_row(const uint32_t* start, const CellGrid& g, int cx, int row, F&& visit) {
@@ -522,13 +538,14 @@ __device__ __forceinline__ void small_row(const uint32_t* start, const CellGrid&
 template <int KIND, int NMAX, int LWX, int LWY, int LPP>
 __global__ void __launch_bounds__(kSmallBlock)
 pair_small_count_kernel(int n, const float* __restrict__ x_all, const float* __restrict__ y_all, CellGrid g, Metric m,
-                        Strides st, uint32_t* __restrict__ cnt_all, uint16_t* __restrict__ nbr_all) {
+                        Strides st, uint32_t* __restrict__ cnt_all, uint16_t* __restrict__ nbr_all,
+                        uint32_t* __restrict__ tab_all, uint32_t* __restrict__ order_all) {
     constexpr int kItems = NMAX / kSmallBlock;
     constexpr uint32_t T = 1u << (LWX + LWY);
     static_assert(NMAX % kSmallBlock == 0 && NMAX <= 65536, "16-bit indices, whole items");
     static_assert(LPP == 1 || LPP == 4, "a lane per particle, or one per stencil row");
     __shared__ float2 pos[NMAX];  // in bucket order
-    __shared__ uint16_t idx[NMAX];
+    __shared__ __align__(4) uint16_t idx[NMAX];
     __shared__ uint32_t start[T + 1];
     __shared__ uint32_t scan_lds[kSmallBlock / 64];
     const int64_t s = blockIdx.y;
@@ -568,6 +585,11 @@ pair_small_count_kernel(int n, const float* __restrict__ x_all, const float* __r
         }
     }
     __syncthreads();
+    if (blockIdx.x == 0) {  // for the rows that the emit finds again
+        for (uint32_t b = t; b <= T; b += kSmallBlock) tab_all[s * kSmallTab + b] = start[b];
+        for (int k = t; k < (n + 1) / 2; k += kSmallBlock)
+            order_all[s * st.rec + k] = reinterpret_cast<const uint32_t*>(idx)[k];
+    }
     const int i = (int)blockIdx.x * (kSmallBlock / LPP) + t / LPP, sub = t % LPP;
     if (i >= n) return;  // all lanes of a particle
     const float xi = x[i], yi = y[i];
@@ -592,40 +614,104 @@ pair_small_count_kernel(int n, const float* __restrict__ x_all, const float* __r
         all = __shfl(at + c, 2, 4);
     }
     if (sub == 0) cnt_all[s * st.row + i] = all;
-    if (c == 0) return;
+    if (c == 0 || all > (uint32_t)kSmallNbr) return;
     uint16_t* row = nbr_all + 2 * s * st.nbr + (int64_t)i * kSmallNbr;
     search([&](uint32_t k) {
         const float2 o = pos[k];
         if (pair_hit<KIND>(m, (int)idx[k] > i, xi, yi, o.x, o.y)) {
-            if (at < (uint32_t)kSmallNbr) row[at] = idx[k];
+            row[at] = idx[k];
             ++at;
         }
     });
 }
 
+// LDS accesses of a wavefront's lanes before and after keep their order: the
+// hardware's is that of the instructions, which the fence makes the compiler keep.
+__device__ __forceinline__ void wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// One crowded row by a wavefront, from its buckets: rc <= kSmallGather partners
+// (found: kSmallGather 16-bit slots of LDS), written sorted to [at, at + rc).
+// from[0 .. 6), len: the row's candidates, as ranges of the bucket order.
 template <int KIND>
+__device__ __forceinline__ void small_gather_row(int n, const float* __restrict__ x, const float* __restrict__ y,
+                                                 const Metric& m, const uint16_t* __restrict__ order, int r, float xr,
+                                                 float yr, const uint32_t (&from)[6], const uint32_t (&len)[6],
+                                                 uint32_t rc, uint32_t at, uint16_t* found, int32_t* __restrict__ pair_i,
+                                                 int32_t* __restrict__ pair_j) {
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t total = 0;
+#pragma unroll
+    for (int q = 0; q < 6; ++q) total += len[q];
+    uint32_t have = 0;
+    for (uint32_t c0 = 0; c0 < total; c0 += 64) {
+        uint32_t c = c0 + lane, k = 0;
+        const bool cand = c < total;
+#pragma unroll
+        for (int q = 0; q < 6; ++q) {  // the range that holds candidate c
+            k = c < len[q] ? from[q] + c : k;
+            c = c < len[q] ? 0xffffffffu : c - len[q];
+        }
+        const int j = cand ? (int)order[k] : 0;
+        const bool hit = pair_hit<KIND>(m, cand && j > r && j < n, xr, yr, x[j], y[j]);
+        const uint64_t hits = __ballot(hit);
+        const uint32_t slot = have + (uint32_t)__popcll(hits & ((1ull << lane) - 1ull));
+        if (hit && slot < rc) found[slot] = (uint16_t)j;
+        have += (uint32_t)__popcll(hits);
+    }
+    have = min(have, rc);
+    // the slots after the last one, read eight at a time below
+    if (lane < 8 && have + lane < kSmallGather) found[have + lane] = 0xffffu;
+    wave_order();
+    for (uint32_t v0 = 0; v0 < have; v0 += 64) {
+        const bool mine = v0 + lane < have;
+        const uint32_t v = mine ? found[v0 + lane] : 0u;
+        uint32_t rank = 0;
+        for (uint32_t q = 0; q < have; q += 8) {
+            const uint4 o = *reinterpret_cast<const uint4*>(found + q);
+            rank += ((o.x & 0xffffu) < v) + ((o.x >> 16) < v) + ((o.y & 0xffffu) < v) + ((o.y >> 16) < v) +
+                    ((o.z & 0xffffu) < v) + ((o.z >> 16) < v) + ((o.w & 0xffffu) < v) + ((o.w >> 16) < v);
+        }
+        if (mine) {
+            pair_i[at + rank] = r;
+            pair_j[at + rank] = (int32_t)v;
+        }
+    }
+    wave_order();
+}
+
+template <int KIND, int LWX, int LWY, int ROWS>
 __global__ void __launch_bounds__(kSmallBlock)
-pair_small_emit_kernel(int n, const float* __restrict__ x_all, const float* __restrict__ y_all, Metric m, Strides st,
-                       const uint32_t* __restrict__ cnt_all, const uint16_t* __restrict__ nbr_all,
+pair_small_emit_kernel(int n, const float* __restrict__ x_all, const float* __restrict__ y_all, CellGrid g, Metric m,
+                       Strides st, const uint32_t* __restrict__ cnt_all, const uint16_t* __restrict__ nbr_all,
+                       const uint32_t* __restrict__ tab_all, const uint16_t* __restrict__ order_all,
                        int32_t* __restrict__ pair_i_all, int32_t* __restrict__ pair_j_all,
                        int64_t* __restrict__ npairs) {
-    __shared__ uint32_t scan_lds[kSmallBlock / 64];
+    constexpr uint32_t WX = 1u << LWX, WY = 1u << LWY;
+    static_assert((WX << LWY) + 1 <= (uint32_t)kSmallTab, "bucket table");
+    __shared__ uint32_t scan_lds[kSmallBlock / 64], crowded;
+    __shared__ uint32_t who[ROWS], count[ROWS], place[ROWS];  // the crowded rows
+    __shared__ __align__(16) uint16_t found[kSmallBlock / 64][kSmallGather];
     const int64_t s = blockIdx.y;
-    const int t = threadIdx.x, lane = t & 63, i0 = (int)blockIdx.x * kSmallBlock, i = i0 + t;
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6, i0 = (int)blockIdx.x * ROWS, i = i0 + t;
+    const bool own = t < ROWS && i < n;
     const uint32_t* cnt = cnt_all + s * st.row;
-    const uint16_t* row = nbr_all + 2 * s * st.nbr + (int64_t)(i < n ? i : 0) * kSmallNbr;
+    const uint16_t* row = nbr_all + 2 * s * st.nbr + (int64_t)(own ? i : 0) * kSmallNbr;
     // this row's count and partners (read whatever the count) and the counts
     // before and after the workgroup's rows load together
-    uint32_t c = i < n ? cnt[i] : 0u;
+    uint32_t c = own ? cnt[i] : 0u;
     const uint4 lo = reinterpret_cast<const uint4*>(row)[0], hi = reinterpret_cast<const uint4*>(row)[1];
     uint32_t before = 0, after = 0;
 #pragma unroll
     for (int q = 0; q < (int)(kSmallMax / kSmallBlock); ++q) {
         const int k = q * kSmallBlock + t;
-        const uint32_t v = k < n && (k < i0 || k >= i0 + kSmallBlock) ? cnt[k] : 0u;
+        const uint32_t v = k < n && (k < i0 || k >= i0 + ROWS) ? cnt[k] : 0u;
         before += k < i0 ? v : 0u;
         after += k < i0 ? 0u : v;
     }
+    if (t == 0) crowded = 0u;
     uint32_t sum_before, sum_after, sum_own;
     (void)small_exclusive_scan(before, scan_lds, &sum_before);
     (void)small_exclusive_scan(after, scan_lds, &sum_after);
@@ -660,16 +746,58 @@ pair_small_emit_kernel(int n, const float* __restrict__ x_all, const float* __re
                 pair_j[o + k] = (int32_t)v[k];
             }
     }
-    // crowded rows, one after another by the whole wavefront
+    if (c > (uint32_t)kSmallNbr) {
+        const uint32_t q = atomicAdd(&crowded, 1u);
+        who[q] = (uint32_t)i;
+        count[q] = c;
+        place[q] = o;
+    }
+    __syncthreads();
+    // the crowded rows, shared out over the wavefronts: lane q of a wavefront
+    // looks up the buckets of its q-th row
+    static_assert(ROWS <= 64 * (kSmallBlock / 64), "a lane per row of a wavefront");
+    if (crowded == 0u) return;  // uniform
     const float* x = x_all + s * st.pos;
     const float* y = y_all + s * st.pos;
-    for (uint64_t left = __ballot(c > (uint32_t)kSmallNbr); left != 0; left &= left - 1) {
-        const int src = __ffsll((unsigned long long)left) - 1;
-        const int r = __shfl(i, src, 64);
-        const uint32_t rc = __shfl(c, src, 64);
-        uint32_t at = __shfl(o, src, 64);
+    const uint32_t* tab = tab_all + s * kSmallTab;
+    const uint16_t* order = order_all + 2 * s * st.rec;
+    const uint32_t entry = (uint32_t)lane * (kSmallBlock / 64) + (uint32_t)wave, e = min(entry, crowded - 1u);
+    const uint32_t rows = crowded > (uint32_t)wave ? (crowded - (uint32_t)wave + kSmallBlock / 64 - 1) / (kSmallBlock / 64) : 0u;
+    const uint32_t my_r = who[e], my_c = count[e], my_o = place[e];
+    const float my_x = x[my_r], my_y = y[my_r];
+    uint32_t my_from[6], my_len[6];
+    int cx, cy;
+    cell_of(g, my_x, my_y, &cx, &cy);
+    const uint32_t a = (uint32_t)(cx > 0 ? cx - 1 : 0) & (WX - 1u);
+    const uint32_t b = (uint32_t)(cx < g.nx - 1 ? cx + 1 : g.nx - 1) & (WX - 1u);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {  // as small_row
+        const int cr = cy + q - 1;
+        const bool ok = cr >= 0 && cr < g.ny, wraps = a > b;
+        const uint32_t base = ((uint32_t)cr & (WY - 1u)) << LWX;
+        const uint32_t s0 = tab[base + a], e0 = tab[base + (wraps ? WX : b + 1u)];
+        const uint32_t s1 = tab[base], e1 = tab[base + b + 1u];
+        my_from[2 * q] = s0;
+        my_len[2 * q] = ok ? e0 - s0 : 0u;
+        my_from[2 * q + 1] = s1;
+        my_len[2 * q + 1] = ok && wraps ? e1 - s1 : 0u;
+    }
+    for (uint32_t q = 0; q < rows; ++q) {
+        const int r = (int)lane_of(my_r, (int)q);
+        const uint32_t rc = lane_of(my_c, (int)q);
+        uint32_t at = lane_of(my_o, (int)q);
+        const float xr = lane_of(my_x, (int)q), yr = lane_of(my_y, (int)q);
+        if (rc <= 128u + (uint32_t)n / 48u) {
+            uint32_t from[6], len[6];
+#pragma unroll
+            for (int w = 0; w < 6; ++w) {
+                from[w] = lane_of(my_from[w], (int)q);
+                len[w] = lane_of(my_len[w], (int)q);
+            }
+            small_gather_row<KIND>(n, x, y, m, order, r, xr, yr, from, len, rc, at, found[wave], pair_i, pair_j);
+            continue;
+        }
         const uint32_t end = at + rc;
-        const float xr = x[r], yr = y[r];
         for (int j0 = r + 1; j0 < n && at < end; j0 += 64) {
             const int j = j0 + lane;
             const float xj = j < n ? x[j] : 0.0f, yj = j < n ? y[j] : 0.0f;
@@ -710,6 +838,7 @@ struct lm_pairs_ws {
     uint32_t* nbr_cnt = nullptr;   // [steps][row]
     uint32_t* nbr = nullptr;       // [steps][n_max * kNbr]
     uint32_t* row_off = nullptr;   // [steps][row]
+    uint32_t* small_tab = nullptr; // [steps][kSmallTab] bucket starts of a small population (its order: vals[0])
     int64_t bytes = 0;
 };
 
@@ -727,6 +856,7 @@ static void pairs_ws_free(lm_pairs_ws* w) {
     (void)hipFree(w->nbr_cnt);
     (void)hipFree(w->nbr);
     (void)hipFree(w->row_off);
+    (void)hipFree(w->small_tab);
     delete w;
 }
 
@@ -772,34 +902,40 @@ static int count_and_emit(lm_pairs_ws* ws, int32_t nsteps, int64_t n, const floa
 // The search of a small population.  A table of 64 x 64 buckets up to 4,096
 // particles, 128 x 64 above: about one particle in each.  Four lanes per
 // particle while the workgroups they take still run at once (one fills a
-// CU's LDS), else one.
+// CU's LDS), else one; and as long as that holds, an emit of 256 rows per
+// workgroup, which finds crowded rows four times as many at a time.
+template <int KIND, int NMAX, int LWX, int LWY>
+static int search_small_table(lm_pairs_ws* ws, int32_t nsteps, int64_t n, const float* lon, const float* lat,
+                              const CellGrid& g, const Metric& m, const Strides& st, int64_t* npairs, int32_t* pair_i,
+                              int32_t* pair_j, hipStream_t s) {
+    uint16_t* nbr = reinterpret_cast<uint16_t*>(ws->nbr);
+    const bool wide = (n + kSmallBlock / 4 - 1) / (kSmallBlock / 4) * nsteps <= 256;
+    const dim3 grid(grid_for(n, wide ? kSmallBlock / 4 : kSmallBlock), (unsigned)nsteps), block(kSmallBlock);
+    auto count = [&](auto kernel) {
+        LM_LAUNCH(K_PAIR_SMALL, kernel, grid, block, 0, s, (int)n, lon, lat, g, m, st, ws->nbr_cnt, nbr, ws->small_tab,
+                  ws->vals[0]);
+    };
+    auto emit = [&](auto kernel) {
+        LM_LAUNCH(K_EMIT_SMALL, kernel, grid, block, 0, s, (int)n, lon, lat, g, m, st, (const uint32_t*)ws->nbr_cnt,
+                  (const uint16_t*)nbr, (const uint32_t*)ws->small_tab, (const uint16_t*)ws->vals[0], pair_i, pair_j,
+                  npairs);
+    };
+    if (wide) count(pair_small_count_kernel<KIND, NMAX, LWX, LWY, 4>);
+    else count(pair_small_count_kernel<KIND, NMAX, LWX, LWY, 1>);
+    LM_LAUNCH_CHECK();
+    if (wide) emit(pair_small_emit_kernel<KIND, LWX, LWY, kSmallBlock / 4>);
+    else emit(pair_small_emit_kernel<KIND, LWX, LWY, kSmallBlock>);
+    LM_LAUNCH_CHECK();
+    return LM_OK;
+}
+
 template <int KIND>
 static int search_small(lm_pairs_ws* ws, int32_t nsteps, int64_t n, const float* lon, const float* lat,
                         const CellGrid& g, const Metric& m, const Strides& st, int64_t* npairs, int32_t* pair_i,
                         int32_t* pair_j, hipStream_t s) {
-    uint16_t* nbr = reinterpret_cast<uint16_t*>(ws->nbr);
-    const bool wide = (n + kSmallBlock / 4 - 1) / (kSmallBlock / 4) * nsteps <= 256;
-    const dim3 grid(grid_for(n, wide ? kSmallBlock / 4 : kSmallBlock), (unsigned)nsteps), block(kSmallBlock);
-    if (n <= 4096) {
-        if (wide)
-            LM_LAUNCH(K_PAIR_SMALL, (pair_small_count_kernel<KIND, 4096, 6, 6, 4>), grid, block, 0, s, (int)n, lon, lat,
-                      g, m, st, ws->nbr_cnt, nbr);
-        else
-            LM_LAUNCH(K_PAIR_SMALL, (pair_small_count_kernel<KIND, 4096, 6, 6, 1>), grid, block, 0, s, (int)n, lon, lat,
-                      g, m, st, ws->nbr_cnt, nbr);
-    } else {
-        if (wide)
-            LM_LAUNCH(K_PAIR_SMALL, (pair_small_count_kernel<KIND, (int)kSmallMax, 7, 6, 4>), grid, block, 0, s, (int)n,
-                      lon, lat, g, m, st, ws->nbr_cnt, nbr);
-        else
-            LM_LAUNCH(K_PAIR_SMALL, (pair_small_count_kernel<KIND, (int)kSmallMax, 7, 6, 1>), grid, block, 0, s, (int)n,
-                      lon, lat, g, m, st, ws->nbr_cnt, nbr);
-    }
-    LM_LAUNCH_CHECK();
-    LM_LAUNCH(K_EMIT_SMALL, pair_small_emit_kernel<KIND>, dim3(grid_for(n, kSmallBlock), (unsigned)nsteps), block, 0, s,
-              (int)n, lon, lat, m, st, (const uint32_t*)ws->nbr_cnt, (const uint16_t*)nbr, pair_i, pair_j, npairs);
-    LM_LAUNCH_CHECK();
-    return LM_OK;
+    if (n <= 4096)
+        return search_small_table<KIND, 4096, 6, 6>(ws, nsteps, n, lon, lat, g, m, st, npairs, pair_i, pair_j, s);
+    return search_small_table<KIND, (int)kSmallMax, 7, 6>(ws, nsteps, n, lon, lat, g, m, st, npairs, pair_i, pair_j, s);
 }
 
 }  // namespace lm
@@ -870,7 +1006,8 @@ int lm_pairs_ws_create_ex(int64_t n_max, int32_t steps_max, double lon_min, doub
         (rc = ws_alloc(&w->xy, S * n_max, &w->bytes)) ||
         (rc = ws_alloc(&w->nbr_cnt, S * w->row_stride, &w->bytes)) ||
         (rc = ws_alloc(&w->nbr, S * n_max * lm::kNbr, &w->bytes)) ||
-        (rc = ws_alloc(&w->row_off, S * w->row_stride, &w->bytes))) {
+        (rc = ws_alloc(&w->row_off, S * w->row_stride, &w->bytes)) ||
+        (rc = ws_alloc(&w->small_tab, S * lm::kSmallTab, &w->bytes))) {
         pairs_ws_free(w);
         return rc;
     }

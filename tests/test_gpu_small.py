@@ -39,6 +39,68 @@ def test_pairs_of_a_crowd(gpu, n):
     assert np.array_equal(gi, bi) and np.array_equal(gj, bj)
 
 
+def clumps(n, sizes, width, rng):
+    """Clumps of the given sizes, each within a tenth of a radius, spread over a patch of the given
+    width, and particles far from each other: the k-th of a clump of m has m - 1 - k partners above."""
+    m = sum(sizes)
+    x, y = 210.0 + width * rng.random(n), 30.0 + 0.2 * rng.random(n)
+    centre = np.repeat(np.arange(len(sizes)), sizes)
+    x[:m] = 210.0 + width * (centre + 0.5) / len(sizes) + 0.1 * R * rng.random(m)
+    y[:m] = 30.1 + 0.1 * R * rng.random(m)
+    o = rng.permutation(n)
+    return x[o].astype(np.float32), y[o].astype(np.float32)
+
+
+# clumps on both sides of the rows that are kept, gathered and found in index order, a chunk of 64
+# candidates and a wavefront's share of rows
+@pytest.mark.parametrize("n,sizes", [(700, [513, 18]), (4096, [17, 18, 64, 66, 513, 514]), (4097, [600, 65, 17, 130] + [19] * 90),
+                                     (12288, [700, 514] + [18] * 300)])
+@pytest.mark.parametrize("width,p", [(0.9, 2.0), (9.0, 1.0), (9.0, 3.0), (2.0, np.inf)])
+def test_pairs_of_crowded_rows(gpu, n, sizes, width, p):
+    x, y = clumps(n, sizes, width, np.random.default_rng(n))
+    gi, gj = gpu_pairs(x, y, R, p)
+    bi, bj = oracle.pairs_bruteforce(x, y, R, p)
+    assert np.array_equal(gi, bi) and np.array_equal(gj, bj)
+
+
+@pytest.mark.parametrize("n,steps", [(3000, 30), (12000, 25)])
+def test_pairs_of_crowded_rows_in_a_batch(gpu, n, steps):
+    # more steps than the workgroups of four lanes per particle and 256 rows are for
+    rng = np.random.default_rng(n)
+    at = [clumps(n, [[600, 30], [17], [], [40] * 20][s % 4], 0.9, rng) for s in range(steps)]
+    x, y = (np.stack([a[k] for a in at]) for k in (0, 1))
+    cap = 300 * n
+    ps = dev.PairSearch(n, (210.0, 210.9, 30.0, 30.2), R, steps_max=steps)
+    pi, pj = (torch.zeros((steps, cap), dtype=torch.int32, device="cuda") for _ in range(2))
+    count = torch.zeros(steps, dtype=torch.int64, device="cuda")
+    ps.query_batch(T(x), T(y), R, 2.0, pi, pj, count)
+    for s in [0, 1, 2, 3, steps - 1]:
+        bi, bj = oracle.pairs_bruteforce(x[s], y[s], R)
+        assert int(count[s]) == len(bi) <= cap
+        assert np.array_equal(pi[s, :len(bi)].cpu().numpy(), bi) and np.array_equal(pj[s, :len(bi)].cpu().numpy(), bj)
+
+
+def search_us(n, n_max, x, y):
+    ps, best = dev.PairSearch(n_max, (210.0, 212.0, 30.0, 32.0), R), np.inf
+    pi, pj = (torch.zeros(40 * n, dtype=torch.int32, device="cuda") for _ in range(2))
+    for _ in range(4):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        ps.query(x, y, R, 2.0, pi, pj, ps.npairs)
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, 1e3 * a.elapsed_time(b))
+    return best
+
+
+def test_search_of_a_dense_population(gpu):
+    # wide bound: finding every crowded row among all particles took 15 times the general kernels
+    rng = np.random.default_rng(0)
+    n, side = 12289, R * np.sqrt(12289 * np.pi / 24.0)  # twelve partners above each
+    x, y = (T((a + side * rng.random(n)).astype(np.float32)) for a in (210.0, 30.0))
+    assert search_us(n - 1, n, x[:-1].contiguous(), y[:-1].contiguous()) < 4 * search_us(n, n, x, y)
+
+
 def star_and_chain(n):
     pairs = {(0, k) for k in range(1, n)} | {(k, k + 1) for k in range(n - 1)}
     return np.array(sorted(pairs), dtype=np.int32)
