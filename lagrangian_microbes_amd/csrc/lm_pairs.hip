@@ -39,6 +39,7 @@
 #include "lm_sort.h"
 
 #include <cmath>
+#include <cstdint>
 #include <type_traits>
 
 namespace lm {
@@ -590,39 +591,41 @@ pair_small_count_kernel(int n, const float* __restrict__ x_all, const float* __r
         for (int k = t; k < (n + 1) / 2; k += kSmallBlock)
             order_all[s * st.rec + k] = reinterpret_cast<const uint32_t*>(idx)[k];
     }
-    const int i = (int)blockIdx.x * (kSmallBlock / LPP) + t / LPP, sub = t % LPP;
-    if (i >= n) return;  // all lanes of a particle
-    const float xi = x[i], yi = y[i];
-    int cx, cy;
-    cell_of(g, xi, yi, &cx, &cy);
-    auto search = [&](auto&& visit) {
-        if constexpr (LPP == 4) {
-            if (sub < 3) small_row<LWX, LWY>(start, g, cx, cy + sub - 1, visit);
-        } else {
-            for (int r = -1; r <= 1; ++r) small_row<LWX, LWY>(start, g, cx, cy + r, visit);
+    const int sub = t % LPP;
+    for (int i = (int)blockIdx.x * (kSmallBlock / LPP) + t / LPP; i < n; i += (int)gridDim.x * (kSmallBlock / LPP)) {
+        // (all lanes of a particle take the loop and its exits together)
+        const float xi = x[i], yi = y[i];
+        int cx, cy;
+        cell_of(g, xi, yi, &cx, &cy);
+        auto search = [&](auto&& visit) {
+            if constexpr (LPP == 4) {
+                if (sub < 3) small_row<LWX, LWY>(start, g, cx, cy + sub - 1, visit);
+            } else {
+                for (int r = -1; r <= 1; ++r) small_row<LWX, LWY>(start, g, cx, cy + r, visit);
+            }
+        };
+        uint32_t c = 0;
+        search([&](uint32_t k) {
+            const float2 o = pos[k];
+            c += pair_hit<KIND>(m, (int)idx[k] > i, xi, yi, o.x, o.y) ? 1u : 0u;
+        });
+        uint32_t at = 0, all = c;
+        if constexpr (LPP == 4) {  // the particle's lanes add up
+            const uint32_t up1 = __shfl_up(c, 1, 4), up2 = __shfl_up(c, 2, 4);
+            at = (sub > 0 ? up1 : 0u) + (sub > 1 ? up2 : 0u);
+            all = __shfl(at + c, 2, 4);
         }
-    };
-    uint32_t c = 0;
-    search([&](uint32_t k) {
-        const float2 o = pos[k];
-        c += pair_hit<KIND>(m, (int)idx[k] > i, xi, yi, o.x, o.y) ? 1u : 0u;
-    });
-    uint32_t at = 0, all = c;
-    if constexpr (LPP == 4) {  // the particle's lanes add up
-        const uint32_t up1 = __shfl_up(c, 1, 4), up2 = __shfl_up(c, 2, 4);
-        at = (sub > 0 ? up1 : 0u) + (sub > 1 ? up2 : 0u);
-        all = __shfl(at + c, 2, 4);
+        if (sub == 0) cnt_all[s * st.row + i] = all;
+        if (c == 0 || all > (uint32_t)kSmallNbr) continue;
+        uint16_t* row = nbr_all + 2 * s * st.nbr + (int64_t)i * kSmallNbr;
+        search([&](uint32_t k) {
+            const float2 o = pos[k];
+            if (pair_hit<KIND>(m, (int)idx[k] > i, xi, yi, o.x, o.y)) {
+                row[at] = idx[k];
+                ++at;
+            }
+        });
     }
-    if (sub == 0) cnt_all[s * st.row + i] = all;
-    if (c == 0 || all > (uint32_t)kSmallNbr) return;
-    uint16_t* row = nbr_all + 2 * s * st.nbr + (int64_t)i * kSmallNbr;
-    search([&](uint32_t k) {
-        const float2 o = pos[k];
-        if (pair_hit<KIND>(m, (int)idx[k] > i, xi, yi, o.x, o.y)) {
-            row[at] = idx[k];
-            ++at;
-        }
-    });
 }
 
 // LDS accesses of a wavefront's lanes before and after keep their order: the
@@ -899,32 +902,74 @@ static int count_and_emit(lm_pairs_ws* ws, int32_t nsteps, int64_t n, const floa
     return LM_OK;
 }
 
+// Turns of 1,024 particles that a workgroup of the count takes, of the `blocks`
+// of a step: binning the step again costs a workgroup about 12 us, a turn 10
+// (12,288 particles), and kSmallFit workgroups run at once, one per CU.
+constexpr int kSmallFit = 256;
+
+static int small_turns(int64_t nsteps, int blocks) {
+    int best = 1;
+    int64_t least = INT64_MAX;
+    for (int turns = 1; turns <= blocks; ++turns) {
+        const int64_t rounds = (nsteps * ((blocks + turns - 1) / turns) + kSmallFit - 1) / kSmallFit;
+        const int64_t cost = rounds * (6 + 5 * turns);
+        if (cost < least) {
+            least = cost;
+            best = turns;
+        }
+    }
+    return best;
+}
+
 // The search of a small population.  A table of 64 x 64 buckets up to 4,096
 // particles, 128 x 64 above: about one particle in each.  Four lanes per
 // particle while the workgroups they take still run at once (one fills a
 // CU's LDS), else one; and as long as that holds, an emit of 256 rows per
-// workgroup, which finds crowded rows four times as many at a time.
+// workgroup, which finds crowded rows four times as many at a time.  With one
+// lane per particle and above 4,096 particles, where binning a step is as much
+// work as searching for 1,024 of them, a step's workgroups each take several
+// turns (see small_turns), and whole multiples of kSmallFit steps, a workgroup
+// each, go out before the rest: 256 steps of 12,288 particles take 213 us, with
+// a workgroup for every 1,024 particles 305 (the general kernels 236); 300
+// steps 269, 363 (268); 64 steps 79, 95 (102).  4,096 particles, 300 steps: 104
+// us with a workgroup per 1,024, 125 in turns.
 template <int KIND, int NMAX, int LWX, int LWY>
 static int search_small_table(lm_pairs_ws* ws, int32_t nsteps, int64_t n, const float* lon, const float* lat,
                               const CellGrid& g, const Metric& m, const Strides& st, int64_t* npairs, int32_t* pair_i,
                               int32_t* pair_j, hipStream_t s) {
     uint16_t* nbr = reinterpret_cast<uint16_t*>(ws->nbr);
     const bool wide = (n + kSmallBlock / 4 - 1) / (kSmallBlock / 4) * nsteps <= 256;
-    const dim3 grid(grid_for(n, wide ? kSmallBlock / 4 : kSmallBlock), (unsigned)nsteps), block(kSmallBlock);
-    auto count = [&](auto kernel) {
-        LM_LAUNCH(K_PAIR_SMALL, kernel, grid, block, 0, s, (int)n, lon, lat, g, m, st, ws->nbr_cnt, nbr, ws->small_tab,
-                  ws->vals[0]);
+    const unsigned blocks = grid_for(n, wide ? kSmallBlock / 4 : kSmallBlock);
+    const dim3 block(kSmallBlock);
+    // steps [s0, s0 + ns), gx workgroups each
+    auto count = [&](auto kernel, int32_t s0, int32_t ns, unsigned gx) {
+        LM_LAUNCH(K_PAIR_SMALL, kernel, dim3(gx, (unsigned)ns), block, 0, s, (int)n, lon + s0 * st.pos,
+                  lat + s0 * st.pos, g, m, st, ws->nbr_cnt + s0 * st.row, nbr + 2 * s0 * st.nbr,
+                  ws->small_tab + (int64_t)s0 * kSmallTab, ws->vals[0] + s0 * st.rec);
     };
     auto emit = [&](auto kernel) {
-        LM_LAUNCH(K_EMIT_SMALL, kernel, grid, block, 0, s, (int)n, lon, lat, g, m, st, (const uint32_t*)ws->nbr_cnt,
-                  (const uint16_t*)nbr, (const uint32_t*)ws->small_tab, (const uint16_t*)ws->vals[0], pair_i, pair_j,
-                  npairs);
+        LM_LAUNCH(K_EMIT_SMALL, kernel, dim3(blocks, (unsigned)nsteps), block, 0, s, (int)n, lon, lat, g, m, st,
+                  (const uint32_t*)ws->nbr_cnt, (const uint16_t*)nbr, (const uint32_t*)ws->small_tab,
+                  (const uint16_t*)ws->vals[0], pair_i, pair_j, npairs);
     };
-    if (wide) count(pair_small_count_kernel<KIND, NMAX, LWX, LWY, 4>);
-    else count(pair_small_count_kernel<KIND, NMAX, LWX, LWY, 1>);
-    LM_LAUNCH_CHECK();
-    if (wide) emit(pair_small_emit_kernel<KIND, LWX, LWY, kSmallBlock / 4>);
-    else emit(pair_small_emit_kernel<KIND, LWX, LWY, kSmallBlock>);
+    if (wide) {
+        count(pair_small_count_kernel<KIND, NMAX, LWX, LWY, 4>, 0, nsteps, blocks);
+        LM_LAUNCH_CHECK();
+        emit(pair_small_emit_kernel<KIND, LWX, LWY, kSmallBlock / 4>);
+    } else {
+        const bool in_turns = NMAX > 4096;
+        const int32_t even = in_turns ? nsteps / kSmallFit * kSmallFit : 0, rest = nsteps - even;
+        if (even > 0) {
+            count(pair_small_count_kernel<KIND, NMAX, LWX, LWY, 1>, 0, even, 1);
+            LM_LAUNCH_CHECK();
+        }
+        if (rest > 0) {
+            const unsigned turns = in_turns ? (unsigned)small_turns(rest, (int)blocks) : 1u;
+            count(pair_small_count_kernel<KIND, NMAX, LWX, LWY, 1>, even, rest, (blocks + turns - 1) / turns);
+            LM_LAUNCH_CHECK();
+        }
+        emit(pair_small_emit_kernel<KIND, LWX, LWY, kSmallBlock>);
+    }
     LM_LAUNCH_CHECK();
     return LM_OK;
 }

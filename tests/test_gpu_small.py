@@ -80,6 +80,26 @@ def test_pairs_of_crowded_rows_in_a_batch(gpu, n, steps):
         assert np.array_equal(pi[s, :len(bi)].cpu().numpy(), bi) and np.array_equal(pj[s, :len(bi)].cpu().numpy(), bj)
 
 
+@pytest.mark.parametrize("n,steps", [(4200, 52), (4200, 300), (5000, 130), (8193, 100), (8200, 257)])
+def test_pairs_of_many_steps(gpu, n, steps):
+    # a step's workgroups in several turns, and batches of more steps than workgroups run at once
+    rng = np.random.default_rng(steps)
+    few = 12  # distinct steps
+    x, y = (210.0 + 0.6 * rng.random((few, n))).astype(np.float32), (30.0 + 0.6 * rng.random((few, n))).astype(np.float32)
+    of = np.arange(steps) % few
+    cap = 4 * n
+    ps = dev.PairSearch(n, (210.0, 210.6, 30.0, 30.6), R, steps_max=steps)
+    pi, pj = (torch.zeros((steps, cap), dtype=torch.int32, device="cuda") for _ in range(2))
+    count = torch.zeros(steps, dtype=torch.int64, device="cuda")
+    ps.query_batch(T(x[of]), T(y[of]), R, 2.0, pi, pj, count)
+    count, pi, pj = count.cpu().numpy(), pi.cpu().numpy(), pj.cpu().numpy()
+    for k in range(few):
+        bi, bj = oracle.pairs_bruteforce(x[k], y[k], R)
+        assert 0 < len(bi) <= cap
+        for s in np.flatnonzero(of == k):
+            assert count[s] == len(bi) and np.array_equal(pi[s, :len(bi)], bi) and np.array_equal(pj[s, :len(bi)], bj), s
+
+
 def search_us(n, n_max, x, y):
     ps, best = dev.PairSearch(n_max, (210.0, 212.0, 30.0, 32.0), R), np.inf
     pi, pj = (torch.zeros(40 * n, dtype=torch.int32, device="cuda") for _ in range(2))
