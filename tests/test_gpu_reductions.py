@@ -41,3 +41,25 @@ def test_histogram_at_the_edges(gpu, kind, n, bins):
     radius = analysis.EARTH_RADIUS_M if bins < 100 else 10.0 ** (0.1 * bins)  # thresholds that increase
     got = analysis.distance_histogram(torch.from_numpy(lon).cuda(), torch.from_numpy(lat).cuda(), bins, radius)
     assert np.array_equal(got, oracle.distance_histogram(lon, lat, analysis.haversine_thresholds(bins, radius)))
+
+
+def histogram_us(lon, lat):
+    """The kernel alone, from events around the call's launches."""
+    lon, lat, best = torch.from_numpy(lon).cuda(), torch.from_numpy(lat).cuda(), np.inf
+    for _ in range(4):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        analysis.distance_histogram(lon, lat)
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, 1e3 * a.elapsed_time(b))
+    return best
+
+
+def test_points_all_over_the_globe_cost_little_more(gpu):
+    # bound between 1.2 (what it takes) and 2.5 times the basin's (with cosines and a search per pair)
+    rng = np.random.default_rng(3)
+    n = 40_000
+    near = histogram_us(rng.uniform(120.0, 280.0, n).astype(np.float32), rng.uniform(-60.0, 60.0, n).astype(np.float32))
+    far = histogram_us(rng.uniform(0.0, 360.0, n).astype(np.float32), rng.uniform(-90.0, 90.0, n).astype(np.float32))
+    assert far < 1.8 * near
