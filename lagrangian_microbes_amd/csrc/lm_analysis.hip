@@ -169,14 +169,12 @@ constexpr int kLutShift = 19;
 constexpr uint32_t kLutBase = (127u - 60u) << (23 - kLutShift);
 constexpr uint32_t kLutCells = 61u << (23 - kLutShift);
 
-// Number of increasing edges e[0 .. m) with e * scale <= v (or < v).
-template <bool STRICT>
+// Number of increasing edges e[0 .. m) with e * scale <= v.
 __device__ __forceinline__ int edges_below(const double* e, int m, double scale, double v) {
     int lo = 0, hi = m;
     while (lo < hi) {
         const int mid = (lo + hi) >> 1;
-        const double x = e[mid] * scale;
-        if (STRICT ? x < v : x <= v) lo = mid + 1;
+        if (e[mid] * scale <= v) lo = mid + 1;
         else hi = mid;
     }
     return lo;
@@ -187,7 +185,7 @@ __device__ __forceinline__ int exact_bin(const double* e, int m, float xi, float
     const double s1 = sin_deg(0.5 * ((double)yj - (double)yi));
     const double s2 = sin_deg(0.5 * ((double)xj - (double)xi));
     const double a = s1 * s1 + (cos_deg((double)yi) * cos_deg((double)yj)) * (s2 * s2);
-    return edges_below<false>(e, m, 1.0, a);
+    return edges_below(e, m, 1.0, a);
 }
 
 // A workgroup takes a tile of 512 points i (two per lane) against `per`
@@ -267,7 +265,7 @@ __device__ __forceinline__ void hist_tile_f64(const HistShared& S, uint32_t* __r
             const float2 e = S.lut[cell];
             const bool above = af > e.x * (1.0f + kHistTol), below = af < e.x * (1.0f - kHistTol);
             uint32_t bin = __float_as_uint(e.y) + (above ? 1u : 0u);
-            if (!(above | below)) bin = a == a ? (uint32_t)edges_below<false>(S.edges, nedges, 1.0, a) : 0u;
+            if (!(above | below)) bin = a == a ? (uint32_t)edges_below(S.edges, nedges, 1.0, a) : 0u;
             if (k > after[u]) atomicAdd(&h[bin * cols + col], 1u);
         }
     }
@@ -337,10 +335,11 @@ dist_hist_kernel(int64_t n, const float* __restrict__ lon, const float* __restri
     for (uint32_t c = t; c <= kLutCells; c += kHistTile) {
         const float from = __uint_as_float((c + kLutBase) << kLutShift);
         const float to = __uint_as_float((c + 1u + kLutBase) << kLutShift);
-        const int b0 = edges_below<false>(S.edges, nedges, 1.0 + (double)kHistTol, (double)from);
-        const int b1 = edges_below<true>(S.edges, nedges, 1.0 - (double)kHistTol, (double)to);
-        float e = b1 == b0 ? FLT_MAX : b1 == b0 + 1 ? (float)S.edges[b0] : NAN;
-        if (c == kLutCells || to >= turn) e = NAN;
+        const int b0 = edges_below(S.edges, nedges, 1.0 + (double)kHistTol, (double)from);
+        // how many of the thresholds from b0 on may lie below the cell's end: none, one, more
+        const double first = b0 < nedges ? S.edges[b0] : INFINITY, second = b0 + 1 < nedges ? S.edges[b0 + 1] : INFINITY;
+        float e = first * (1.0 - (double)kHistTol) < (double)to ? (float)first : FLT_MAX;
+        if (c == kLutCells || to >= turn || second * (1.0 - (double)kHistTol) < (double)to) e = NAN;
         S.lut[c] = make_float2(e, __uint_as_float((uint32_t)b0));
     }
     for (int q = 0; q < per; ++q) {
