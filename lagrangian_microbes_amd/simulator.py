@@ -134,9 +134,11 @@ class FusedRunner:
         the advection of chunk c + 2 (FP64 arithmetic) runs on its own stream
         beside the pair search and grouping of chunk c + 1 (memory-latency
         bound) on a side stream, while chunk c replays the species on a
-        stream of its own (a small population's on the caller's), which the
-        caller's waits for before the callback.  The advection of a chunk waits for the replay that
-        last used its set; the grouping waits for its advection.  After each
+        stream of its own (a small population's, and that of a run of one chunk,
+        on the caller's), for which the caller's waits before the callback, and
+        without one at the end of the run.  The advection of a chunk waits for
+        the replay that last used its set; the grouping waits for its advection.
+        After each
         chunk, ``on_chunk(k, rec_x, rec_y, rec_s, npairs)`` receives that
         chunk's records (device views, valid until the callback returns; if
         it returns a torch.cuda.Event, e.g. after copies on another stream
@@ -155,9 +157,14 @@ class FusedRunner:
         nsets = self.PIPELINE_SETS
         main = torch.cuda.current_stream(self.device)
         side, adv = self._side, self._adv
-        # a small population's replay is one launch: the caller's stream does
-        play = self._play if self.n > SMALL_POPULATION else main
         sizes = chunk_schedule(total, self.chunk)
+        # a small population's replay is one launch, and a single chunk has no
+        # other to run beside: the caller's stream does (4 steps of 13,000 in
+        # one chunk take 365 us, 415 with a stream of its own)
+        play = self._play if self.n > SMALL_POPULATION and len(sizes) > 1 else main
+        # without a callback the caller's stream waits for the replays at the end
+        # only (8 steps of 13,000 in chunks of 4 take 610 us, 660 with a wait per chunk)
+        seen = on_chunk is not None
         if max(sizes) > self.chunk:  # the chunk buffers hold self.chunk steps
             raise RuntimeError(f"chunk schedule exceeds the buffers: {sizes}")
         self.last_schedule = list(sizes)  # chunk lengths of this call, one batched launch each
@@ -186,8 +193,9 @@ class FusedRunner:
         # has been issued (chunk c + 3 reuses chunk c's set)
         ev_adv, ev_prep, ev_play, ev_count, ev_replay, ev_join = self._events
         ev_join[0].record(main)          # the state as the caller left it
-        for st in {side, adv, play} - {main}:
-            st.wait_event(ev_join[0])
+        for st in (side, adv, play):
+            if st is not main:
+                st.wait_event(ev_join[0])
 
         def advect(c):
             b, k = c % nsets, sizes[c]
@@ -216,7 +224,7 @@ class FusedRunner:
         def replay(c):
             b, k = c % nsets, sizes[c]
             play.wait_event(prepared[c])
-            if c > 0 and play is not main:  # the callback may read the species
+            if c > 0 and seen and play is not main:  # the callback may read the species
                 play.wait_event(played[(c - 1) % nsets])
             rs = recs(c)[2]
             # The replay goes out before the host has seen the chunk's pair
@@ -244,7 +252,7 @@ class FusedRunner:
                     self.species.copy_(backup)
                     eng.play_set(b, k, self.species, rs)
                     worst = eng.worst_count(b, k)
-            if play is not main:
+            if seen and play is not main:
                 ev_replay.record(play)
                 main.wait_event(ev_replay)
 
@@ -267,8 +275,8 @@ class FusedRunner:
                 if on_chunk is not None:
                     rx, ry, rs = recs(c)
                     ret = on_chunk(k, rx, ry, rs, eng.npairs_sets[b][:k])
-                ev = ev_play[b]  # after the callback's own work on this stream
-                ev.record(main)
+                ev = ev_play[b]  # after the callback's own work on the caller's stream
+                ev.record(main if seen else play)
                 played[b] = ev
                 released[b] = ret if isinstance(ret, torch.cuda.Event) else None
                 self.step += k
