@@ -63,3 +63,31 @@ def test_points_all_over_the_globe_cost_little_more(gpu):
     near = histogram_us(rng.uniform(120.0, 280.0, n).astype(np.float32), rng.uniform(-60.0, 60.0, n).astype(np.float32))
     far = histogram_us(rng.uniform(0.0, 360.0, n).astype(np.float32), rng.uniform(-90.0, 90.0, n).astype(np.float32))
     assert far < 1.8 * near
+
+
+def haversine_term(lon, lat, i, j):
+    """The term of one pair as the oracle computes it."""
+    xi, yi, xj, yj = (float(v) for v in (lon[i], lat[i], lon[j], lat[j]))
+    s1, s2 = oracle.sin_deg(0.5 * (yj - yi)), oracle.sin_deg(0.5 * (xj - xi))
+    return s1 * s1 + (oracle.cos_deg(yi) * oracle.cos_deg(yj)) * (s2 * s2)
+
+
+@pytest.mark.parametrize("n", [2, 513, 1300])
+def test_thresholds_that_terms_meet(gpu, n):
+    # the thresholds are terms of the points' own pairs, and their neighbours, so that every
+    # one of them has a term on it or one step away; near and far apart, and increasing as they have to
+    from lagrangian_microbes_amd import _lib
+    rng = np.random.default_rng(n)
+    for spread_deg in (8.0, 300.0):
+        lon = (20.0 + spread_deg * rng.random(n)).astype(np.float32)
+        lat = (-0.2 * spread_deg + 0.4 * spread_deg * rng.random(n)).clip(-90, 90).astype(np.float32)
+        i, j = rng.integers(0, n - 1, 36), rng.integers(0, n, 36)
+        j = np.where(j > i, j, i + 1)
+        term = np.array([haversine_term(lon, lat, a, b) for a, b in zip(i, j)])
+        near = [term, np.nextafter(term, 0), np.nextafter(term, 1)]
+        edges = np.unique(np.concatenate(near + [term * (1 + 1e-6 * f) for f in (-5, -3, 3, 5)])[:255])
+        hist = torch.zeros(len(edges) + 1, dtype=torch.int64, device="cuda")
+        dev = [torch.from_numpy(a).cuda() for a in (lon, lat, edges)]
+        _lib.check(_lib.load().lm_distance_histogram(n, _lib.ptr(dev[0]), _lib.ptr(dev[1]), len(edges) + 1, _lib.ptr(dev[2]),
+                                                     _lib.ptr(hist), _lib.stream_ptr()))
+        assert np.array_equal(hist.cpu().numpy().astype(np.uint64), oracle.distance_histogram(lon, lat, edges))
