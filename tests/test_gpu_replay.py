@@ -41,6 +41,52 @@ def test_component_classes(gpu, n):
     assert st.wide_components == len(wide) and st.wide_pairs == sum(wide)
 
 
+def components(n, sizes, rng):
+    """Sorted pairs of components of (particles, pairs) each on shuffled indices."""
+    perm, pairs, at = rng.permutation(n), set(), 0
+    for size, count in sizes:
+        ids = np.sort(perm[at:at + size])
+        at += size
+        mine = {(int(ids[int(rng.integers(max(0, a - 3), a))]), int(ids[a])) for a in range(1, size)}  # a spanning tree
+        while len(mine) < count:
+            a, b = np.sort(rng.choice(ids, 2, replace=False))
+            mine.add((int(a), int(b)))
+        assert len(mine) == count
+        pairs |= mine
+    assert at <= n
+    return np.array(sorted(pairs), dtype=np.int32)
+
+
+# on both sides of the number of steps from which the links of smaller and larger components take a
+# launch each, and of the population from which components of 17 to 32 pairs are small
+@pytest.mark.parametrize("n,steps", [(12_289, 23), (12_289, 24), (140_000, 25)])
+def test_component_classes_of_a_batch(gpu, n, steps):
+    import torch
+    from lagrangian_microbes_amd import device as dev
+    rng = np.random.default_rng(n + steps)
+    # pairs on both sides of the launches' limit (256) with few particles and with as many as pairs allow, on both
+    # sides of the tables' slots (264, 2,048), and more particles than the replay holds in LDS (4,112)
+    sizes = [(16, 16), (17, 17), (32, 32), (30, 33), (65, 64), (66, 65), (200, 255), (257, 256), (60, 256), (258, 257),
+             (60, 257), (264, 300), (265, 300), (266, 300), (500, 2000), (2048, 2100), (2049, 2100)]
+    lists = [components(n, sizes, rng), components(n, sizes[:10] + [(4112, 4200)], rng),
+             components(n, sizes[8:] + [(4113, 4500)], rng), components(n, sizes[:4], rng)]
+    cap = max(len(a) for a in lists)
+    pi, pj = np.zeros((steps, cap), np.int32), np.zeros((steps, cap), np.int32)
+    count = np.zeros(steps, np.int64)
+    for s in range(steps):
+        a = lists[s % 4]
+        pi[s, :len(a)], pj[s, :len(a)], count[s] = a[:, 0], a[:, 1], len(a)
+    sp = rng.integers(0, 5, n).astype(np.int8)
+    up = dev.RPSUpdater(n, steps_max=steps)
+    up.prepare(n, *(torch.from_numpy(a).cuda() for a in (pi, pj, count)), 0.55, 0.5, 0.45, (3, 4), 17)
+    rec = torch.zeros((steps, n), dtype=torch.int8, device="cuda")
+    up.play_steps(steps, torch.from_numpy(sp).cuda(), rec)
+    rec = rec.cpu().numpy()
+    for s in range(steps):
+        sp = oracle.rps_sequential(sp, pi[s, :count[s]], pj[s, :count[s]], 0.55, 0.5, 0.45, (3, 4), 17 + s)
+        assert np.array_equal(rec[s], sp), s
+
+
 @pytest.mark.parametrize("form", ["plain", "read-only", "strided", "reversed"])
 def test_reset_takes_any_array(gpu, form):
     from lagrangian_microbes_amd import FusedRunner, VelocityField
