@@ -49,9 +49,9 @@
 //   small    one lane per component of <= 16 or 32 pairs, replayed in order
 //   copy     particles without pairs keep their species
 //
-// Small populations (workspaces of kSmallMax particles, no runs) take two kernels instead,
-// one for the whole prepare and one that replays all steps of a batch (see
-// "small populations" below).
+// Small populations (workspaces of kSmallMax particles, no runs; see
+// kSmallSure) take two kernels instead, one for the whole prepare and one that
+// replays all steps of a batch.
 #include "lm_common.h"
 #include "lm_scan.h"
 #include "lm_small.h"
@@ -1105,9 +1105,8 @@ rps_play_kernel(int64_t n, int64_t s, RpsArrays A, RpsStrides st, const int8_t* 
 // small populations
 // ---------------------------------------------------------------------------
 // Up to kSmallMax particles the whole state of a step fits a workgroup, and
-// launches are what the general path's time goes to (24 steps of 10,000
-// particles: 78 prepare launches and 24 replays of 8 to 28 us).  No
-// components here:
+// launches are what the general path's time goes to where pairs are few (see
+// kSmallSure).  No components here:
 //   prepare  a workgroup per step: per pair its outcome bits and, for each of
 //            its two particles, the pairs before and after it that touch the
 //            particle
@@ -1119,10 +1118,10 @@ rps_play_kernel(int64_t n, int64_t s, RpsArrays A, RpsStrides st, const int8_t* 
 //            then, round by round, only the pairs right after one whose result
 //            changed.  Values only travel where they change: 6,500 pairs whose
 //            longest chain is 126 settle in 10 to 18 rounds of ever fewer
-//            pairs (levels, one after another, would take 126).  A step of
-//            10,000 particles and 6,500 pairs takes about 11 us, where the
-//            general replay's launch takes 8 to 28; a run of 24 such steps
-//            from the lattice went from 1,070 to 635 us in all.
+//            pairs (levels, one after another, would take 126).  In a batch,
+//            a step with 1,450 pairs takes 7 us, with 3,600 9, with a whole
+//            window of 8,192 13; a run of 24 steps of 2,500 particles 760 us,
+//            1,170 by the general kernels as they were then.
 // Pairs go in windows of kSmallWindow; a pair whose predecessor is in an
 // earlier window starts from the particle's species, which a window's last
 // pair at it updates.  A pair whose j is no other particle changes nothing.
@@ -1130,6 +1129,17 @@ rps_play_kernel(int64_t n, int64_t s, RpsArrays A, RpsStrides st, const int8_t* 
 // outcome bits << 28 | kSmallNoop; source = 2 * (pair in the window) + side,
 // or kSmallSpecies + particle; next = pair in the window or kSmallNone.
 // links: i | j << 14 | kSmallValid.
+// The class: up to kSmallSure particles, whose pairs fit about one window unless
+// the population hangs together, always; up to kSmallMax where the caller's pair
+// capacity, grown to two and a half pairs per particle, says that it does (the
+// general replay has one wavefront for a component: 24 steps of 12,288
+// particles with 2.4 partners above each take 9.0 ms there, 1.3 here).  In
+// between a step takes several windows, one after another, and the general
+// replay, 7 us a step, is the faster one but for the sparsest: 24 steps of
+// 12,288, prepare and replay, with 0.3 partners 217 us here and 240 there, 0.6:
+// 359 and 268, 1.2: 691 and 307, 1.8: 1,061 and 428.  At the line, 24 steps of
+// 5,184 with their search: 0.6 partners 232 and 329, 1.6: 450 and 362.
+constexpr int64_t kSmallSure = 5120;
 constexpr uint32_t kSmallValid = 0x80000000u, kSmallNoop = 0x80000000u;
 constexpr int kSmallPairs = 8;  // pairs per thread in a window
 constexpr uint32_t kSmallWindow = kSmallBlock * kSmallPairs;
@@ -1763,7 +1773,8 @@ static int rps_prepare_impl(lm_rps_ws* ws, int32_t nsteps, int64_t n, const int3
     const unsigned S = (unsigned)nsteps;
     // one workgroup holds a small step; without pairs the general replay's
     // copy is all there is to do, and an ensemble's runs have keys of their own
-    ws->small = ws->n_max <= lm::kSmallMax && run == nullptr && pair_stride > 0;
+    ws->small = ws->n_max <= lm::kSmallMax && run == nullptr && pair_stride > 0 &&
+                (n <= lm::kSmallSure || pair_stride >= n * 5 / 2);
     if (ws->small) {
         LM_LAUNCH(lm::K_RPS_SMALL, lm::rps_small_kernel, dim3(S), dim3(lm::kSmallBlock), 0, s, (uint32_t)n, pair_i,
                   pair_j, npairs, A, sp, pRS, pPR, pSP, key0, key1, step0);

@@ -31,7 +31,10 @@ logger = logging.getLogger(__name__)
 
 # Smallest chunk the tapered end of a pipelined run uses.
 TAPER_MIN = 8
-# Largest population whose batches take a launch per phase (kSmallMax of liblm).
+# Largest population whose chunks replay on the caller's stream: a stream more
+# costs more in events than the overlap gives (200 steps of 8,000 microbes in
+# chunks of 24, dense and sparse, 3.3 to 5.2 ms, 3.5 to 7.2 with it; 24 steps
+# 0.92 to 0.95, 1.05 to 1.09), while above it gives more (see _ensure_pipeline).
 SMALL_POPULATION = 12288
 
 
@@ -158,9 +161,9 @@ class FusedRunner:
         main = torch.cuda.current_stream(self.device)
         side, adv = self._side, self._adv
         sizes = chunk_schedule(total, self.chunk)
-        # a small population's replay is one launch, and a single chunk has no
-        # other to run beside: the caller's stream does (4 steps of 13,000 in
-        # one chunk take 365 us, 415 with a stream of its own)
+        # a small population's replay is short, and a single chunk has no other
+        # to run beside: the caller's stream does (4 steps of 13,000 in one
+        # chunk take 365 us, 415 with a stream of its own)
         play = self._play if self.n > SMALL_POPULATION and len(sizes) > 1 else main
         # without a callback the caller's stream waits for the replays at the end
         # only (8 steps of 13,000 in chunks of 4 take 610 us, 660 with a wait per chunk)

@@ -162,6 +162,38 @@ def test_rps_pairs_in_any_direction(gpu, n):
     assert np.array_equal(g, ref)
 
 
+def batch_us(n, pi, pj, counts):
+    """Prepare and replay of a batch."""
+    up, best = dev.RPSUpdater(n, steps_max=len(counts)), np.inf
+    species = torch.ones(n, dtype=torch.int8, device="cuda")
+    species[::3], species[1::3] = 2, 3
+    rec = torch.zeros((len(counts), n), dtype=torch.int8, device="cuda")
+    for _ in range(5):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        up.prepare(n, pi, pj, counts, 0.5, 0.5, 0.5, (1, 2), 0)
+        up.play_steps(len(counts), species, rec)
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, 1e3 * a.elapsed_time(b))
+    return best
+
+
+def test_a_batch_is_not_slower_below_the_line(gpu):
+    # 12,288 particles with 1.5 partners above each, 24 steps: the general kernels, which 12,289
+    # take, need 315 us, one workgroup 915; the bound lies between
+    rng = np.random.default_rng(5)
+    n, S = 12288, 24
+    side = R * np.sqrt(n * np.pi / 3.0)
+    x, y = (T((a + side * rng.random((S, n))).astype(np.float32)) for a in (210.0, 30.0))
+    ps = dev.PairSearch(n, (210.0, 210.0 + side, 30.0, 30.0 + side), R, steps_max=S)
+    pi, pj = (torch.zeros((S, 2 * n), dtype=torch.int32, device="cuda") for _ in range(2))
+    counts = torch.zeros(S, dtype=torch.int64, device="cuda")
+    ps.query_batch(x, y, R, 2.0, pi, pj, counts)
+    assert int(counts.max()) <= 2 * n
+    assert batch_us(n, pi, pj, counts) < 1.7 * batch_us(n + 1, pi, pj, counts)
+
+
 def crowded(kind, n, rng):
     """Sorted pair lists with many pairs of one j."""
     ids = np.arange(n)
@@ -181,6 +213,13 @@ def crowded(kind, n, rng):
     return np.unique(np.array(pairs, dtype=np.int32), axis=0)
 
 
+def buffers(arr, cap):
+    """The pairs in buffers of a larger capacity."""
+    out = np.zeros((2, max(cap, len(arr))), np.int32)
+    out[:, :len(arr)] = arr.T
+    return T(out[0]), T(out[1])
+
+
 @pytest.mark.parametrize("n", [66, 2500, 12288])
 @pytest.mark.parametrize("kind", ["hub last", "hub between", "crowd", "lists of 16", "one list of 17"])
 def test_rps_many_pairs_of_one_j(gpu, kind, n):
@@ -188,12 +227,36 @@ def test_rps_many_pairs_of_one_j(gpu, kind, n):
     arr = crowded(kind, n, rng)
     sp = rng.integers(0, 5, n).astype(np.int8)
     args = (0.5, 0.6, 0.4, (n, 2), 5)
-    g, _ = gpu_rps(sp, arr[:, 0], arr[:, 1], *args)
-    assert np.array_equal(g, oracle.rps_sequential(sp, arr[:, 0], arr[:, 1], *args))
+    got = T(sp)
+    dev.RPSUpdater(n).update(got, *buffers(arr, 3 * n), T(np.array([len(arr)])), *args)
+    assert np.array_equal(got.cpu().numpy(), oracle.rps_sequential(sp, arr[:, 0], arr[:, 1], *args))
+
+
+# on both sides of the populations and of the pair capacity that the small kernels are for
+@pytest.mark.parametrize("n", [5120, 5121, 12288])
+@pytest.mark.parametrize("over", [-1, 0])
+def test_rps_at_the_lines_of_the_class(gpu, n, over):
+    rng = np.random.default_rng(n + over)
+    S, cap = 4, n * 5 // 2 + over
+    lists = [np.stack(random_pairs(rng, n, m), 1) for m in (n // 2, n, 2 * n, n * 5 // 2 - 1)]
+    lists[1] = star_and_chain(n)
+    pi, pj = (torch.stack(b) for b in zip(*(buffers(a, cap) for a in lists)))
+    counts = np.array([len(a) for a in lists])
+    assert counts.max() <= cap
+    sp = rng.integers(0, 5, n).astype(np.int8)
+    up = dev.RPSUpdater(n, steps_max=S)
+    up.prepare(n, pi, pj, T(counts), 0.55, 0.5, 0.45, (3, 4), 17)
+    rec = torch.zeros((S, n), dtype=torch.int8, device="cuda")
+    up.play_steps(S, T(sp), rec)
+    for s, a in enumerate(lists):
+        sp = oracle.rps_sequential(sp, a[:, 0], a[:, 1], 0.55, 0.5, 0.45, (3, 4), 17 + s)
+        assert np.array_equal(rec[s].cpu().numpy(), sp), s
+    st = up.component_stats(1)
+    assert st.components == 1 and st.pairs == st.max_pairs == len(lists[1]) and st.touched == st.max_particles == n
 
 
 def prepare_us(n, arr):
-    pi, pj = T(arr[None, :, 0].copy()), T(arr[None, :, 1].copy())
+    pi, pj = (b[None] for b in buffers(arr, 3 * n))
     count, up, best = T(np.array([len(arr)])), dev.RPSUpdater(n), np.inf
     for _ in range(4):
         a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
