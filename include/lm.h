@@ -210,9 +210,9 @@ int lm_rps_prepare(lm_rps_ws* ws, int32_t nsteps, int64_t n, const int32_t* pair
                    double pRS, double pPR, double pSP, uint64_t key0, uint64_t key1,
                    uint64_t step0, void* stream);
 /* Launch shape of lm_rps_play: workgroups (64 lanes) that take wide
- * components (one wavefront each, by level) and that take small components
- * (one lane each); both loop over their components, so any counts >= 1 give
- * the same result (defaults 2048 and 2048).  No reference counterpart (set by
+ * components (one wavefront each, 64 pairs at a time) and that take small
+ * components (one lane each); both loop over their components, so any counts
+ * >= 1 give the same result (defaults 2048 and 2048).  No reference counterpart (set by
  * the ensemble's autotuner). */
 int lm_rps_ws_set_play_blocks(lm_rps_ws* ws, int32_t wide_blocks, int32_t narrow_blocks);
 
@@ -257,8 +257,9 @@ int lm_rps_play_steps(lm_rps_ws* ws, int32_t nsteps, int64_t n, const int8_t* sp
 /* Size statistics of the interaction components of step `step` of the last
  * prepare, written to device int64[8]: components with at least one pair,
  * largest component (pairs), largest component (particles), total pairs,
- * components replayed by a wavefront (more than 32 pairs), their pairs, their
- * particles, particles with at least one pair.  Diagnostic only. */
+ * components of more than 32 pairs, their pairs, their particles (whatever
+ * lm_rps_play replays them by), particles with at least one pair.  Diagnostic
+ * only. */
 int lm_rps_component_stats(lm_rps_ws* ws, int32_t step, int64_t* out8, void* stream);
 
 /* ------------------------------------------------------------------------ */

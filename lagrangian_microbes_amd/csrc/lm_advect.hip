@@ -126,7 +126,8 @@ __device__ __forceinline__ float cos_deg_f32(float lat_deg) {
     return fmaf(p, z, 1.0f);
 }
 
-// divide_near_one in float32.
+// divide_near_one in float32: the IEEE quotient for |n| zero or at least 2^-100
+// (1e-25 m/s in degrees per second).
 __device__ __forceinline__ float divide_near_one_f32(float n, float d) {
     float r = __builtin_amdgcn_rcpf(d);
     r = fmaf(fmaf(-d, r, 1.0f), r, r);

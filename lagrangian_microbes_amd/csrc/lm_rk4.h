@@ -1,5 +1,6 @@
-// One sample of a gridded velocity field and one RK4 step, FP64: what the
-// advection and the adjoint's forward share, bit for bit.
+// One FP64 sample of a gridded velocity field, which the advection and the
+// adjoint's forward share; each has an RK4 step of its own around it, in the
+// same operation order and so with the same bits.
 //
 // Operation order (mirrored operation by operation in oracle/lm_oracle.c):
 //   fx  = (x - x0) * inv_dx,          i = trunc(fx) clamped to nx-2, xi  = fx - i
@@ -44,10 +45,16 @@ __device__ __forceinline__ double cos_deg_from(const CosCoefs& K, double lat_deg
     return lm_horner<12>(K.c, t * t);
 }
 
-// n / d rounded as the IEEE division rounds it, without its scaling: the
-// operands are velocities (m/s to degrees) and cosines, far from the ends of
-// the exponent range, where the scaling steps multiply by one.  Zeros,
-// infinities and NaN come from the fix-up, as in the division.
+// n / d by Newton-Raphson: the hardware's reciprocal, two steps, the quotient
+// and one correction by its residual, whose last fma rounds as the IEEE division
+// does (Markstein).  Without that division's scaling, which keeps the reciprocal,
+// the quotient and the residual in range: here d is a cosine and n a velocity in
+// degrees per second.  Equal to the IEEE quotient while |n| is zero or at least
+// 2^-960 and the quotient is finite; smaller numerators, whose residual
+// underflows, may be off by the last bit, and a finite n over so small a d that
+// the quotient overflows gives NaN instead of infinity (as a position, outside
+// every grid like it).  Zeros, infinities and NaN come from the fix-up, as in the
+// division.
 __device__ __forceinline__ double divide_near_one(double n, double d) {
     double r = __builtin_amdgcn_rcp(d);
     r = fma(r, fma(-d, r, 1.0), r);

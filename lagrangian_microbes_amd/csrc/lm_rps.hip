@@ -63,10 +63,13 @@ constexpr uint32_t kUnset = 0xffffffffu;
 // A component of up to 32 pairs is small: one lane replays it, pair after pair
 // (about 100 ns each); a larger one takes a wavefront.  Up to kFewParticles
 // particles the limit is 16: a step's replay then waits for its longest serial
-// chain, and the components between the limits find wavefronts free.  124,000
-// particles, 60 steps: 1,748 us with 32, 1,572 with 16; but 242,000 dense
-// ones, 100 steps: 6.54 and 6.74 ms, and 4,000,000, 96 steps: 81.9 and 87.2
-// ms, where these components are thousands.
+// chain, and the components between the limits find wavefronts free; they no
+// longer do where there are thousands of them, which grows with the density as
+// well as with the population, but only that is known when a batch is prepared.
+// Replay of 24 steps of 120,000 with 0.6, 1.2, 1.5, 1.8 partners above each: 189,
+// 216, 264, 469 us with 16, 240, 279, 294, 412 with 32; of 12 steps of 400,000
+// with 0.6, 0.9, 1.2, 1.5: 125, 144, 218, 278 with 16, 148, 166, 180, 203 with 32;
+// 96 steps of 4,000,000 81.9 ms with 32, 87.2 with 16.
 constexpr uint32_t kNarrowPairs = 32, kNarrowPairsFew = 16;
 constexpr int64_t kFewParticles = 1 << 17;
 constexpr uint32_t kNarrowSlots = kNarrowPairs + 1;  // a component of P pairs has <= P + 1 particles
@@ -503,8 +506,8 @@ rps_keys_kernel(int64_t n, RpsArrays A, RpsStrides st, bool write_vals) {
 // ~2^10 particles),
 // 11 up to 2^21 (half the counters to clear and scan and one bit less to rank
 // by than with 12, for a 10-bit radix pass in place of a 9-bit one: sixteen
-// runs of 1,280,000 particles, 96 steps, 21.95 -> 21.30 ms; 1,950,000, 30
-// steps, 13.46 -> 13.14), 12 up to 2^22, 14 up to 2^24 (ensembles; 64 KB of
+// runs of 1,280,000 particles, 96 steps, 20.3 -> 20.0 ms, means of nine whose
+// range is 1.8; 1,950,000, 30 steps, 12.0 -> 11.7), 12 up to 2^22, 14 up to 2^24 (ensembles; 64 KB of
 // counters).
 constexpr uint32_t kGroupFineBits = 10;
 constexpr uint32_t kGroupFineBitsMid = 11;

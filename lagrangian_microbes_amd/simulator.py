@@ -302,8 +302,8 @@ class FusedRunner:
             # queues out in turn, so consecutive streams are on different ones
             # and their kernels run side by side.  With two, and the replay on
             # the caller's stream, the three met on one queue in half of the
-            # runners: up to 127 ms for 720 steps of 490,000 microbes, 61 to 92 now (by the
-            # field, whose eddies set the longest chain of pairs).
+            # runners: 57 to 164 ms for 720 steps of 490,000 microbes in eight
+            # runners, 56 to 64 now (of which the replay's own gain is a part).
             self._play, self._side, self._adv = (torch.cuda.Stream(self.device) for _ in range(3))
             self._backup = torch.empty_like(self.species)  # a chunk's starting species
             self._worst_host = torch.zeros((), dtype=torch.int64, pin_memory=True)
