@@ -29,8 +29,12 @@ from .velocity_fields import VelocityField
 logger = logging.getLogger(__name__)
 
 
-# Smallest chunk the tapered end of a pipelined run uses.
-TAPER_MIN = 8
+# Smallest chunk the tapered end of a pipelined run uses; of a population up to
+# SMALL_POPULATION, whose chunk costs the host 0.15 to 0.25 ms and whose steps
+# replay in 7 to 10 us, so that a tail shorter than this is not worth a chunk of
+# its own (24 steps of 2,500, 8,000 and 12,200 microbes: 757, 811 and 951 us with
+# 8, 529, 589 and 652 with 32).
+TAPER_MIN, TAPER_MIN_SMALL = 8, 32
 # Largest population whose chunks replay on the caller's stream: a stream more
 # costs more in events than the overlap gives (200 steps of 8,000 microbes in
 # chunks of 24, dense and sparse, 3.3 to 5.2 ms, 3.5 to 7.2 with it; 24 steps
@@ -112,6 +116,10 @@ class FusedRunner:
         self.clock_steps = 0   # steps since the field's first time level
         self.oob.zero_()
 
+    def schedule(self, total):
+        """Chunk lengths of a run of `total` steps."""
+        return chunk_schedule(total, self.chunk, TAPER_MIN if self.n > SMALL_POPULATION else TAPER_MIN_SMALL)
+
     def advance(self, nsteps):
         """Run up to self.chunk steps; returns the number of steps done.
 
@@ -160,7 +168,7 @@ class FusedRunner:
         nsets = self.PIPELINE_SETS
         main = torch.cuda.current_stream(self.device)
         side, adv = self._side, self._adv
-        sizes = chunk_schedule(total, self.chunk)
+        sizes = self.schedule(total)
         # a small population's replay is short, and a single chunk has no other
         # to run beside: the caller's stream does (4 steps of 13,000 in one
         # chunk take 365 us, 415 with a stream of its own)
@@ -442,7 +450,7 @@ class MicrobeSimulator:
             if ds is not None:
                 ds.write_block(t0, {name: arrays[name] for name in ("longitude", "latitude", "species")})
 
-        stream = RecordStream(fields, self.chunk, sink, self.device, chunks=len(chunk_schedule(iters, self.chunk)),
+        stream = RecordStream(fields, self.chunk, sink, self.device, chunks=len(runner.schedule(iters)),
                               ring_bytes=self.ring_bytes)
         t_setup = time() - tic
         done = [0]
