@@ -694,7 +694,7 @@ pair_small_emit_kernel(int n, const float* __restrict__ x_all, const float* __re
                        int64_t* __restrict__ npairs) {
     constexpr uint32_t WX = 1u << LWX, WY = 1u << LWY;
     static_assert((WX << LWY) + 1 <= (uint32_t)kSmallTab, "bucket table");
-    __shared__ uint32_t scan_lds[kSmallBlock / 64], crowded;
+    __shared__ uint32_t sums[3][kSmallBlock / 64], crowded;  // per wavefront: before, own, after
     __shared__ uint32_t who[ROWS], count[ROWS], place[ROWS];  // the crowded rows
     __shared__ __align__(16) uint16_t found[kSmallBlock / 64][kSmallGather];
     const int64_t s = blockIdx.y;
@@ -715,11 +715,22 @@ pair_small_emit_kernel(int n, const float* __restrict__ x_all, const float* __re
         after += k < i0 ? 0u : v;
     }
     if (t == 0) crowded = 0u;
-    uint32_t sum_before, sum_after, sum_own;
-    (void)small_exclusive_scan(before, scan_lds, &sum_before);
-    (void)small_exclusive_scan(after, scan_lds, &sum_after);
-    const uint32_t o = sum_before + small_exclusive_scan(c, scan_lds, &sum_own);
-    const uint32_t total = sum_before + sum_own + sum_after;
+    const uint32_t inc = wave_inclusive_scan(c);
+    before = wave_sum(before);
+    after = wave_sum(after);
+    if (lane == 63) {
+        sums[0][wave] = before;
+        sums[1][wave] = inc;
+        sums[2][wave] = after;
+    }
+    __syncthreads();
+    uint32_t o = inc - c, total = 0;
+#pragma unroll
+    for (int w = 0; w < kSmallBlock / 64; ++w) {
+        const uint32_t own_w = sums[1][w];
+        o += sums[0][w] + (w < wave ? own_w : 0u);
+        total += sums[0][w] + own_w + sums[2][w];
+    }
     if (blockIdx.x == 0 && t == 0) npairs[s] = (int64_t)total;
     if ((int64_t)total > st.pair) return;  // caller enlarges and calls again
     int32_t* pair_i = pair_i_all + s * st.pair;
