@@ -200,12 +200,12 @@ class TrajectoryLoss(torch.autograd.Function):
         if torch.is_grad_enabled():  # a gradient that is to be differentiated again
             return torch.autograd.grad(_mean_great_circle_sq(*packed), packed, by, create_graph=True)[0]
         if (_watched() or type(by) is not torch.Tensor or not torch._C._has_storage(by) or _dual(by)
-                or grad.dtype != torch.float64 or not grad.is_contiguous() or grad.device != by.device):
+                or grad.dtype != torch.float64 or not grad.is_contiguous() or grad.is_neg() or grad.device != by.device):
             # a batch of gradients (vectorised Jacobians), a mode that has to see
             # the operation, or what a hook made of the saved gradients
             return grad * by
         out = torch.empty_like(grad)
-        by = by.to(torch.float64).contiguous()
+        by = by.to(torch.float64).contiguous().resolve_neg()
         check(_lib.load().lm_scale_by(out.numel(), ptr(grad), ptr(by), ptr(out), stream_ptr()))
         return out
 
@@ -223,12 +223,13 @@ def _dual(t):
 
 
 def _plain_f64(tensors):
-    """Plain contiguous float64 tensors of one shape on the current GPU, with no
-    tracing, transform, mode or forward-mode tangent that would have to see the
-    single operations."""
+    """Plain contiguous float64 tensors of one shape on the current GPU (none a
+    lazy negative, whose memory holds the other sign), with no tracing,
+    transform, mode or forward-mode tangent that would have to see the single
+    operations."""
     t0 = tensors[0]
     if not all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.dtype == torch.float64 and t.device == t0.device
-               and t.shape == t0.shape and t.is_contiguous() for t in tensors):
+               and t.shape == t0.shape and t.is_contiguous() and not t.is_neg() for t in tensors):
         return False
     if t0.device.type != "cuda" or t0.device.index != torch.cuda.current_device() or t0.numel() == 0:
         return False

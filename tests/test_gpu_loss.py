@@ -95,7 +95,22 @@ def test_arguments_changed_in_place_before_a_second_differentiation(gpu):
         got.append((*first, *torch.autograd.grad(sum((v[1:] ** 2).sum() for v in first), leaves[:3])))
     for a, b in zip(*got):
         # rtol: as in test_second_derivatives; atol: entries that cancel to near zero
-        torch.testing.assert_close(a[1:], b[1:], rtol=1e-12, atol=1e-16 * float(b[1:].abs().max()))
+        torch.testing.assert_close(a[1:], b[1:], rtol=1e-12, atol=1e-16 * float(b[1:].detach().abs().max()))
+
+
+def test_lazy_negatives(gpu):
+    # the imaginary part of a lazy conjugate: its memory holds the other sign, and a single one is contiguous
+    z = torch.tensor([3.0 + 40.0j], dtype=torch.complex128, device="cuda")
+    lat = z.conj().imag
+    assert lat.is_neg() and lat.is_contiguous()
+    one = torch.ones(1, dtype=torch.float64, device="cuda")
+    torch.testing.assert_close(adjoint.trajectory_loss(one, lat, 2.0 * one, one),
+                               adjoint._mean_great_circle_sq(one, -40.0 * one, 2.0 * one, one), rtol=1e-13, atol=0.0)
+    x = one.clone().requires_grad_()
+    by = z.conj().imag[0]
+    got, = torch.autograd.grad(adjoint.trajectory_loss(x, one, 2.0 * one, one), x, by)
+    want, = torch.autograd.grad(adjoint.trajectory_loss(x, one, 2.0 * one, one), x)
+    torch.testing.assert_close(got, -40.0 * want, rtol=1e-15, atol=0.0)
 
 
 def test_what_the_loss_keeps(gpu):
