@@ -504,7 +504,9 @@ pair_emit_kernel(int64_t n, const float* __restrict__ x_all, const float* __rest
 // apart may share one, and the distance test drops what the stencil does not
 // reach), so the table fits LDS whatever the box.
 constexpr int kSmallNbr = 16;  // 16-bit partners kept per particle, in the bytes of kNbr 32-bit ones
-constexpr int kSmallTab = (1 << 13) + 4;  // bucket table entries per step in memory (>= 2^(LWX + LWY) + 1)
+constexpr int64_t kSmallTable = 4096;  // particles up to which the table has 2^12 buckets (2^13 above)
+// Entries per step, in memory, of a table of 2^bits buckets.
+constexpr int64_t small_tab(int bits) { return ((int64_t)1 << bits) + 4; }
 
 // A crowded row's partners are gathered from its buckets and ranked against
 // each other (the work grows with their square) up to 128 + n / 48 of them, and
@@ -587,7 +589,7 @@ pair_small_count_kernel(int n, const float* __restrict__ x_all, const float* __r
     }
     __syncthreads();
     if (blockIdx.x == 0) {  // for the rows that the emit finds again
-        for (uint32_t b = t; b <= T; b += kSmallBlock) tab_all[s * kSmallTab + b] = start[b];
+        for (uint32_t b = t; b <= T; b += kSmallBlock) tab_all[s * small_tab(LWX + LWY) + b] = start[b];
         for (int k = t; k < (n + 1) / 2; k += kSmallBlock)
             order_all[s * st.rec + k] = reinterpret_cast<const uint32_t*>(idx)[k];
     }
@@ -693,7 +695,6 @@ pair_small_emit_kernel(int n, const float* __restrict__ x_all, const float* __re
                        int32_t* __restrict__ pair_i_all, int32_t* __restrict__ pair_j_all,
                        int64_t* __restrict__ npairs) {
     constexpr uint32_t WX = 1u << LWX, WY = 1u << LWY;
-    static_assert((WX << LWY) + 1 <= (uint32_t)kSmallTab, "bucket table");
     __shared__ uint32_t sums[3][kSmallBlock / 64], crowded;  // per wavefront: before, own, after
     __shared__ uint32_t who[ROWS], count[ROWS], place[ROWS];  // the crowded rows
     __shared__ __align__(16) uint16_t found[kSmallBlock / 64][kSmallGather];
@@ -773,7 +774,7 @@ pair_small_emit_kernel(int n, const float* __restrict__ x_all, const float* __re
     if (crowded == 0u) return;  // uniform
     const float* x = x_all + s * st.pos;
     const float* y = y_all + s * st.pos;
-    const uint32_t* tab = tab_all + s * kSmallTab;
+    const uint32_t* tab = tab_all + s * small_tab(LWX + LWY);
     const uint16_t* order = order_all + 2 * s * st.rec;
     const uint32_t entry = (uint32_t)lane * (kSmallBlock / 64) + (uint32_t)wave, e = min(entry, crowded - 1u);
     const uint32_t rows = crowded > (uint32_t)wave ? (crowded - (uint32_t)wave + kSmallBlock / 64 - 1) / (kSmallBlock / 64) : 0u;
@@ -852,7 +853,7 @@ struct lm_pairs_ws {
     uint32_t* nbr_cnt = nullptr;   // [steps][row]
     uint32_t* nbr = nullptr;       // [steps][n_max * kNbr]
     uint32_t* row_off = nullptr;   // [steps][row]
-    uint32_t* small_tab = nullptr; // [steps][kSmallTab] bucket starts of a small population (its order: vals[0])
+    uint32_t* small_tab = nullptr; // [steps][small_tab] bucket starts of a small population (its order: vals[0])
     int64_t bytes = 0;
 };
 
@@ -956,7 +957,7 @@ static int search_small_table(lm_pairs_ws* ws, int32_t nsteps, int64_t n, const 
     auto count = [&](auto kernel, int32_t s0, int32_t ns, unsigned gx) {
         LM_LAUNCH(K_PAIR_SMALL, kernel, dim3(gx, (unsigned)ns), block, 0, s, (int)n, lon + s0 * st.pos,
                   lat + s0 * st.pos, g, m, st, ws->nbr_cnt + s0 * st.row, nbr + 2 * s0 * st.nbr,
-                  ws->small_tab + (int64_t)s0 * kSmallTab, ws->vals[0] + s0 * st.rec);
+                  ws->small_tab + s0 * small_tab(LWX + LWY), ws->vals[0] + s0 * st.rec);
     };
     auto emit = [&](auto kernel) {
         LM_LAUNCH(K_EMIT_SMALL, kernel, dim3(blocks, (unsigned)nsteps), block, 0, s, (int)n, lon, lat, g, m, st,
@@ -968,7 +969,7 @@ static int search_small_table(lm_pairs_ws* ws, int32_t nsteps, int64_t n, const 
         LM_LAUNCH_CHECK();
         emit(pair_small_emit_kernel<KIND, LWX, LWY, kSmallBlock / 4>);
     } else {
-        const bool in_turns = NMAX > 4096;
+        const bool in_turns = NMAX > kSmallTable;
         const int32_t even = in_turns ? nsteps / kSmallFit * kSmallFit : 0, rest = nsteps - even;
         if (even > 0) {
             count(pair_small_count_kernel<KIND, NMAX, LWX, LWY, 1>, 0, even, 1);
@@ -989,8 +990,8 @@ template <int KIND>
 static int search_small(lm_pairs_ws* ws, int32_t nsteps, int64_t n, const float* lon, const float* lat,
                         const CellGrid& g, const Metric& m, const Strides& st, int64_t* npairs, int32_t* pair_i,
                         int32_t* pair_j, hipStream_t s) {
-    if (n <= 4096)
-        return search_small_table<KIND, 4096, 6, 6>(ws, nsteps, n, lon, lat, g, m, st, npairs, pair_i, pair_j, s);
+    if (n <= kSmallTable)
+        return search_small_table<KIND, (int)kSmallTable, 6, 6>(ws, nsteps, n, lon, lat, g, m, st, npairs, pair_i, pair_j, s);
     return search_small_table<KIND, (int)kSmallMax, 7, 6>(ws, nsteps, n, lon, lat, g, m, st, npairs, pair_i, pair_j, s);
 }
 
@@ -1063,7 +1064,7 @@ int lm_pairs_ws_create_ex(int64_t n_max, int32_t steps_max, double lon_min, doub
         (rc = ws_alloc(&w->nbr_cnt, S * w->row_stride, &w->bytes)) ||
         (rc = ws_alloc(&w->nbr, S * n_max * lm::kNbr, &w->bytes)) ||
         (rc = ws_alloc(&w->row_off, S * w->row_stride, &w->bytes)) ||
-        (rc = ws_alloc(&w->small_tab, S * lm::kSmallTab, &w->bytes))) {
+        (rc = ws_alloc(&w->small_tab, S * lm::small_tab(n_max <= lm::kSmallTable ? 12 : 13), &w->bytes))) {
         pairs_ws_free(w);
         return rc;
     }
